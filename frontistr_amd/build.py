@@ -33,6 +33,7 @@ SOURCES = [
     ("learned.hip", True),
     ("coarse.hip", True),
     ("noalloc.hip", True),
+    ("resident.hip", True),
 ]
 
 

@@ -112,7 +112,7 @@ struct KrylovState {
   int32_t n_indef;
   int32_t recheck;   // recompute the true residual in this iteration
   int32_t nrec;      // true-residual period (50 CG, 100 BiCGSTAB)
-  int32_t pad;
+  int32_t resume;    // resident solve: 0 new, 1 continue where the last launch ended
   // flexible CG with FP32 operators (reliable updates)
   double zq, pq, rp;   // z.q_prev, p.q, r.p of the current iteration
   double rr_ref;       // |r|^2 at the last FP64 true-residual update
@@ -130,6 +130,7 @@ struct KrylovState {
   // the learned step is dropped when |r|^2 at a replacement exceeds drop2 times the smallest
   // FP64 |r|^2 seen so far (rr_min)
   double drop2, rr_min;
+  double time_Ax, time_precond;  // seconds of the resident solve's sweeps
 };
 
 constexpr int kMaxPartials = 65536;  // per reduction component
@@ -229,6 +230,57 @@ void bi_spmv_omega(const Sell<double>& a, const double* stv, const double* sv, d
                    double* part, hipStream_t s, hipEvent_t after = nullptr, const MpcOp* mpc = nullptr);
 void bi_update(int64_t n3, const double* pt, const double* stv, const double* t, const double* sv, double* x,
                double* r, KrylovState* st, double* part, double* hist, hipStream_t s);
+
+// ---- resident SSOR-CG (resident.hip) ------------------------------------------------
+// Off-diagonal blocks packed into tasks: task t holds the blocks of up to
+// kResidentRows consecutive row slots of one colour.  A row takes whole lanes of
+// the task, K consecutive blocks to a lane: block k of the row is block k % K of
+// lane row.x % 64 + k / K, at column col[(t K + k % K) * 64 + lane] with its values
+// in A's paired planes (aval_index, group t K + k % K).  Blocks without an entry
+// have value 0 and column ns, a record that is always there.  The tasks of L'
+// come first, then those of U'.
+constexpr int kResidentGridMax = 256;   // workgroups (one per CU)
+constexpr int kResidentSync = 64 * 10;  // words of the grid barrier's counters
+constexpr int kResidentPlanes = 27;     // of 16 slots in a row record: six vectors and the LU
+constexpr int kResidentPackets = 4;     // most blocks per lane
+constexpr int kResidentRows = 16;       // most rows of a task
+struct ResidentOp {
+  Sell<double> A;  // natural order, for the true residual
+  const int32_t* color_task = nullptr;  // [2][ncolor+1] first task of every colour of L', U'
+  const int4* task = nullptr;           // first row slot, rows, lanes used
+  const int2* row = nullptr;            // [2][ns] first lane of a row (64 t + lane), its lanes
+  const int32_t* col = nullptr;         // row slot of every packed block's column
+  const double* val = nullptr;
+  int32_t ncolor = 0, ns = 0, n = 0;    // colours, row slots, internal nodes
+  const double* dsig = nullptr;         // (1 - sigma) diag D, [3][ns]; null for sigma = 1
+  const int32_t* row_old = nullptr;
+  const int32_t* node_slot = nullptr;
+  double* rec = nullptr;                // r, x, p, q, g, h and the LU of D': per 16 slots, kResidentPlanes planes
+  double* zw = nullptr;                 // the gathered vectors, two copies of ns + 1 records
+  double* xn = nullptr;               // x in node order
+  const double* b = nullptr;          // right-hand side in node order
+  double* part = nullptr;
+  double* hist = nullptr;
+  uint32_t* sync = nullptr;
+  KrylovState* state = nullptr;
+};
+// Launch shape: workgroups and blocks per lane
+struct ResidentShape {
+  int grid = 0, packets = 2;
+};
+// values (and with_col: columns) of a SELL factor into its packets
+void resident_pack(const Sell<double>& s, const int2* row, int packets, int32_t* col, double* val, bool with_col,
+                   hipStream_t st);
+void resident_dsig(int32_t ns, const int32_t* row_old, const double* D, double sigma, double* out, hipStream_t st);
+// the LU factors (planes of `rows` slots) into the row records
+void resident_alu(const ResidentOp& o, const double* alu, int rows, hipStream_t st);
+// r (node order) and x (o.xn) into slot order, the other vectors to their initial state
+void resident_init(const ResidentOp& o, const ResidentShape& sh, const double* r, hipStream_t st);
+// whether a single workgroup can keep the gathered vectors of ns rows in LDS
+bool resident_one_group(int ncolor, int ns);
+// up to `budget` CG iterations; a cooperative launch, so that every workgroup
+// is on the GPU before the first grid barrier
+hipError_t resident_cg(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s);
 
 // ---- flexible CG with FP32 operators and FP64 recurrences ------------------------
 // z32 = M^-1 r32 in FP32 (kind 0 copy, 1 SSOR, 3 DIAG)

@@ -244,6 +244,19 @@ struct Context {
   int32_t ssor_last_bwd_empty = 0;  // the last colour's U' rows are all empty
   SellDev L, U;
   DMem row_old, node_slot, alu_ssor, vzs, vzs32;
+  // resident SSOR-CG: packed copies of L'/U' and its slot-order vectors
+  uint64_t val_gen = 0;         // bumped whenever the matrix values change
+  uint64_t ssor_gen = 0;        // val_gen that the SSOR factors were made from
+  double ssor_sigma = 1.0;
+  std::vector<int32_t> h_lenL, h_lenU;  // blocks of every row slot
+  int32_t res_packets = 0;      // blocks per lane of the packed structure (0: none built)
+  uint64_t res_num = 0;         // numeric set-up (ssor_num) that the packed values hold
+  uint64_t ssor_num = 0;        // bumped at every numeric SSOR set-up
+  int32_t res_cus = 0;          // compute units (0: no cooperative launches)
+  int32_t last_resident = 0;    // workgroups of the last solve's resident kernel (0: launch per colour)
+  bool ssor_proper = false;     // no L'/U' column lies in its row's own colour
+  ResidentOp res;
+  DMem res_color_task, res_task, res_row, res_col, res_val, res_vec, res_sync, res_dsig;
   bool ssor16 = true;          // the flexible CG's FP32 sweeps read BF16 copies of the L'/U' values
   bool ssor16_valid = false;   // L.val16 / U.val16 hold the current values
   // DIAG
@@ -347,6 +360,8 @@ struct Context {
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
                     &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
       m->release();
+    for (DMem* m : {&res_color_task, &res_task, &res_row, &res_col, &res_val, &res_vec, &res_sync, &res_dsig})
+      m->release();
     if (blas) rocblas_destroy_handle(blas);
     for (DMem* m : {&mpc_slave, &mpc_mptr, &mpc_mdof, &mpc_mval, &mpc_tptr, &mpc_tslave, &mpc_tval, &mpc_w1, &mpc_w2})
       m->release();
@@ -405,6 +420,11 @@ static int32_t ctx_init(Context& c) {
     set_error("no HIP device visible");
     return HECMW33_ERROR_DEVICE;
   }
+  int dev = 0;
+  HIPC(hipGetDevice(&dev));
+  int coop = 0;
+  HIPC(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+  if (coop) HIPC(hipDeviceGetAttribute(&c.res_cus, hipDeviceAttributeMultiprocessorCount, dev));
   HIPC(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   HIPC(hipHostMalloc((void**)&c.h_st, 2 * sizeof(KrylovState), hipHostMallocDefault));
   if (c.st.ensure(sizeof(KrylovState)) || c.part.ensure(sizeof(double) * 4 * kMaxPartials))
@@ -511,6 +531,7 @@ static int32_t load_values(Context& c, const hecmw33_sys* A) {
   launch_fill_values_a(c.A.view, c.A.src.as<int64_t>(), c.dD.as<double>(), c.dAL.as<double>(), c.dAU.as<double>(),
                      c.N, c.NPL, c.stream);
   HIPC(hipGetLastError());
+  ++c.val_gen;
   c.a32_valid = false;
   c.mat_valid = false;
   c.coarse_num = false;
@@ -565,6 +586,15 @@ static int32_t setup_ssor_symbolic(Context& c, int32_t ncolor_in) {
                          c.iperm.data());
   std::vector<int32_t> iLp, tLp, iUp, tUp;
   reorder_profile(N, c.perm.data(), c.iperm.data(), iL, tL, iU, tU, iLp, tLp, iUp, tUp);
+  // a profile that is not symmetric can leave couplings inside a colour
+  bool proper = true;
+#pragma omp parallel for schedule(dynamic, 1) reduction(&& : proper)
+  for (int32_t k = 0; k < c.ncolor; ++k)
+    for (int32_t i = c.colorindex[k]; i < c.colorindex[k + 1]; ++i) {
+      for (int32_t q = iLp[i]; q < iLp[i + 1]; ++q) proper = proper && tLp[q] <= c.colorindex[k];
+      for (int32_t q = iUp[i]; q < iUp[i + 1]; ++q) proper = proper && tUp[q] > c.colorindex[k + 1];
+    }
+  c.ssor_proper = proper;
   // Rows per slice: 16 (four lanes per row) or 64 (a lane per row).  The
   // lane-per-row sweep needs a quarter of the waves, which pays once a colour
   // holds many more slices than the GPU keeps resident; HECMW33_SSOR_ROWS
@@ -659,6 +689,9 @@ static int32_t setup_ssor_symbolic(Context& c, int32_t ncolor_in) {
     build_lu(std::integral_constant<int, kRowsS>{});
   if (int32_t e = upload_sell(hl, c.L, c.stream)) return e;
   if (int32_t e = upload_sell(hu, c.U, c.stream)) return e;
+  c.h_lenL = std::move(hl.len);
+  c.h_lenU = std::move(hu.len);
+  c.res_packets = 0;
   // the slot of every node, for staging r into slot order and z back out
   std::vector<int32_t> node_slot(N, -1);
   for (int64_t t = 0; t < (int64_t)row_old.size(); ++t)
@@ -703,6 +736,9 @@ static int32_t setup_ssor(Context& c, double sigma, int32_t ncolor_in, bool symb
   c.ssor_init = true;
   c.ssor32_valid = false;
   c.ssor16_valid = false;
+  c.ssor_gen = c.val_gen;
+  c.ssor_sigma = sigma;
+  ++c.ssor_num;
   return 0;
 }
 
@@ -1298,6 +1334,160 @@ static void enqueue_fcg_sym_iteration(Context& c, int32_t kind, bool spmv64, hip
   fcg_reliable(c.A.view, c.vx.as<double>(), c.vb.as<double>(), r, st, part, c.hist.as<double>(), c.stream);
 }
 
+// ---- resident SSOR-CG (resident.hip) ------------------------------------------------------
+// The packed structure: per direction the rows of a colour in slot order, cut
+// where the rows or the lanes of a task are full.
+static int32_t resident_tasks(Context& c, const ResidentShape& sh) {
+  const int64_t ns = c.ssor_rows;
+  const int32_t K = sh.packets;
+  std::vector<int32_t> ct;
+  std::vector<int4> task;
+  std::vector<int2> row(2 * (size_t)ns, make_int2(0, 0));
+  for (int d = 0; d < 2; ++d) {
+    const std::vector<int32_t>& len = d ? c.h_lenU : c.h_lenL;
+    for (int32_t k = 0; k < c.ncolor; ++k) {
+      ct.push_back((int32_t)task.size());
+      const int64_t s0 = (int64_t)c.color_slice[k] * c.ssor_R, cnt = c.colorindex[k + 1] - c.colorindex[k];
+      int4 cur = make_int4(0, kResidentRows, 0, 0);
+      for (int64_t t = s0; t < s0 + cnt; ++t) {
+        const int32_t lanes = (len[t] + K - 1) / K;
+        if (cur.y == kResidentRows || cur.z + lanes > kWave) {
+          cur = make_int4((int)t, 0, 0, 0);
+          task.push_back(cur);
+        }
+        row[d * ns + t] = make_int2((int)(task.size() - 1) * kWave + cur.z, lanes);
+        cur.y += 1;
+        cur.z += lanes;
+        task.back() = cur;
+      }
+    }
+    ct.push_back((int32_t)task.size());
+  }
+  const size_t nblk = (size_t)kWave * K * task.size();
+  if (c.res_color_task.ensure(sizeof(int32_t) * ct.size()) || c.res_task.ensure(sizeof(int4) * task.size()) ||
+      c.res_row.ensure(sizeof(int2) * row.size()) || c.res_col.ensure(sizeof(int32_t) * nblk) ||
+      c.res_val.ensure(sizeof(double) * 9 * nblk) ||
+      c.res_vec.ensure(sizeof(double) * (kResidentPlanes * (size_t)ns + 16 * ((size_t)ns + 1))) ||
+      c.res_sync.ensure(sizeof(uint32_t) * kResidentSync)) {
+    for (DMem* m : {&c.res_color_task, &c.res_task, &c.res_row, &c.res_col, &c.res_val, &c.res_vec}) m->release();
+    (void)hipGetLastError();
+    return 1;
+  }
+  HIPC(hipMemcpyAsync(c.res_color_task.p, ct.data(), sizeof(int32_t) * ct.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipMemcpyAsync(c.res_task.p, task.data(), sizeof(int4) * task.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipMemcpyAsync(c.res_row.p, row.data(), sizeof(int2) * row.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipMemsetD32Async((hipDeviceptr_t)c.res_col.p, (int)ns, nblk, c.stream));
+  HIPC(hipMemsetAsync(c.res_val.p, 0, sizeof(double) * 9 * nblk, c.stream));
+  HIPC(hipStreamSynchronize(c.stream));  // the host vectors end here
+  return 0;
+}
+
+// The launch shape for this system; grid 0: the launch-per-colour solve.
+//  * Two blocks per lane: one block doubles the tasks, and the row work of a task
+//    costs the same (30^3 cube, 256 workgroups: 70.5 us per iteration against
+//    66.6); four make it slower again (80.8). Four only where a row of more than
+//    128 blocks needs them; more than 256 blocks in a row do not fit a task.
+//  * Workgroups by the tasks of an average colour step: beyond a few tasks each,
+//    more workgroups add bandwidth (30^3, 195 tasks: 128 and 256 workgroups 71.6
+//    and 66.6 us; 72^3, 641 and 379 us), below that only barrier time (14^3, 21
+//    tasks: 61-65 us from 32 to 256; 10^3, 8 tasks: 60 us with 32).
+//  * One workgroup, its gathered vectors in LDS, up to 1000 nodes where they fit
+//    (6^3 cube, 343 nodes: 47 us against 53 with 32 workgroups; TET10 box, 315
+//    nodes: 55 against 65; 10^3, 1331 nodes: equal).
+static ResidentShape resident_shape(const Context& c) {
+  ResidentShape sh;
+  int32_t longest = 0;
+  int64_t lanes = 0;
+  for (const std::vector<int32_t>* len : {&c.h_lenL, &c.h_lenU})
+    for (int32_t l : *len) {
+      longest = std::max(longest, l);
+      lanes += (l + 1) / 2;
+    }
+  if (longest > kWave * kResidentPackets || c.res_cus < 1) return sh;
+  if (longest > 2 * kWave) sh.packets = 4;
+  const int64_t tasks = lanes / (2 * (int64_t)c.ncolor * kWave);
+  sh.grid = tasks < 16 ? 32 : tasks < 64 ? 128 : 256;
+  if (c.N <= 1000 && resident_one_group(c.ncolor, (int)c.ssor_rows)) sh.grid = 1;
+  sh.grid = std::min(sh.grid, std::min(c.res_cus, kResidentGridMax));
+  return sh;
+}
+
+// Whether this solve can run resident: plain FP64 CG whose SSOR factors were
+// made from the present values (a recycled preconditioner has other L' and U'
+// than A), all columns internal, no couplings inside a colour, one application
+// per iteration, no constraint products; gathered records
+// within the 4 GiB of a buffer resource, the colours' ranges within LDS.
+static bool resident_fits(const Context& c, int32_t method, int32_t kind, int32_t iterpremax, bool mixed) {
+  return method == 1 && kind == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N &&
+         c.ssor_gen == c.val_gen && c.ssor_proper && c.ssor_rows < 30000000 && c.ncolor <= 512;
+}
+
+// 1: no memory for the packed copy (the launch-per-colour solve needs none)
+static int32_t resident_setup(Context& c, const ResidentShape& sh) {
+  ResidentOp& o = c.res;
+  const int32_t ns = (int32_t)c.ssor_rows;
+  const bool sym = c.res_packets != sh.packets;
+  if (sym) {
+    c.res_packets = 0;
+    if (int32_t e = resident_tasks(c, sh)) return e;
+    c.res_packets = sh.packets;
+  }
+  o.ns = ns;
+  o.rec = c.res_vec.as<double>();
+  o.zw = o.rec + kResidentPlanes * (size_t)ns;
+  if (sym || c.res_num != c.ssor_num) {
+    for (int d = 0; d < 2; ++d)
+      resident_pack(d ? c.U.view : c.L.view, c.res_row.as<int2>() + d * (size_t)ns, sh.packets, c.res_col.as<int32_t>(),
+                    c.res_val.as<double>(), sym, c.stream);
+    resident_alu(o, c.alu_ssor.as<double>(), c.ssor_R, c.stream);
+    c.res_num = c.ssor_num;
+  }
+  o.dsig = nullptr;
+  if (c.ssor_sigma != 1.0) {
+    if (c.res_dsig.ensure(sizeof(double) * 3 * (size_t)ns)) return HECMW33_ERROR_DEVICE;
+    resident_dsig(ns, c.row_old.as<int32_t>(), c.dD.as<double>(), c.ssor_sigma, c.res_dsig.as<double>(), c.stream);
+    o.dsig = c.res_dsig.as<double>();
+  }
+  o.A = c.A.view;
+  o.ncolor = c.ncolor;
+  o.n = c.N;
+  o.row_old = c.row_old.as<int32_t>();
+  o.node_slot = c.node_slot.as<int32_t>();
+  o.color_task = c.res_color_task.as<int32_t>();
+  o.task = c.res_task.as<int4>();
+  o.row = c.res_row.as<int2>();
+  o.col = c.res_col.as<int32_t>();
+  o.val = c.res_val.as<double>();
+  o.xn = c.vx.as<double>();
+  o.b = c.vb.as<double>();
+  o.part = c.part.as<double>();
+  o.hist = c.hist.as<double>();
+  o.sync = c.res_sync.as<uint32_t>();
+  o.state = c.st.as<KrylovState>();
+  HIPC(hipGetLastError());
+  return 0;
+}
+
+// The Krylov loop as resident launches of `kResidentBudget` iterations (a bounded
+// stay on the GPU), from r0 in vr and the initial state on the device; the end
+// state in c.h_st[0].
+constexpr int kResidentBudget = 512;
+static int32_t resident_solve(Context& c, const ResidentShape& sh) {
+  resident_init(c.res, sh, c.vr.as<double>(), c.stream);
+  for (;;) {
+    HIPC(resident_cg(c.res, sh, kResidentBudget, c.stream));
+    uint32_t abort = 0;
+    HIPC(hipMemcpyAsync(&c.h_st[0], c.st.p, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
+    HIPC(hipMemcpyAsync(&abort, c.res.sync + 64 * 9, sizeof(abort), hipMemcpyDeviceToHost, c.stream));
+    HIPC(hipStreamSynchronize(c.stream));
+    if (abort) {
+      set_error("resident solve: a workgroup waited 20 s for the others");
+      return HECMW33_ERROR_DEVICE;
+    }
+    if (c.h_st[0].done) return 0;
+  }
+}
+
 // Diagonal scaling of the device copies, hecmw_solver_scaling_fw_33 / _bk_33
 // (hecmw_solver_scaling_33.f90:20-208): forward scales the uploaded D/AL/AU
 // and b in place (x0 is left as given), backward unscales x and restores b
@@ -1331,6 +1521,7 @@ static int32_t scaling_apply(Context& c, bool fw) {
                    c.dItemU.as<int32_t>(), c.dD.as<double>(), c.dAL.as<double>(), c.dAU.as<double>(), sc, c.stream);
   launch_fill_values_a(c.A.view, c.A.src.as<int64_t>(), c.dD.as<double>(), c.dAL.as<double>(), c.dAU.as<double>(),
                      c.N, c.NPL, c.stream);
+  ++c.val_gen;
   c.a32_valid = false;
   c.coarse_num = false;
   HIPC(hipGetLastError());
@@ -1789,6 +1980,16 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
     for (DMem* m : {&c.vrt, &c.vs, &c.vt, &c.vv, &c.vpt, &c.vst})
       if (m->ensure(vbytes)) return HECMW33_ERROR_DEVICE;
   }
+  ResidentShape shape;
+  if (resident_fits(c, method, kind, iterpremax, mixed)) {
+    shape = resident_shape(c);
+    if (shape.grid > 0) {
+      const int32_t e = resident_setup(c, shape);
+      if (e < 0) return e;
+      if (e > 0) shape.grid = 0;
+    }
+  }
+  c.last_resident = shape.grid;
   // r0 = b - A x0; bnrm2 = b.b  (hecmw_solver_CG.f90:131-141)
   if (mixed && c.x_zero) {
     // x0 = 0 (the learned modes' sample solves): r0 = b exactly, without the FP64 product
@@ -1840,6 +2041,8 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
   h.n_indef = 0;
   h.recheck = 0;
   h.nrec = method == 1 ? 50 : 100;
+  h.resume = 0;
+  h.time_Ax = h.time_precond = 0.0;
   h.zq = h.pq = h.rp = 0.0;
   const double delta = RA(rarray, R_SOLVER_OPT) > 0.0 && RA(rarray, R_SOLVER_OPT) < 1.0 ? RA(rarray, R_SOLVER_OPT)
                                                                                          : kFcgDelta;
@@ -1863,54 +2066,61 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
   HIPC(hipStreamSynchronize(c.stream));
   const double t1 = now_s();
   out->Tset = t1 - t0;
-  // iterations: enqueue in chunks and poll the previous chunk's state while
-  // the current one runs; kernels after the exit return at once
   const int chunk = 8;
   const int nev = method == 1 ? 4 : 8;
-  hipEvent_t ev[2];
-  HIPC(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-  HIPC(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
   int32_t enq = 0, nchunk = 0;
-  bool finished = false;
-  std::vector<hipEvent_t> itev(nev);
-  while (enq < maxit && !finished) {
-    const int k = std::min(chunk, maxit - enq);
-    for (int i = 0; i < k; ++i) {
-      // TIMELOG times the first iteration of each chunk: an event between two
-      // kernels costs a few microseconds of idle GPU, so one iteration in
-      // `chunk` carries them and the totals are scaled to all iterations
-      hipEvent_t* e = nullptr;
-      if (timelog && i == 0) {
-        for (int j = 0; j < nev; ++j) itev[j] = c.event((size_t)nev * nchunk + j);
-        e = itev.data();
+  if (shape.grid > 0) {
+    if (int32_t e = resident_solve(c, shape)) return e;
+  } else {
+    // iterations: enqueue in chunks and poll the previous chunk's state while
+    // the current one runs; kernels after the exit return at once
+    hipEvent_t ev[2];
+    HIPC(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
+    HIPC(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
+    bool finished = false;
+    std::vector<hipEvent_t> itev(nev);
+    while (enq < maxit && !finished) {
+      const int k = std::min(chunk, maxit - enq);
+      for (int i = 0; i < k; ++i) {
+        // TIMELOG times the first iteration of each chunk: an event between two
+        // kernels costs a few microseconds of idle GPU, so one iteration in
+        // `chunk` carries them and the totals are scaled to all iterations
+        hipEvent_t* e = nullptr;
+        if (timelog && i == 0) {
+          for (int j = 0; j < nev; ++j) itev[j] = c.event((size_t)nev * nchunk + j);
+          e = itev.data();
+        }
+        if (c.coarse_sym_use)
+          enqueue_fcg_sym_iteration(c, kind, spmv64, e);
+        else if (mixed)
+          enqueue_fcg_iteration(c, kind, spmv64, e);
+        else if (method == 1)
+          enqueue_cg_iteration(c, kind, iterpremax, e);
+        else
+          enqueue_bicg_iteration(c, kind, iterpremax, e);
       }
-      if (c.coarse_sym_use)
-        enqueue_fcg_sym_iteration(c, kind, spmv64, e);
-      else if (mixed)
-        enqueue_fcg_iteration(c, kind, spmv64, e);
-      else if (method == 1)
-        enqueue_cg_iteration(c, kind, iterpremax, e);
-      else
-        enqueue_bicg_iteration(c, kind, iterpremax, e);
+      enq += k;
+      const int slot = nchunk & 1;
+      HIPC(hipMemcpyAsync(&c.h_st[slot], st, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
+      HIPC(hipEventRecord(ev[slot], c.stream));
+      if (nchunk > 0) {
+        HIPC(hipEventSynchronize(ev[slot ^ 1]));
+        if (c.h_st[slot ^ 1].done) finished = true;
+      }
+      ++nchunk;
     }
-    enq += k;
-    const int slot = nchunk & 1;
-    HIPC(hipMemcpyAsync(&c.h_st[slot], st, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
-    HIPC(hipEventRecord(ev[slot], c.stream));
-    if (nchunk > 0) {
-      HIPC(hipEventSynchronize(ev[slot ^ 1]));
-      if (c.h_st[slot ^ 1].done) finished = true;
-    }
-    ++nchunk;
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpyAsync(&c.h_st[0], st, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
+    HIPC(hipStreamSynchronize(c.stream));
+    (void)hipEventDestroy(ev[0]);
+    (void)hipEventDestroy(ev[1]);
   }
-  HIPC(hipGetLastError());
-  HIPC(hipMemcpyAsync(&c.h_st[0], st, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
-  HIPC(hipStreamSynchronize(c.stream));
-  (void)hipEventDestroy(ev[0]);
-  (void)hipEventDestroy(ev[1]);
   h = c.h_st[0];
   out->Tsol = now_s() - t1;
-  if (timelog) {
+  if (timelog && shape.grid > 0) {
+    out->time_Ax = h.time_Ax;
+    out->time_precond = h.time_precond;
+  } else if (timelog) {
     // kernel time of the sampled iterations that ran (later ones returned at
     // once), scaled to the iterations that ran
     const int64_t ran = std::min<int64_t>(std::min(h.iter, maxit), enq);
@@ -2364,7 +2574,7 @@ int32_t hecmw33_ctx_info(hecmw33_ctx* ctx, int64_t* info, int32_t n) {
     for (int32_t k : kept) az_kept += k;
     az_sym = c.coarse_nw;
   }
-  const int64_t v[21] = {c.A.view.nslots,
+  const int64_t v[22] = {c.A.view.nslots,
                         (int64_t)c.N,
                         (int64_t)c.NPL,
                         (int64_t)c.NPU,
@@ -2384,8 +2594,9 @@ int32_t hecmw33_ctx_info(hecmw33_ctx* ctx, int64_t* info, int32_t n) {
                         (int64_t)c.modes_iters,
                         (int64_t)std::llround(c.modes_harvest_s * 1e6),
                         (int64_t)std::llround(c.modes_fit_s * 1e6),
-                        (int64_t)c.coarse.nc};
-  for (int i = 0; i < n && i < 21; ++i) info[i] = v[i];
+                        (int64_t)c.coarse.nc,
+                        (int64_t)c.last_resident};
+  for (int i = 0; i < n && i < 22; ++i) info[i] = v[i];
   return 0;
 }
 

@@ -549,14 +549,15 @@ class DeviceContext:
         return h[:n]
 
     def info(self):
-        v = np.zeros(21, np.int64)
-        _check(lib().hecmw33_ctx_info(self._h, _ptr(v), 21))
+        v = np.zeros(22, np.int64)
+        _check(lib().hecmw33_ctx_info(self._h, _ptr(v), 22))
         return {"nslots": int(v[0]), "N": int(v[1]), "NPL": int(v[2]), "NPU": int(v[3]), "ncolor": int(v[4]),
                 "ssor_slots": int(v[5]), "nreliable": int(v[6]), "fallback_iter": int(v[7]), "learned_off": int(v[8]),
                 "spmv64": int(v[9]), "learned_modes": int(v[10]), "coarse": int(v[11]), "coarse_pairs": int(v[12]),
                 "az_entries": int(v[13]), "az_entries_symbolic": int(v[14]), "modes_per_aggregate": int(v[15]),
                 "mode_samples": int(v[16]), "mode_sample_iters": int(v[17]), "mode_harvest_s": v[18] * 1e-6,
-                "mode_fit_s": v[19] * 1e-6, "coarse_unknowns": int(v[20])}
+                "mode_fit_s": v[19] * 1e-6, "coarse_unknowns": int(v[20]),
+                "resident": int(v[21])}
 
     def coarse(self, with_E=True):
         """The last two-level set-up: dict(n_agg, n_pair, agg [N], dv [N,3], pair_a, pair_b [n_pair],
