@@ -112,7 +112,7 @@ struct KrylovState {
   int32_t n_indef;
   int32_t recheck;   // recompute the true residual in this iteration
   int32_t nrec;      // true-residual period (50 CG, 100 BiCGSTAB)
-  int32_t resume;    // resident solve: 0 new, 1 continue where the last launch ended
+  int32_t resume;    // resident solve: 0 new, else where the last launch ended
   // flexible CG with FP32 operators (reliable updates)
   double zq, pq, rp;   // z.q_prev, p.q, r.p of the current iteration
   double rr_ref;       // |r|^2 at the last FP64 true-residual update

@@ -648,8 +648,8 @@ __device__ __forceinline__ double true_resid_phase(const Resident<T, K, MEM>& k)
 }
 
 // `budget` CG iterations (hecmw_solver_CG.f90:164-279) from the state in o.state;
-// its `resume` is 0 for a new solve (r and x in slot order), 1 + the copy that
-// holds z when z and rho stand as an earlier launch left them.  Every thread runs the scalar logic on
+// bit 0 of its `resume` says that z and rho stand as an earlier launch left them
+// (else r and x do), bit 1 is the present copy.  Every thread runs the scalar logic on
 // the same totals.
 template <int T, int K, int MEM>
 __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
@@ -662,10 +662,10 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
   int iter = st.iter, n_indef = st.n_indef, error = 0;
   const int maxit = st.maxit, nrec = st.nrec;
   const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
-  bool refresh = st.resume == 0;  // h and z have to be made from r first
+  bool refresh = !(st.resume & 1);  // h and z have to be made from r first
   bool done = false, xn_current = false;
   uint64_t ticks[2] = {0, 0};  // forward and backward sweeps
-  k.par = st.resume == 2 ? 1 : 0;
+  k.par = st.resume >> 1;
   k.begin(0);
   double* const part0 = o.part;
   double* const part1 = o.part + 2 * k.G;
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
     st.n_indef = n_indef;
     st.error = error;
     st.done = done ? 1 : 0;
-    st.resume = refresh ? 0 : 1 + k.par;
+    st.resume = (refresh ? 0 : 1) | k.par << 1;
     st.time_Ax += 1e-8 * (double)ticks[0];
     st.time_precond += 1e-8 * (double)ticks[1];
   }
