@@ -231,7 +231,7 @@ void bi_spmv_omega(const Sell<double>& a, const double* stv, const double* sv, d
 void bi_update(int64_t n3, const double* pt, const double* stv, const double* t, const double* sv, double* x,
                double* r, KrylovState* st, double* part, double* hist, hipStream_t s);
 
-// ---- resident SSOR-CG (resident.hip) ------------------------------------------------
+// ---- resident SSOR-CG and SSOR-BiCGSTAB (resident.hip) ------------------------------------------------
 // Off-diagonal blocks packed into tasks: task t holds the blocks of up to
 // kResidentRows consecutive row slots of one colour.  A row takes whole lanes of
 // the task, K consecutive blocks to a lane: block k of the row is block k % K of
@@ -241,7 +241,8 @@ void bi_update(int64_t n3, const double* pt, const double* stv, const double* t,
 // come first, then those of U'.
 constexpr int kResidentGridMax = 256;   // workgroups (one per CU)
 constexpr int kResidentSync = 64 * 10;  // words of the grid barrier's counters
-constexpr int kResidentPlanes = 27;     // of 16 slots in a row record: six vectors and the LU
+constexpr int kResidentPlanesCg = 27;   // of 16 slots in a row record: the LU and six vectors (CG)
+constexpr int kResidentPlanesBi = 39;   // or ten (BiCGSTAB)
 constexpr int kResidentPackets = 4;     // most blocks per lane
 constexpr int kResidentRows = 16;       // most rows of a task
 struct ResidentOp {
@@ -255,7 +256,8 @@ struct ResidentOp {
   const double* dsig = nullptr;         // (1 - sigma) diag D, [3][ns]; null for sigma = 1
   const int32_t* row_old = nullptr;
   const int32_t* node_slot = nullptr;
-  double* rec = nullptr;                // r, x, p, q, g, h and the LU of D': per 16 slots, kResidentPlanes planes
+  double* rec = nullptr;                // the LU of D' and the vectors: per 16 slots, `planes` planes
+  int32_t planes = 0;                   // kResidentPlanesCg or kResidentPlanesBi, which picks the method
   double* zw = nullptr;                 // the gathered vectors, two copies of ns + 1 records
   double* xn = nullptr;               // x in node order
   const double* b = nullptr;          // right-hand side in node order
@@ -278,9 +280,9 @@ void resident_alu(const ResidentOp& o, const double* alu, int rows, hipStream_t 
 void resident_init(const ResidentOp& o, const ResidentShape& sh, const double* r, hipStream_t st);
 // whether a single workgroup can keep the gathered vectors of ns rows in LDS
 bool resident_one_group(int ncolor, int ns);
-// up to `budget` CG iterations; a cooperative launch, so that every workgroup
+// up to `budget` iterations; a cooperative launch, so that every workgroup
 // is on the GPU before the first grid barrier
-hipError_t resident_cg(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s);
+hipError_t resident_run(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s);
 
 // ---- flexible CG with FP32 operators and FP64 recurrences ------------------------
 // z32 = M^-1 r32 in FP32 (kind 0 copy, 1 SSOR, 3 DIAG)

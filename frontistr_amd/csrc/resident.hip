@@ -1,5 +1,5 @@
-// SSOR-CG as one resident kernel: every workgroup stays on the GPU for many
-// iterations and the colours of the sweeps are separated by grid barriers.
+// SSOR-CG and SSOR-BiCGSTAB as one resident kernel: every workgroup stays on the
+// GPU for many iterations.
 //
 // What bounds the launch-per-colour solve below about a million rows is not the
 // matrix stream but the chain of ~35 dependent launches per SSOR application
@@ -252,6 +252,13 @@ struct Resident {
         break;
       }
   }
+  // grid barrier for stores that the callers have drained
+  __device__ __forceinline__ void grid_sync() {
+    wg_barrier();
+    if (MEM == kOneGroup) return;
+    if (wave == 0) arrive_and_wait();
+    wg_barrier();
+  }
   // barrier for plain stores too: x in node order, which the product reads
   // through the caches
   __device__ __forceinline__ void full_sync() {
@@ -463,13 +470,17 @@ struct Resident {
   }
 };
 
-// Row work of the sweeps, one entry of a row per lane.  A row's vectors and the
-// LU of its D' sit in one record per 16 slots (plane = 16 slots,
-// kResidentPlanes planes), so that a lane reaches all of them from one address.
-enum Vec : int { kR = 0, kX = 3, kP = 6, kQ = 9, kG = 12, kH = 15, kAlu = 18 };
-static_assert(kAlu + 9 == kResidentPlanes, "planes of a row record");
+// Row work of the sweeps, one entry of a row per lane.  The LU of a row's D' and
+// its vectors sit in one record per 16 slots (plane = 16 slots, o.planes
+// planes), so that a lane reaches all of them from one address.
+enum Vec : int {
+  kAlu = 0, kR = 9, kX = 12,                                // both methods
+  kP = 15, kQ = 18, kG = 21, kH = 24, kCgPlanes = 27,       // CG
+  kRt = 15, kBp = 18, kV = 21, kT = 24, kHr = 27, kHp = 30, kHv = 33, kHt = 36, kBiPlanes = 39,  // BiCGSTAB
+};
+static_assert(kCgPlanes == kResidentPlanesCg && kBiPlanes == kResidentPlanesBi, "planes of a row record");
 __device__ __forceinline__ double* rec(const ResidentOp& o, int slot) {
-  return o.rec + (int64_t)(slot / kRowsS) * (kResidentPlanes * kRowsS) + slot % kRowsS;
+  return o.rec + (int64_t)(slot / kRowsS) * (o.planes * kRowsS) + slot % kRowsS;
 }
 template <class R, int MEM>
 struct Row {
@@ -784,6 +795,262 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
   }
 }
 
+// ---- BiCGSTAB (hecmw_solver_BiCGSTAB.f90:164-275) ---------------------------------
+// The same two sweeps give p^ = M^-1 p, v = A p^ and s^ = M^-1 s, t = A s^; all
+// other vectors are linear combinations, so their D'-multiplied transforms h =
+// D' (D'+L)^-1 (.) follow by the same combinations (hr, hp of r and p, hv, ht from
+// the forward sweeps of v and t).  s and hs replace r and hr (the reference too
+// keeps s in r's place).
+
+// backward row of p^ (half 0) or s^ (half 1)
+template <class R, int MEM>
+struct RowBiBack : Row<R, MEM> {
+  int half;
+  bool first, mark_w;
+  double alpha, beta, omega;
+  double r, hr, v, hv, p, hp, x, pt;
+  __device__ __forceinline__ RowBiBack(const R& res, int hf, bool f, bool mw, double al, double be, double om)
+      : Row<R, MEM>(res), half(hf), first(f), mark_w(mw), alpha(al), beta(be), omega(om) {}
+  __device__ __forceinline__ void pre(int slot, int e) {
+    this->begin(slot, e);
+    r = this->get(kR);
+    hr = this->get(kHr);
+    if (half || !first) {
+      v = this->get(kV);
+      hv = this->get(kHv);
+    }
+    if (half) {
+      x = this->get(kX);
+      pt = ld<MEM>(this->zw(this->k.par ^ 1, slot) + e);
+    } else if (!first) {
+      p = this->get(kBp);
+      hp = this->get(kHp);
+    }
+  }
+  __device__ __forceinline__ void post(int slot, int e, bool writes, const double (&s)[1]) {
+    if (half) {
+      r = r - alpha * v;
+      hr = hr - alpha * hv;
+      x = x + alpha * pt;
+    } else {
+      p = first ? r : r + beta * (p - omega * v);
+      hp = first ? hr : hr + beta * (hp - omega * hv);
+    }
+    const double z = this->solve((half ? hr : hp) - s[0], e);
+    if (!writes) return;
+    double* now = this->zw(this->k.par, slot) + e;
+    double* old = this->zw(this->k.par ^ 1, slot) + e;
+    this->put_zw(now, unmarked(z));
+    this->put_zw(old, mark());
+    this->put_zw(old + 3, mark());
+    if (mark_w) this->put_zw(now + 3, mark());
+    if (half) {
+      this->put(kR, r);
+      this->put(kHr, hr);
+      this->put(kX, x);
+    } else {
+      this->put(kBp, p);
+      this->put(kHp, hp);
+    }
+  }
+};
+
+// forward row of v (half 0) or t (half 1); refresh: only hr from r
+template <class R, int MEM>
+struct RowBiFwd : Row<R, MEM> {
+  int half;
+  bool refresh;
+  double acc[2] = {0.0, 0.0};  // r~.v; t.s, t.t
+  double h, z, u, ds;
+  __device__ __forceinline__ RowBiFwd(const R& res, int hf, bool rf) : Row<R, MEM>(res), half(hf), refresh(rf) {}
+  __device__ __forceinline__ void pre(int slot, int e) {
+    this->begin(slot, e);
+    h = this->get(refresh ? kR : (half ? kHr : kHp));
+    z = u = ds = 0.0;
+    if (!refresh) {
+      if (this->k.o.dsig) ds = this->k.o.dsig[3 * (int64_t)slot + e];
+      z = ld<MEM>(this->zw(this->k.par, slot) + e);
+      u = this->get(half ? kR : kRt);
+    }
+  }
+  __device__ __forceinline__ void post(int slot, int e, bool writes, const double (&s)[2]) {
+    const double az = s[0] + h + ds * z;
+    const double t = (refresh ? h : az) - s[1];
+    const double w = this->solve(t, e);
+    if (!writes) return;
+    this->put_zw(this->zw(this->k.par ^ (refresh ? 1 : 0), slot) + 3 + e, unmarked(w));
+    if (refresh) {
+      this->put(kHr, t);
+    } else {
+      this->put(half ? kT : kV, az);
+      this->put(half ? kHt : kHv, t);
+      acc[0] += u * az;
+      acc[1] += az * az;
+    }
+  }
+};
+
+// x += omega s^, and r = s - omega t, hr = hs - omega ht with the partials r.r and
+// r~.r unless the iteration recomputes the residual
+template <class R, int MEM>
+__device__ __forceinline__ void bi_update_phase(const R& k, double omega, bool with_r, double (&acc)[2], int T) {
+  const ResidentOp& o = k.o;
+#pragma unroll 1
+  for (int64_t i = (int64_t)k.blk * T + threadIdx.x; i < 3 * (int64_t)o.ns; i += (int64_t)k.G * T) {
+    const int slot = (int)(i / 3), e = (int)(i % 3);
+    if (o.row_old[slot] < 0) continue;
+    double* b = rec(o, slot) + e * kRowsS;
+    st<MEM>(b + kX * kRowsS, ld<MEM>(b + kX * kRowsS) + omega * ld<MEM>(k.zw(k.par, slot) + e));
+    if (with_r) {
+      const double v = ld<MEM>(b + kR * kRowsS) - omega * ld<MEM>(b + kT * kRowsS);
+      st<MEM>(b + kR * kRowsS, v);
+      st<MEM>(b + kHr * kRowsS, ld<MEM>(b + kHr * kRowsS) - omega * ld<MEM>(b + kHt * kRowsS));
+      acc[0] += v * v;
+      acc[1] += v * ld<MEM>(b + kRt * kRowsS);
+    }
+  }
+  drain_stores();
+}
+// r~.r of a recomputed residual
+template <class R, int MEM>
+__device__ __forceinline__ double bi_rho_phase(const R& k, int T) {
+  const ResidentOp& o = k.o;
+  double acc = 0.0;
+#pragma unroll 1
+  for (int64_t i = (int64_t)k.blk * T + threadIdx.x; i < 3 * (int64_t)o.ns; i += (int64_t)k.G * T) {
+    const double* b = rec(o, (int)(i / 3)) + i % 3 * kRowsS;
+    acc += ld<MEM>(b + kR * kRowsS) * ld<MEM>(b + kRt * kRowsS);
+  }
+  return acc;
+}
+
+// `budget` BiCGSTAB iterations, as k_resident_cg
+template <int T, int K, int MEM>
+__global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
+  extern __shared__ double lds[];
+  using Res = Resident<T, K, MEM>;
+  Res k(o, lds);
+  KrylovState& st = *o.state;
+  double rho = st.rho, rho1 = st.rho1, alpha = st.alpha, omega = st.omega, resid = st.resid, dnrm2 = st.dnrm2;
+  double c2 = st.c2, ts = st.ts, tt = st.tt;
+  const double bnrm2 = st.bnrm2, tol = st.tol;
+  int iter = st.iter, error = 0;
+  const int maxit = st.maxit, nrec = st.nrec;
+  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+  bool refresh = !(st.resume & 1);  // hr has to be made from r first
+  bool done = false, xn_current = false;
+  uint64_t ticks[2] = {0, 0};  // forward and backward sweeps
+  k.par = st.resume >> 1;
+  double* const part0 = o.part;
+  double* const part1 = o.part + 2 * k.G;
+  int half = 0;
+  bool after_refresh = false;
+  k.begin(refresh ? 0 : 1);
+
+#pragma unroll 1
+  for (int n = 0; n < budget;) {
+    // p^ or s^, unless hr is made first
+    if (!refresh) {
+      const uint64_t t0 = wall_clock64();
+      k.par ^= 1;
+      const double beta = iter > 1 ? (rho / rho1) * (alpha / omega) : 0.0;
+      RowBiBack<Res, MEM> f(k, half, iter == 1, after_refresh, alpha, beta, omega);
+      k.template sweep<1>(1, k.par, f);
+      k.grid_sync();
+      after_refresh = false;
+      ticks[1] += wall_clock64() - t0;
+    }
+    double tot[2];
+    {
+      const uint64_t t0 = wall_clock64();
+      RowBiFwd<Res, MEM> f(k, half, refresh);
+      k.template sweep<2>(0, k.par ^ (refresh ? 1 : 0), f);
+      k.reduce(f.acc, part1, tot);
+      ticks[refresh ? 1 : 0] += wall_clock64() - t0;
+    }
+    if (refresh) {
+      double v[1] = {bi_rho_phase<Res, MEM>(k, T)}, t[1];
+      k.reduce(v, part0, t);
+      rho = t[0];
+      refresh = false;
+      after_refresh = true;
+      continue;
+    }
+    if (half == 0) {
+      c2 = tot[0];
+      alpha = rho / c2;
+      half = 1;
+      continue;
+    }
+    half = 0;
+    ts = tot[0];
+    tt = tot[1];
+    omega = ts / tt;
+    const bool periodic = iter % nrec == 0;
+    {
+      double v[2] = {0.0, 0.0};
+      bi_update_phase<Res, MEM>(k, omega, !periodic, v, T);
+      k.reduce(v, part0, tot);
+    }
+    xn_current = false;
+    if (!periodic) {
+      dnrm2 = tot[0];
+      resid = sqrt(dnrm2 / bnrm2);
+      if (writer) o.hist[iter - 1] = resid;
+    }
+    bool again = false;
+    if (periodic || resid <= tol) {
+      x_to_nodes(k);
+      k.full_sync();
+      double v[1] = {true_resid_phase(k)}, t[1];
+      k.reduce(v, part1, t);
+      dnrm2 = t[0];
+      resid = sqrt(dnrm2 / bnrm2);
+      xn_current = true;
+      if (writer && periodic) o.hist[iter - 1] = resid;
+      done = resid <= tol;
+      again = true;
+    }
+    if (done) break;
+    if (iter >= maxit) {
+      error = kErrNoconv;
+      iter = maxit + 1;
+      done = true;
+      break;
+    }
+    rho1 = rho;
+    rho = tot[1];
+    ++iter;
+    ++n;
+    if (again) {
+      refresh = true;
+      k.begin(0);
+    }
+  }
+  if (!xn_current) x_to_nodes(k);
+  if (writer) {
+    st.rho = rho;
+    st.rho1 = rho1;
+    st.alpha = alpha;
+    st.omega = omega;
+    st.c2 = c2;
+    st.ts = ts;
+    st.tt = tt;
+    st.resid = resid;
+    st.dnrm2 = dnrm2;
+    st.iter = iter;
+    st.error = error;
+    st.done = done ? 1 : 0;
+    st.resume = (refresh ? 0 : 1) | k.par << 1;
+    st.time_Ax += 1e-8 * (double)ticks[0];
+    st.time_precond += 1e-8 * (double)ticks[1];
+  }
+  if (MEM == kOneGroup) {
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < 2 * k.copy_size; i += T) o.zw[i] = k.zw0[i];
+  }
+}
+
 // ---- set-up ------------------------------------------------------------------
 // the blocks of every row from its SELL slice into the lanes of its task: K
 // consecutive blocks to a lane
@@ -833,11 +1100,12 @@ __global__ __launch_bounds__(kBlock) void k_resident_init(ResidentOp o, const do
   for (int64_t t = i0; t < o.ns; t += stride) {
     const int32_t i = o.row_old[t];
     double* b = rec(o, (int)t);
-    for (int v = 0; v < kAlu; ++v) b[v * kRowsS] = 0.0;
+    for (int v = kR; v < o.planes; ++v) b[v * kRowsS] = 0.0;
 #pragma unroll
     for (int e = 0; e < 3; ++e) {
       b[(kR + e) * kRowsS] = i >= 0 ? r[3 * (int64_t)i + e] : 0.0;
       b[(kX + e) * kRowsS] = i >= 0 ? o.xn[3 * (int64_t)i + e] : 0.0;
+      if (o.planes == kBiPlanes) b[(kRt + e) * kRowsS] = b[(kR + e) * kRowsS];  // r~ = r0
     }
   }
 }
@@ -849,7 +1117,7 @@ __global__ void k_resident_reset(uint32_t* sync) {
 
 template <int T, int K, int MEM>
 hipError_t launch(const ResidentOp& o, int grid, int budget, hipStream_t s) {
-  const auto f = k_resident_cg<T, K, MEM>;
+  const auto f = o.planes == kBiPlanes ? k_resident_bicg<T, K, MEM> : k_resident_cg<T, K, MEM>;
   const size_t lds = LdsMap<T>::bytes(o.ncolor, MEM == kOneGroup ? o.ns : 0);
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
@@ -878,7 +1146,7 @@ void resident_init(const ResidentOp& o, const ResidentShape& sh, const double* r
 }
 bool resident_one_group(int ncolor, int ns) { return LdsMap<512>::bytes(ncolor, ns) <= 160 * 1024; }
 
-hipError_t resident_cg(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s) {
+hipError_t resident_run(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s) {
   if (sh.grid == 1) {
     switch (sh.packets) {
       case 2: return launch<512, 2, kOneGroup>(o, 1, budget, s);

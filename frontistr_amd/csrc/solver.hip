@@ -1334,7 +1334,13 @@ static void enqueue_fcg_sym_iteration(Context& c, int32_t kind, bool spmv64, hip
   fcg_reliable(c.A.view, c.vx.as<double>(), c.vb.as<double>(), r, st, part, c.hist.as<double>(), c.stream);
 }
 
-// ---- resident SSOR-CG (resident.hip) ------------------------------------------------------
+// ---- resident SSOR-CG and SSOR-BiCGSTAB (resident.hip) ------------------------------------------------------
+static int32_t resident_no_memory(Context& c) {
+  for (DMem* m : {&c.res_color_task, &c.res_task, &c.res_row, &c.res_col, &c.res_val, &c.res_vec}) m->release();
+  c.res_packets = 0;
+  (void)hipGetLastError();
+  return 1;
+}
 // The packed structure: per direction the rows of a colour in slot order, cut
 // where the rows or the lanes of a task are full.
 static int32_t resident_tasks(Context& c, const ResidentShape& sh) {
@@ -1366,13 +1372,8 @@ static int32_t resident_tasks(Context& c, const ResidentShape& sh) {
   const size_t nblk = (size_t)kWave * K * task.size();
   if (c.res_color_task.ensure(sizeof(int32_t) * ct.size()) || c.res_task.ensure(sizeof(int4) * task.size()) ||
       c.res_row.ensure(sizeof(int2) * row.size()) || c.res_col.ensure(sizeof(int32_t) * nblk) ||
-      c.res_val.ensure(sizeof(double) * 9 * nblk) ||
-      c.res_vec.ensure(sizeof(double) * (kResidentPlanes * (size_t)ns + 16 * ((size_t)ns + 1))) ||
-      c.res_sync.ensure(sizeof(uint32_t) * kResidentSync)) {
-    for (DMem* m : {&c.res_color_task, &c.res_task, &c.res_row, &c.res_col, &c.res_val, &c.res_vec}) m->release();
-    (void)hipGetLastError();
-    return 1;
-  }
+      c.res_val.ensure(sizeof(double) * 9 * nblk))
+    return resident_no_memory(c);
   HIPC(hipMemcpyAsync(c.res_color_task.p, ct.data(), sizeof(int32_t) * ct.size(), hipMemcpyHostToDevice, c.stream));
   HIPC(hipMemcpyAsync(c.res_task.p, task.data(), sizeof(int4) * task.size(), hipMemcpyHostToDevice, c.stream));
   HIPC(hipMemcpyAsync(c.res_row.p, row.data(), sizeof(int2) * row.size(), hipMemcpyHostToDevice, c.stream));
@@ -1412,18 +1413,18 @@ static ResidentShape resident_shape(const Context& c) {
   return sh;
 }
 
-// Whether this solve can run resident: plain FP64 CG whose SSOR factors were
+// Whether this solve can run resident: plain FP64 CG or BiCGSTAB whose SSOR factors were
 // made from the present values (a recycled preconditioner has other L' and U'
 // than A), all columns internal, no couplings inside a colour, one application
 // per iteration, no constraint products; gathered records
 // within the 4 GiB of a buffer resource, the colours' ranges within LDS.
-static bool resident_fits(const Context& c, int32_t method, int32_t kind, int32_t iterpremax, bool mixed) {
-  return method == 1 && kind == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N &&
+static bool resident_fits(const Context& c, int32_t kind, int32_t iterpremax, bool mixed) {
+  return kind == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N &&
          c.ssor_gen == c.val_gen && c.ssor_proper && c.ssor_rows < 30000000 && c.ncolor <= 512;
 }
 
 // 1: no memory for the packed copy (the launch-per-colour solve needs none)
-static int32_t resident_setup(Context& c, const ResidentShape& sh) {
+static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t method) {
   ResidentOp& o = c.res;
   const int32_t ns = (int32_t)c.ssor_rows;
   const bool sym = c.res_packets != sh.packets;
@@ -1432,14 +1433,20 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh) {
     if (int32_t e = resident_tasks(c, sh)) return e;
     c.res_packets = sh.packets;
   }
+  const int32_t planes = method == 2 ? kResidentPlanesBi : kResidentPlanesCg;
+  const bool new_rec = sym || o.planes != planes;
+  if (new_rec && (c.res_vec.ensure(sizeof(double) * (planes * (size_t)ns + 16 * ((size_t)ns + 1))) ||
+                  c.res_sync.ensure(sizeof(uint32_t) * kResidentSync)))
+    return resident_no_memory(c);
   o.ns = ns;
+  o.planes = planes;
   o.rec = c.res_vec.as<double>();
-  o.zw = o.rec + kResidentPlanes * (size_t)ns;
+  o.zw = o.rec + planes * (size_t)ns;
+  if (new_rec || c.res_num != c.ssor_num) resident_alu(o, c.alu_ssor.as<double>(), c.ssor_R, c.stream);
   if (sym || c.res_num != c.ssor_num) {
     for (int d = 0; d < 2; ++d)
       resident_pack(d ? c.U.view : c.L.view, c.res_row.as<int2>() + d * (size_t)ns, sh.packets, c.res_col.as<int32_t>(),
                     c.res_val.as<double>(), sym, c.stream);
-    resident_alu(o, c.alu_ssor.as<double>(), c.ssor_R, c.stream);
     c.res_num = c.ssor_num;
   }
   o.dsig = nullptr;
@@ -1475,7 +1482,7 @@ constexpr int kResidentBudget = 512;
 static int32_t resident_solve(Context& c, const ResidentShape& sh) {
   resident_init(c.res, sh, c.vr.as<double>(), c.stream);
   for (;;) {
-    HIPC(resident_cg(c.res, sh, kResidentBudget, c.stream));
+    HIPC(resident_run(c.res, sh, kResidentBudget, c.stream));
     uint32_t abort = 0;
     HIPC(hipMemcpyAsync(&c.h_st[0], c.st.p, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
     HIPC(hipMemcpyAsync(&abort, c.res.sync + 64 * 9, sizeof(abort), hipMemcpyDeviceToHost, c.stream));
@@ -1981,10 +1988,10 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
       if (m->ensure(vbytes)) return HECMW33_ERROR_DEVICE;
   }
   ResidentShape shape;
-  if (resident_fits(c, method, kind, iterpremax, mixed)) {
+  if (resident_fits(c, kind, iterpremax, mixed)) {
     shape = resident_shape(c);
     if (shape.grid > 0) {
-      const int32_t e = resident_setup(c, shape);
+      const int32_t e = resident_setup(c, shape, method);
       if (e < 0) return e;
       if (e > 0) shape.grid = 0;
     }

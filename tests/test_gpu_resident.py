@@ -1,12 +1,14 @@
-"""The resident SSOR-CG kernel (csrc/resident.hip) against the plain-C restatement of
-hecmw_solve_CG (oracle/restate.c) and against the launch-per-colour solve, which a
+"""The resident SSOR-CG and SSOR-BiCGSTAB kernels (csrc/resident.hip) against the plain-C
+restatement of hecmw_solve_CG and hecmw_solve_BiCGSTAB (oracle/restate.c) and against the launch-per-colour solve, which a
 system with an external node takes.
 
 Both sides form the same sums in another order, so the residual histories differ by
 rounding: about 1e-16 per operation, 1e3 operations deep and amplified by the
 condition of these systems (up to 1e5) over the first iterations, hence 1e-8 on the
 first fifteen.  (The entries are relative to |b|: one at the level of 1e-7 or below
-holds rounding of 1e-16 |b| that is more than 1e-9 of it, and says nothing here.)  Solutions to a 1e-10 residual agree to 1e-6, the bar of every solve
+holds rounding of 1e-16 |b| that is more than 1e-9 of it, and says nothing here.)
+BiCGSTAB's polynomial amplifies rounding faster than CG's: five entries, and iteration
+counts within the tenth that its other tests allow.  Solutions to a 1e-10 residual agree to 1e-6, the bar of every solve
 here (the condition bounds the factor by 1e4).
 """
 import numpy as np
@@ -19,8 +21,8 @@ from tests.systems import random_system
 pytestmark = pytest.mark.gpu
 
 
-def _same_start(h, ref):
-    k = min(15, len(h), len(ref))
+def _same_start(h, ref, most=15):
+    k = min(most, len(h), len(ref))
     k = min([k] + [i for i in range(k) if ref[i] <= 1e-7])
     np.testing.assert_allclose(h[:k], ref[:k], rtol=1e-8)
 
@@ -104,6 +106,74 @@ def test_iteration_limit_and_residual_period(n, maxit):
         # the recurrence carries a rounding unit of its largest entry per iteration
         np.testing.assert_allclose(h, info["history"], rtol=1e-5, atol=maxit * 1.1e-16 * h.max())
         assert np.linalg.norm(x - xr) <= 1e-6 * np.linalg.norm(xr)
+
+
+@pytest.mark.parametrize("sigma", [1.0, 1.35])
+@pytest.mark.parametrize("name", sorted(SYSTEMS))
+def test_resident_bicgstab_matches_the_restatement(name, sigma):
+    make, groups = SYSTEMS[name]
+    m = make()
+    m.set_iter(3000)
+    m.set_method(2)
+    m.set_precond(1)
+    m.set_resid(1e-10)
+    m.set_sigma_diag(sigma)
+    x, res, h, resident = _device_solve(m)
+    assert resident > 0 and (groups is None or resident == groups), resident
+    xr, info = restate.solve_krylov(m)
+    assert res.error == 0 and info["error"] == 0
+    assert abs(res.iter - info["iter"]) <= 2 + 0.1 * info["iter"], (res.iter, info["iter"])
+    assert res.resid <= 1e-10
+    r = m.B[:3 * m.N] - restate.matvec(m, x)
+    assert np.linalg.norm(r) <= 1.001e-10 * np.linalg.norm(m.B)
+    assert np.linalg.norm(x - xr) <= 1e-6 * np.linalg.norm(xr)
+    _same_start(h, info["history"], 5)
+    x2, res2, h2, launches = _device_solve(_with_external_node(m))
+    assert launches == 0
+    _same_start(h, h2, 5)
+
+
+@pytest.mark.parametrize("maxit", [1, 2, 99, 100, 101])
+def test_bicgstab_iteration_limit_and_residual_period(maxit):
+    """NOCONV at MAXIT, on both sides of the iteration that recomputes the residual (every 100)."""
+    m = fa.gen_hex8(11, kind="lognormal", seed=4)
+    m.set_iter(maxit)
+    m.set_method(2)
+    m.set_precond(1)
+    m.set_resid(1e-14)
+    x0 = np.random.default_rng(7).standard_normal(3 * m.NP) * 1e-3
+    x, res, h, resident = _device_solve(m, x0)
+    _, info = restate.solve_krylov(m, x0=x0)
+    assert resident > 0
+    assert (res.iter, res.error) == (info["iter"], info["error"]) == (maxit + 1, 3001)
+    _same_start(h, info["history"], 5)
+    # RESID is the residual of the x that is returned
+    r = m.B - restate.matvec(m, x)
+    assert abs(np.linalg.norm(r) / np.linalg.norm(m.B) - res.resid) <= 1e-6 * res.resid + maxit * 1.1e-16 * h.max()
+
+
+def test_method_change_on_one_context():
+    """CG, BiCGSTAB and CG again on the same context: the row records change layout."""
+    import torch
+    m = fa.gen_hex8(9, kind="lognormal", seed=3)
+    m.set_iter(2000)
+    m.set_precond(1)
+    m.set_resid(1e-10)
+    ctx = fa.DeviceContext()
+    ctx.load(m)
+    b = torch.from_numpy(m.B).cuda()
+    out = []
+    for method in (1, 2, 1):
+        ia = m.Iarray.copy()
+        ia[m.I_METHOD - 1] = method
+        ia[m.I_FLAG_NUMFACT - 1] = ia[m.I_FLAG_SYMBFACT - 1] = 0
+        x = torch.zeros_like(b)
+        torch.cuda.synchronize()
+        res = ctx.solve_device(b.data_ptr(), x.data_ptr(), ia, m.Rarray)
+        assert res.error == 0 and ctx.info()["resident"] > 0
+        out.append(x.cpu().numpy())
+    assert np.array_equal(out[0], out[2])
+    assert np.linalg.norm(out[1] - out[0]) <= 1e-6 * np.linalg.norm(out[0])
 
 
 def test_more_iterations_than_one_launch():
