@@ -34,6 +34,7 @@ SOURCES = [
     ("coarse.hip", True),
     ("noalloc.hip", True),
     ("resident.hip", True),
+    ("chol.hip", True),
 ]
 
 
@@ -58,8 +59,7 @@ def build(jobs=4, verbose=False):
     with cf.ThreadPoolExecutor(jobs) as ex:
         objs = list(ex.map(lambda s: compile_one(s[0], s[1], objdir), SOURCES))
     out = os.path.join(LIBDIR, "libhecmw33.so")
-    cmd = [HIPCC, "--offload-arch=" + ARCH, "-shared", "-fopenmp", "-o", out + ".tmp"] + objs + [
-        "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lrocsolver", "-lrocblas"]
+    cmd = [HIPCC, "--offload-arch=" + ARCH, "-shared", "-fopenmp", "-o", out + ".tmp"] + objs
     p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if p.returncode != 0:
         raise RuntimeError("link failed: %s\n%s" % (" ".join(cmd), p.stdout))

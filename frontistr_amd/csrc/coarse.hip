@@ -134,34 +134,29 @@ __global__ void k_coarse_unit_pivots(int32_t nc, double* __restrict__ E, int32_t
   if (k < nc && E[(int64_t)k * lda + k] == 0.0) E[(int64_t)k * lda + k] = 1.0;
 }
 
-// W = E^-1 in FP32, full symmetric from the lower triangle the inverse leaves
-__global__ void k_coarse_inv32(int32_t nc, const double* __restrict__ Ei, int32_t lda, float* __restrict__ W,
-                               int32_t ldw) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)nc * ldw) return;
-  const int row = (int)(t / ldw), col = (int)(t % ldw);
-  float v = 0.f;
-  if (col < nc) {
-    const int lo = row > col ? row : col, hi = row > col ? col : row;  // (lo, hi) is in the lower triangle
-    v = (float)Ei[(int64_t)hi * lda + lo];
+// W = the full array mirrored from the lower triangle that coarse_factor leaves
+// row-major in E's upper half ((r, c), c <= r, at E[r lda + c]): E^-1 in FP32, or
+// L^-1 below and on the diagonal with L^-T above in FP64 (with the learned modes E
+// is too ill-conditioned for FP32).  64 x 64 tiles through LDS, so that both halves
+// are written in rows.
+template <typename T>
+__global__ __launch_bounds__(kCoarseBlock) void k_coarse_mirror(int32_t nc, const double* __restrict__ E, int32_t lda,
+                                                                  T* __restrict__ W, int32_t ldw) {
+  const int r0 = 64 * blockIdx.x, c0 = 64 * blockIdx.y;
+  if (c0 > r0) return;
+  __shared__ double tile[64][65];
+  for (int k = threadIdx.x; k < 64 * 64; k += kCoarseBlock) {
+    const int r = r0 + k / 64, c = c0 + k % 64;
+    double v = r < nc && c < nc ? E[(int64_t)max(r, c) * lda + min(r, c)] : 0.0;
+    tile[k / 64][k % 64] = v;
+    if (r < nc && c < ldw) W[(int64_t)r * ldw + c] = (T)v;
   }
-  W[t] = v;
-}
-
-// W = the lower triangle of Ei mirrored into a full FP64 array: L^-1 below and
-// on the diagonal, L^-T above (the twelve-mode step: with the learned modes E
-// is too ill-conditioned for FP32)
-__global__ void k_coarse_inv64(int32_t nc, const double* __restrict__ Ei, int32_t lda, double* __restrict__ W,
-                               int32_t ldw) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)nc * ldw) return;
-  const int row = (int)(t / ldw), col = (int)(t % ldw);
-  double v = 0.0;
-  if (col < nc) {
-    const int lo = row > col ? row : col, hi = row > col ? col : row;
-    v = Ei[(int64_t)hi * lda + lo];
+  if (r0 == c0) return;
+  __syncthreads();
+  for (int k = threadIdx.x; k < 64 * 64; k += kCoarseBlock) {
+    const int r = c0 + k / 64, c = r0 + k % 64;
+    if (r < nc && c < ldw) W[(int64_t)r * ldw + c] = (T)tile[k % 64][k / 64];
   }
-  W[t] = v;
 }
 
 // y = W c in FP64, one wavefront per row, double2 loads (ldw a multiple of 64).
@@ -868,14 +863,12 @@ void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, c
   k_coarse_unit_pivots<<<(op.nc + 255) / 256, 256, 0, s>>>(op.nc, E, lda);
 }
 
-void coarse_inverse_f64(const CoarseOp& op, const double* Ei, int32_t lda, hipStream_t s) {
-  const int64_t ne = (int64_t)op.nc * op.ldw;
-  k_coarse_inv64<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(op.nc, Ei, lda, op.W64, op.ldw);
-}
-
-void coarse_inverse_f32(const CoarseOp& op, const double* Ei, int32_t lda, hipStream_t s) {
-  const int64_t ne = (int64_t)op.nc * op.ldw;
-  k_coarse_inv32<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(op.nc, Ei, lda, op.W, op.ldw);
+void coarse_mirror(const CoarseOp& op, const double* E, int32_t lda, hipStream_t s) {
+  const dim3 g((unsigned)(op.ldw / 64), (unsigned)(op.ldw / 64));
+  if (op.nm == 12)
+    k_coarse_mirror<double><<<g, kCoarseBlock, 0, s>>>(op.nc, E, lda, op.W64, op.ldw);
+  else
+    k_coarse_mirror<float><<<g, kCoarseBlock, 0, s>>>(op.nc, E, lda, op.W, op.ldw);
 }
 
 int coarse_apply(const CoarseOp& op, int32_t n, const float* r, float* z, const float* q, const KrylovState* st,

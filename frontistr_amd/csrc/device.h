@@ -347,10 +347,15 @@ struct CoarseOp {
 // (Eblk: nm*nm doubles per pair)
 void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, const int32_t* pa, const int32_t* pb,
                      const int32_t* pn_ptr, const int32_t* pn, double* Eblk, double* E, int32_t lda, hipStream_t s);
-// the iterations' copies: E^-1 (potri's lower triangle) mirrored into FP32 W,
-// or L^-1 (trtri's lower triangle) mirrored into FP64 W64
-void coarse_inverse_f32(const CoarseOp& op, const double* Ei, int32_t lda, hipStream_t s);
-void coarse_inverse_f64(const CoarseOp& op, const double* Ei, int32_t lda, hipStream_t s);
+// Cholesky factorization and inverse of the dense banded E (chol.hip): E is
+// column-major of order coarse_padded(nc), half bandwidth `band`; its upper triangle
+// receives, row-major, L^-1 (E = L L^T) or with `both` E^-1.  Linv: 64 doubles per
+// (padded) row; *info is set when E is not positive definite.
+int32_t coarse_padded(int32_t nc);
+void coarse_factor(double* E, int32_t nc, int32_t band, double* Linv, bool both, int32_t* info, hipStream_t s);
+// the iterations' copies: E^-1 in FP32 (W) or, with twelve modes, L^-1 in FP64 (W64),
+// mirrored into full arrays
+void coarse_mirror(const CoarseOp& op, const double* E, int32_t lda, hipStream_t s);
 // The symmetric two-level step (W = A Z per node and touched aggregate):
 // build W from the symbolic node-major lists ncnt/nagg into the compacted
 // sc (per node: first slot, count) / aggW / W, dropping the entries that are

@@ -16,8 +16,6 @@
 //   ALU    : 3x3 LU of the diagonal blocks, 9-plane slice layout
 //   vectors: b, x, r, z, p, q (+ BiCGSTAB's) of 3*NP doubles
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <chrono>
@@ -311,9 +309,8 @@ struct Context {
   int32_t coarse_nm_num = 0;      // modes per aggregate of the E^-1 built (6 or 12)
   int32_t coarse_w_nm = 0;        // modes per aggregate of the A Z built
   int64_t coarse_nw = 0;          // node-aggregate entries of A Z
-  DMem cg_agg, cg_aptr, cg_anodes, cg_dv, cg_pa, cg_pb, cg_pnptr, cg_pn, cg_Eblk, cg_E, cg_W, cg_cv, cg_tv, cg_yv, cg_info;
+  DMem cg_agg, cg_aptr, cg_anodes, cg_dv, cg_pa, cg_pb, cg_pnptr, cg_pn, cg_Eblk, cg_E, cg_W, cg_cv, cg_tv, cg_yv, cg_info, cg_Linv;
   DMem cg_ncnt, cg_nagg, cg_AZ, cg_sc, cg_aggW, cg_kept, vr1_32, vt32, vw32, vaz32;
-  rocblas_handle blas = nullptr;
   // multipoint constraints (hecMESH%mpc) for the MPC-CG product T^T A T
   // (Iarray 83 set, as hecmw_solve_iterative sets it for MPC_METHOD = 2)
   int32_t mpc_n = 0, mpc_N = 0;  // constraints given, for N internal nodes
@@ -358,11 +355,10 @@ struct Context {
                     &vmask})
       m->release();
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
-                    &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
+                    &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
       m->release();
     for (DMem* m : {&res_color_task, &res_task, &res_row, &res_col, &res_val, &res_vec, &res_sync, &res_dsig})
       m->release();
-    if (blas) rocblas_destroy_handle(blas);
     for (DMem* m : {&mpc_slave, &mpc_mptr, &mpc_mdof, &mpc_mval, &mpc_tptr, &mpc_tslave, &mpc_tval, &mpc_w1, &mpc_w2})
       m->release();
     for (DMem* m : {&dD, &dAL, &dAU, &row_old, &node_slot, &alu_ssor, &row_diag, &alu_diag, &alu_ssor32, &alu_diag32, &vr32,
@@ -1152,39 +1148,9 @@ static int32_t coarse_symbolic(Context& c, int32_t target) {
   return 0;
 }
 
-// E = Z^T A Z on the device with nm modes per aggregate (6 rigid-body; 12 with
-// the learned ones in cg_xm), Cholesky factor and inverse (six modes) or
-// inverse factor (twelve) in FP64 (chol_band, then rocSOLVER), then the copy the iterations
-// read
-// Cholesky E = L L^T of the coarse matrix (lower, column-major, n x n), which
-// is banded: aggregates couple only when their cells touch, and the cells are
-// numbered in order of first appearance over the nodes, so on a mesh numbered
-// along its axes every nonzero lies within `band` rows below the diagonal (at
-// 160^3 with 1000 aggregates: 1332 of 12,000 rows), and so does every nonzero
-// of L.  Right-looking over panels of kCholPanel columns: rocSOLVER factors the
-// panel's diagonal block, a triangular solve gives the at most `band` rows
-// below it, and a rank-kb product updates the trailing band; the zeros outside
-// the band are never touched.  info[p] != 0: panel p's block is not positive
-// definite.  Same operations as the dense right-looking factorization, minus
-// the ones on zeros.
-constexpr int32_t kCholPanel = 256;
-static int32_t chol_band(rocblas_handle h, int32_t n, double* A, int32_t band, int32_t* info) {
-  const double one = 1.0, mone = -1.0;
-  for (int32_t k = 0, p = 0; k < n; k += kCholPanel, ++p) {
-    const int32_t kb = std::min(kCholPanel, n - k);
-    double* Akk = A + (size_t)k * n + k;
-    if (rocsolver_dpotrf(h, rocblas_fill_lower, kb, Akk, n, info + p) != rocblas_status_success) return 1;
-    const int32_t m = std::min(n - k - kb, band);
-    if (m <= 0) continue;
-    if (rocblas_dtrsm(h, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,
-                      rocblas_diagonal_non_unit, m, kb, &one, Akk, n, Akk + kb, n) != rocblas_status_success ||
-        rocblas_dsyrk(h, rocblas_fill_lower, rocblas_operation_none, m, kb, &mone, Akk + kb, n, &one,
-                      A + (size_t)(k + kb) * n + k + kb, n) != rocblas_status_success)
-      return 1;
-  }
-  return 0;
-}
-
+// E = Z^T A Z on the device with nm modes per aggregate (6 rigid-body; 12 with the
+// learned ones in cg_xm), its Cholesky factor and inverse (six modes) or inverse factor
+// (twelve) in FP64, then the copy the iterations read
 static int32_t coarse_numeric(Context& c, int32_t nm) {
   CoarseOp& op = c.coarse;
   op.nm = nm;
@@ -1194,10 +1160,10 @@ static int32_t coarse_numeric(Context& c, int32_t nm) {
   const int32_t nc = op.nc;
   // six modes: E^-1, c and y in FP32; twelve: in FP64
   const size_t we = nm == 12 ? sizeof(double) : sizeof(float);
-  const int32_t npanel = (nc + kCholPanel - 1) / kCholPanel;
-  if (c.cg_info.ensure(sizeof(int32_t) * (npanel + 1)) ||
+  const int32_t lda = coarse_padded(nc);
+  if (c.cg_info.ensure(sizeof(int32_t)) || c.cg_Linv.ensure(sizeof(double) * 64 * (size_t)lda) ||
       c.cg_Eblk.ensure(sizeof(double) * nm * nm * (size_t)std::max(c.coarse_npair, 1)) ||
-      c.cg_E.ensure(sizeof(double) * (size_t)nc * nc) || c.cg_W.ensure(we * (size_t)nc * op.ldw) ||
+      c.cg_E.ensure(sizeof(double) * (size_t)lda * lda) || c.cg_W.ensure(we * (size_t)nc * op.ldw) ||
       c.cg_cv.ensure(we * op.ldw) || c.cg_yv.ensure(we * op.ldw) || c.cg_tv.ensure(we * op.ldw))
     return HECMW33_ERROR_DEVICE;
   op.W = nm == 12 ? nullptr : c.cg_W.as<float>();
@@ -1209,45 +1175,23 @@ static int32_t coarse_numeric(Context& c, int32_t nm) {
   op.tv64 = nm == 12 ? c.cg_tv.as<double>() : nullptr;
   HIPC(hipMemsetAsync(c.cg_cv.p, 0, we * op.ldw, c.stream));
   HIPC(hipMemsetAsync(c.cg_tv.p, 0, we * op.ldw, c.stream));
-  HIPC(hipMemsetAsync(c.cg_E.p, 0, sizeof(double) * (size_t)nc * nc, c.stream));
+  HIPC(hipMemsetAsync(c.cg_E.p, 0, sizeof(double) * (size_t)lda * lda, c.stream));
+  HIPC(hipMemsetAsync(c.cg_info.p, 0, sizeof(int32_t), c.stream));
   coarse_assemble(c.A.view, op, c.coarse_npair, c.cg_pa.as<int32_t>(), c.cg_pb.as<int32_t>(),
-                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.cg_Eblk.as<double>(), c.cg_E.as<double>(), nc,
+                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.cg_Eblk.as<double>(), c.cg_E.as<double>(), lda,
                   c.stream);
   HIPC(hipGetLastError());
-  if (!c.blas && rocblas_create_handle(&c.blas) != rocblas_status_success) {
-    c.blas = nullptr;
-    set_error("rocblas_create_handle failed");
-    return HECMW33_ERROR_DEVICE;
-  }
-  if (rocblas_set_stream(c.blas, c.stream) != rocblas_status_success) {
-    set_error("rocblas_set_stream failed");
-    return HECMW33_ERROR_DEVICE;
-  }
-  // six modes: E^-1 (potri) for one FP32 product per coarse solve; twelve:
-  // L^-1 (trtri) for two FP64 triangular products, y = L^-T (L^-1 c), the
-  // same bytes read without forming L^-T L^-1 (at 12,000 coarse unknowns
-  // potri takes 57 ms, trtri 22 ms)
-  int32_t* info = c.cg_info.as<int32_t>();
+  // six modes: E^-1 for one FP32 product per coarse solve; twelve: L^-1 for two FP64
+  // triangular products, y = L^-T (L^-1 c), the same bytes read without forming
+  // L^-T L^-1.  E's bandwidth follows from the coupled aggregate pairs.
   const int32_t band = std::max(0, std::min(nc - 1, nm * (c.coarse_band_agg + 1) - 1));
-  if (chol_band(c.blas, nc, c.cg_E.as<double>(), band, info) ||
-      (nm == 12 ? rocsolver_dtrtri(c.blas, rocblas_fill_lower, rocblas_diagonal_non_unit, nc, c.cg_E.as<double>(), nc,
-                                   info + npanel)
-                : rocsolver_dpotri(c.blas, rocblas_fill_lower, nc, c.cg_E.as<double>(), nc, info + npanel)) !=
-          rocblas_status_success) {
-    set_error("coarse factorization (rocSOLVER potrf/potri/trtri, rocBLAS trsm/syrk) failed");
-    return HECMW33_ERROR_DEVICE;
-  }
-  std::vector<int32_t> hinfo(npanel + 1, 0);
-  HIPC(hipMemcpyAsync(hinfo.data(), info, sizeof(int32_t) * (npanel + 1), hipMemcpyDeviceToHost, c.stream));
+  coarse_factor(c.cg_E.as<double>(), nc, band, c.cg_Linv.as<double>(), nm != 12, c.cg_info.as<int32_t>(), c.stream);
+  int32_t info = 0;
+  HIPC(hipMemcpyAsync(&info, c.cg_info.p, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
   HIPC(hipStreamSynchronize(c.stream));
-  c.coarse_ok = std::all_of(hinfo.begin(), hinfo.end(), [](int32_t v) { return v == 0; });
+  c.coarse_ok = info == 0;
   c.coarse_w_valid = false;
-  if (c.coarse_ok) {
-    if (nm == 12)
-      coarse_inverse_f64(op, c.cg_E.as<double>(), nc, c.stream);
-    else
-      coarse_inverse_f32(op, c.cg_E.as<double>(), nc, c.stream);
-  }
+  if (c.coarse_ok) coarse_mirror(op, c.cg_E.as<double>(), lda, c.stream);
   HIPC(hipGetLastError());
   c.coarse_num = true;
   c.coarse_nm_num = nm;
