@@ -34,6 +34,7 @@ SOURCES = [
     ("coarse.hip", True),
     ("noalloc.hip", True),
     ("resident.hip", True),
+    ("resident_diag.hip", True),
     ("chol.hip", True),
 ]
 

@@ -240,7 +240,7 @@ void bi_update(int64_t n3, const double* pt, const double* stv, const double* t,
 // have value 0 and column ns, a record that is always there.  The tasks of L'
 // come first, then those of U'.
 constexpr int kResidentGridMax = 256;   // workgroups (one per CU)
-constexpr int kResidentSync = 64 * 10;  // words of the grid barrier's counters
+constexpr int kResidentSync = 640 + 12 * kResidentGridMax;  // words: abort flag, counts, entries of the exchanges
 constexpr int kResidentPlanesCg = 27;   // of 16 slots in a row record: the LU and six vectors (CG)
 constexpr int kResidentPlanesBi = 39;   // or ten (BiCGSTAB)
 constexpr int kResidentPackets = 4;     // most blocks per lane
@@ -261,7 +261,6 @@ struct ResidentOp {
   double* zw = nullptr;                 // the gathered vectors, two copies of ns + 1 records
   double* xn = nullptr;               // x in node order
   const double* b = nullptr;          // right-hand side in node order
-  double* part = nullptr;
   double* hist = nullptr;
   uint32_t* sync = nullptr;
   KrylovState* state = nullptr;
@@ -283,6 +282,32 @@ bool resident_one_group(int ncolor, int ns);
 // up to `budget` iterations; a cooperative launch, so that every workgroup
 // is on the GPU before the first grid barrier
 hipError_t resident_run(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s);
+
+// ---- resident CG with block-diagonal scaling (resident_diag.hip) -----------------
+// Task t: the rows task[t].x .. + task[t].y - 1 of A, at most kResidentRows, whole
+// aligned groups of four (rows past the last are empty).  A row takes
+// ceil(blocks / kDiagK) lanes; lane[64 t + l] says which: row | part << 4 | place of
+// its sums << 14, or -1; the places of a row are consecutive from row[].x on.
+constexpr int kDiagK = 7;
+struct DiagOp {
+  Sell<double> A;
+  const int4* task = nullptr;
+  const int32_t* lane = nullptr;
+  const int2* row = nullptr;       // first place, lanes
+  int32_t ntasks = 0, n = 0;
+  int32_t zero_rec = 0, ring = 0;  // the record that stays zero; copies in the ring
+  int64_t copy = 0;                // doubles of a copy: records {z0 z1 z2 -}
+  double* z = nullptr;
+  const double* alu = nullptr;     // LU of the diagonal blocks, planes of kRowsA rows
+  double *x = nullptr, *r = nullptr, *p = nullptr, *q = nullptr;
+  const double* b = nullptr;
+  double* hist = nullptr;
+  uint32_t* sync = nullptr;
+  KrylovState* state = nullptr;
+};
+size_t diag_lds_bytes(int ntasks, int grid);  // LDS of a workgroup
+// up to `budget` iterations, as resident_run
+hipError_t resident_diag_run(const DiagOp& o, int grid, int budget, hipStream_t s);
 
 // ---- flexible CG with FP32 operators and FP64 recurrences ------------------------
 // z32 = M^-1 r32 in FP32 (kind 0 copy, 1 SSOR, 3 DIAG)

@@ -49,76 +49,11 @@
 #include <cstdint>
 
 #include "device.h"
+#include "resident.h"
 #include "rows.h"
 
 namespace hecmw33 {
 namespace {
-
-constexpr int32_t kErrNoconv = 3001;
-constexpr int32_t kErrDivergeMat = 3002;
-constexpr int32_t kErrDivergePc = 3003;
-constexpr int32_t kErrDivergeNan = 3004;
-
-// How the waves exchange vectors: between workgroups every exchanged value is
-// written and read at agent scope (sc1: past the caches that other XCDs do not
-// see); a single workgroup keeps the gathered vectors in LDS.
-enum Exchange : int { kOneGroup = 0, kGrid = 1 };
-
-constexpr uint64_t kWaitTicks = 20ull * 100000000ull;  // 20 s of the 100 MHz wall clock
-
-template <int MEM>
-__device__ __forceinline__ double ld(const double* p) {
-  if (MEM == kGrid) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return *p;
-}
-template <int MEM>
-__device__ __forceinline__ void st(double* p, double v) {
-  if (MEM == kGrid)
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else
-    *p = v;
-}
-
-// The mark of an entry that has not been computed: a quiet NaN with a payload
-// that no computed value keeps (unmarked replaces it by the plain NaN).
-constexpr int kMarkHi = 0x7FFADEAD;
-__device__ __forceinline__ double mark() { return __hiloint2double(kMarkHi, 0); }
-__device__ __forceinline__ bool marked(double v) { return __double2hiint(v) == kMarkHi; }
-__device__ __forceinline__ double unmarked(double v) {
-  return marked(v) ? __hiloint2double(0x7FF80000, 0) : v;
-}
-
-// barrier of the workgroup that orders LDS but leaves global loads in flight
-// (__syncthreads would wait for the prefetched matrix data)
-__device__ __forceinline__ void wg_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-}
-// this wave's stores have completed
-__device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// orders a wave's own LDS accesses (the LDS serves a wave in order)
-__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
-// o.sync: [0] root count, [64 (1 + i)] count of group i, [64 * 9] abort
-__device__ __forceinline__ uint32_t cnt_add(uint32_t* c) {
-  return __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t cnt_get(const uint32_t* c) {
-  return __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void cnt_set(uint32_t* c, uint32_t v) {
-  __hip_atomic_store(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <int J>
-__device__ __forceinline__ double quad_bcast(double v) {
-  constexpr int ctrl = J | (J << 2) | (J << 4) | (J << 6);
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
 
 // The gathered vectors z and w of a row share a record {z0 z1 z2 w0 w1 w2}, of 64
 // bytes in memory, read with 16-byte loads: three requests for both vectors,
@@ -154,23 +89,26 @@ struct LdsMap {
 };
 
 template <int T, int K, int MEM>
-struct Resident {
+struct Resident : GridGroup<T, MEM> {
   using Map = LdsMap<T>;
-  static constexpr int kWaves = T / kWave;
+  using Group = GridGroup<T, MEM>;
+  using Group::blk;
+  using Group::dead;
+  using Group::G;
+  using Group::kWaves;
+  using Group::lane;
+  using Group::wave;
   static constexpr int kRec = MEM == kGrid ? 8 : 6;  // doubles of a gathered record
 
   const ResidentOp& o;
   __amdgpu_buffer_rsrc_t rsrc;
   double* zw0;           // the two copies of the gathered records, copy_size doubles each
   int64_t copy_size;
-  double *prod, *red;
+  double* prod;
   uint32_t* fin;
   const int2* range;
-  int lane, wave, G, blk;
   int par = 0;           // copy that holds the present z and w
-  uint32_t epoch = 0;    // grid barriers passed
   uint32_t fin0 = 0;     // tasks finished before this sweep
-  bool dead = false;     // a wait ran out (this wave's view): go on without waiting
   // the wave's next task: its place in the workgroup's order of the sweep, its
   // colour step and the tasks before that, its rows and lanes, its matrix data
   int j, step, before;
@@ -178,13 +116,8 @@ struct Resident {
   double v[K][9];
   int32_t c[K];
 
-  __device__ __forceinline__ Resident(const ResidentOp& op, double* lds) : o(op) {
-    lane = threadIdx.x & (kWave - 1);
-    wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    G = gridDim.x;
-    blk = xcd_block(blockIdx.x, G);
+  __device__ __forceinline__ Resident(const ResidentOp& op, double* lds) : Group(op.sync, lds + Map::red), o(op) {
     prod = lds + Map::prod + wave * kWave * kComp;
-    red = lds + Map::red;
     fin = reinterpret_cast<uint32_t*>(lds + Map::fin);
     int2* rg = reinterpret_cast<int2*>(lds + Map::range);
     range = rg;
@@ -220,106 +153,6 @@ struct Resident {
   }
 
   __device__ __forceinline__ double* zw(int cp, int slot) const { return zw0 + cp * copy_size + (int64_t)kRec * slot; }
-
-  // a wait that has run long: whether to give it up
-  __device__ __forceinline__ bool give_up(uint64_t& t0) {
-    const uint64_t now = wall_clock64();
-    if (t0 == 0) t0 = now;
-    if (now - t0 > kWaitTicks) cnt_set(o.sync + 64 * 9, 1u);
-    return cnt_get(o.sync + 64 * 9) != 0;
-  }
-
-  // Grid barrier, by wave 0.  A two-level count keeps the arrivals of many
-  // workgroups from queueing on one address (256 workgroups: 2.3 us against
-  // 3.7 us for a single counter; below 96 the single counter is faster, 1.4 us
-  // at 64).
-  __device__ __forceinline__ void arrive_and_wait() {
-    ++epoch;
-    if (lane != 0 || dead) return;
-    uint32_t target;
-    if (G >= 96) {
-      const uint32_t g = blockIdx.x % 8, members = (G - g + 7) / 8;
-      if (cnt_add(o.sync + 64 * (1 + g)) + 1 == members * epoch) cnt_add(o.sync);
-      target = 8 * epoch;
-    } else {
-      cnt_add(o.sync);
-      target = (uint32_t)G * epoch;
-    }
-    uint64_t t0 = 0;
-    for (uint32_t spins = 1; (int32_t)(cnt_get(o.sync) - target) < 0; ++spins)
-      if ((spins & 1023u) == 0 && give_up(t0)) {
-        dead = true;
-        break;
-      }
-  }
-  // grid barrier for stores that the callers have drained
-  __device__ __forceinline__ void grid_sync() {
-    wg_barrier();
-    if (MEM == kOneGroup) return;
-    if (wave == 0) arrive_and_wait();
-    wg_barrier();
-  }
-  // barrier for plain stores too: x in node order, which the product reads
-  // through the caches
-  __device__ __forceinline__ void full_sync() {
-    drain_stores();
-    wg_barrier();
-    if (MEM == kOneGroup) return;
-    if (wave == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      arrive_and_wait();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    wg_barrier();
-  }
-
-  // totals of K2 per-lane sums over the grid, the same on every thread: a wave
-  // tree, the workgroup's waves in order, then a fixed tree over the
-  // workgroups.  Also a grid barrier, for stores that the callers have drained.
-  template <int K2>
-  __device__ __forceinline__ void reduce(const double (&in)[K2], double* part, double (&tot)[K2]) {
-#pragma unroll
-    for (int k = 0; k < K2; ++k) {
-      const double w = wave_sum(in[k]);
-      if (lane == 0) red[k * kWaves + wave] = w;
-    }
-    wg_barrier();
-    if (wave == 0) {
-      double s = 0.0;
-      if (lane < K2) {
-        s = red[lane * kWaves];
-        for (int w = 1; w < kWaves; ++w) s += red[lane * kWaves + w];
-      }
-      if (MEM == kGrid) {
-        if (lane < K2) __hip_atomic_store(part + lane * G + blk, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        drain_stores();
-        arrive_and_wait();
-        constexpr int kPer = kResidentGridMax / kWave;
-        double u[K2][kPer];
-#pragma unroll
-        for (int k = 0; k < K2; ++k)
-#pragma unroll
-          for (int q = 0; q < kPer; ++q) {
-            const int i = lane + q * kWave;
-            u[k][q] = i < G ? __hip_atomic_load(part + k * G + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-          }
-#pragma unroll
-        for (int k = 0; k < K2; ++k) {
-          double t = u[k][0];
-#pragma unroll
-          for (int q = 1; q < kPer; ++q) t += u[k][q];
-          t = wave_sum(t);
-          if (lane == 0) red[2 * kWaves + k] = t;
-        }
-      } else if (lane < K2) {
-        red[2 * kWaves + lane] = s;
-      }
-    }
-    wg_barrier();
-#pragma unroll
-    for (int k = 0; k < K2; ++k) tot[k] = red[2 * kWaves + k];
-    wg_barrier();
-  }
 
   // The wave's place j in the workgroup's order of the sweep in direction d (0
   // forward, 1 backward): its task (-1: past the end), the step's number and
@@ -393,7 +226,7 @@ struct Resident {
         more |= want[k];
       }
       if (!__any(more) || dead) break;
-      if ((spins & 1023u) == 0) dead = __any(lane == 0 && give_up(t0));
+      if ((spins & 1023u) == 0) dead = __any(lane == 0 && this->give_up(t0));
     }
   }
 
@@ -678,8 +511,6 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
   uint64_t ticks[2] = {0, 0};  // forward and backward sweeps
   k.par = st.resume >> 1;
   k.begin(0);
-  double* const part0 = o.part;
-  double* const part1 = o.part + 2 * k.G;
 
 #pragma unroll 1
   for (int n = 0; n < budget; ++n) {
@@ -690,7 +521,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
       RowCgFwd<Res, MEM> f(k, iter > 1 ? rho / rho1 : 0.0, iter == 1, refresh);
       k.template sweep<2>(0, k.par ^ (refresh ? 1 : 0), f);
       double tot[1];
-      k.reduce(f.acc, part1, tot);
+      k.reduce(f.acc, tot);
       if (!refresh) c1 = tot[0];
     }
     uint64_t t1 = wall_clock64();
@@ -708,7 +539,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
       xn_current = false;
       if (periodic || iter >= maxit) {
         double v[1] = {cg_update_phase(k, alpha, !periodic)}, tot[1];
-        k.reduce(v, part0, tot);
+        k.reduce(v, tot);
         if (!periodic) dnrm2 = tot[0];
         ended = true;
       }
@@ -719,7 +550,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
       RowCgBack<Res, MEM> f(k, alpha, upd);
       k.template sweep<1>(1, k.par, f);
       double tot[2];
-      k.reduce(f.acc, part0, tot);
+      k.reduce(f.acc, tot);
       if (upd) dnrm2 = tot[0];
       rho_next = tot[1];
       ticks[1] += wall_clock64() - t1;
@@ -734,7 +565,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
         x_to_nodes(k);
         k.full_sync();
         double v[1] = {true_resid_phase(k)}, tot[1];
-        k.reduce(v, part1, tot);
+        k.reduce(v, tot);
         dnrm2 = tot[0];
         resid = sqrt(dnrm2 / bnrm2);
         xn_current = true;
@@ -941,8 +772,6 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
   bool done = false, xn_current = false;
   uint64_t ticks[2] = {0, 0};  // forward and backward sweeps
   k.par = st.resume >> 1;
-  double* const part0 = o.part;
-  double* const part1 = o.part + 2 * k.G;
   int half = 0;
   bool after_refresh = false;
   k.begin(refresh ? 0 : 1);
@@ -965,12 +794,12 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
       const uint64_t t0 = wall_clock64();
       RowBiFwd<Res, MEM> f(k, half, refresh);
       k.template sweep<2>(0, k.par ^ (refresh ? 1 : 0), f);
-      k.reduce(f.acc, part1, tot);
+      k.reduce(f.acc, tot);
       ticks[refresh ? 1 : 0] += wall_clock64() - t0;
     }
     if (refresh) {
       double v[1] = {bi_rho_phase<Res, MEM>(k, T)}, t[1];
-      k.reduce(v, part0, t);
+      k.reduce(v, t);
       rho = t[0];
       refresh = false;
       after_refresh = true;
@@ -990,7 +819,7 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
     {
       double v[2] = {0.0, 0.0};
       bi_update_phase<Res, MEM>(k, omega, !periodic, v, T);
-      k.reduce(v, part0, tot);
+      k.reduce(v, tot);
     }
     xn_current = false;
     if (!periodic) {
@@ -1003,7 +832,7 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
       x_to_nodes(k);
       k.full_sync();
       double v[1] = {true_resid_phase(k)}, t[1];
-      k.reduce(v, part1, t);
+      k.reduce(v, t);
       dnrm2 = t[0];
       resid = sqrt(dnrm2 / bnrm2);
       xn_current = true;
@@ -1110,10 +939,8 @@ __global__ __launch_bounds__(kBlock) void k_resident_init(ResidentOp o, const do
   }
 }
 
-// the grid barrier counts from zero in every launch
-__global__ void k_resident_reset(uint32_t* sync) {
-  for (int i = threadIdx.x; i < kResidentSync; i += blockDim.x) sync[i] = 0;
-}
+// every launch starts with the exchange's entries marked
+__global__ void k_resident_reset(uint32_t* sync) { reset_sync(sync); }
 
 template <int T, int K, int MEM>
 hipError_t launch(const ResidentOp& o, int grid, int budget, hipStream_t s) {

@@ -254,6 +254,9 @@ struct Context {
   int32_t last_resident = 0;    // workgroups of the last solve's resident kernel (0: launch per colour)
   bool ssor_proper = false;     // no L'/U' column lies in its row's own colour
   ResidentOp res;
+  DiagOp dres;
+  bool dres_sym = false;        // its tasks stand for this structure
+  DMem dres_task, dres_lane, dres_row, dres_z;
   DMem res_color_task, res_task, res_row, res_col, res_val, res_vec, res_sync, res_dsig;
   bool ssor16 = true;          // the flexible CG's FP32 sweeps read BF16 copies of the L'/U' values
   bool ssor16_valid = false;   // L.val16 / U.val16 hold the current values
@@ -357,6 +360,7 @@ struct Context {
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
                     &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
       m->release();
+    for (DMem* m : {&dres_task, &dres_lane, &dres_row, &dres_z}) m->release();
     for (DMem* m : {&res_color_task, &res_task, &res_row, &res_col, &res_val, &res_vec, &res_sync, &res_dsig})
       m->release();
     for (DMem* m : {&mpc_slave, &mpc_mptr, &mpc_mdof, &mpc_mval, &mpc_tptr, &mpc_tslave, &mpc_tval, &mpc_w1, &mpc_w2})
@@ -509,6 +513,7 @@ static int32_t load_structure(Context& c, const hecmw33_sys* A, bool force) {
   c.coarse_sym = false;
   c.mpc_built = false;
   c.diag_init = false;
+  c.dres_sym = false;
   c.dindex_valid = false;
   const size_t vb = sizeof(double) * 3 * (size_t)NP;
   for (DMem* m : {&c.vb, &c.vx, &c.vr, &c.vz, &c.vp, &c.vq})
@@ -1411,7 +1416,6 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t metho
   o.val = c.res_val.as<double>();
   o.xn = c.vx.as<double>();
   o.b = c.vb.as<double>();
-  o.part = c.part.as<double>();
   o.hist = c.hist.as<double>();
   o.sync = c.res_sync.as<uint32_t>();
   o.state = c.st.as<KrylovState>();
@@ -1423,13 +1427,12 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t metho
 // stay on the GPU), from r0 in vr and the initial state on the device; the end
 // state in c.h_st[0].
 constexpr int kResidentBudget = 512;
-static int32_t resident_solve(Context& c, const ResidentShape& sh) {
-  resident_init(c.res, sh, c.vr.as<double>(), c.stream);
+static int32_t resident_loop(Context& c, const std::function<hipError_t()>& run, const uint32_t* sync) {
   for (;;) {
-    HIPC(resident_run(c.res, sh, kResidentBudget, c.stream));
+    HIPC(run());
     uint32_t abort = 0;
     HIPC(hipMemcpyAsync(&c.h_st[0], c.st.p, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
-    HIPC(hipMemcpyAsync(&abort, c.res.sync + 64 * 9, sizeof(abort), hipMemcpyDeviceToHost, c.stream));
+    HIPC(hipMemcpyAsync(&abort, sync, sizeof(abort), hipMemcpyDeviceToHost, c.stream));
     HIPC(hipStreamSynchronize(c.stream));
     if (abort) {
       set_error("resident solve: a workgroup waited 20 s for the others");
@@ -1437,6 +1440,105 @@ static int32_t resident_solve(Context& c, const ResidentShape& sh) {
     }
     if (c.h_st[0].done) return 0;
   }
+}
+static int32_t resident_solve(Context& c, const ResidentShape& sh) {
+  resident_init(c.res, sh, c.vr.as<double>(), c.stream);
+  return resident_loop(c, [&] { return resident_run(c.res, sh, kResidentBudget, c.stream); }, c.res.sync);
+}
+
+// ---- resident CG with block-diagonal scaling (resident_diag.hip) -------------------------------
+// Workgroups for this system, 0: the launch-per-kernel solve.  The tasks are made here;
+// rows whose four-row group needs more than 64 lanes, or more tasks than the LDS of the
+// workgroups hold, are not taken.
+static int32_t diag_tasks(Context& c) {
+  if (c.dres_sym) return 0;
+  const int32_t N = c.N, nrow = (N + 3) / 4 * 4;
+  const int32_t *iL = c.h_indexL.data(), *iU = c.h_indexU.data();
+  std::vector<int4> task;
+  std::vector<int32_t> lane, lanes(nrow, 0);
+  std::vector<int2> row(nrow);
+  for (int32_t i = 0; i < N; ++i) lanes[i] = (1 + iL[i + 1] - iL[i] + iU[i + 1] - iU[i] + kDiagK - 1) / kDiagK;
+  DiagOp& o = c.dres;
+  o.ntasks = 0;
+  for (int32_t i = 0; i < nrow;) {
+    int32_t used = 0, n = 0;
+    while (n < kResidentRows && i + n < nrow) {
+      const int32_t add = lanes[i + n] + lanes[i + n + 1] + lanes[i + n + 2] + lanes[i + n + 3];
+      if (used + add > kWave) break;
+      used += add;
+      n += 4;
+    }
+    if (n == 0) {
+      c.dres_sym = true;
+      return 0;  // no tasks: not taken
+    }
+    task.push_back(make_int4(i, n, used, 0));
+    lane.resize(task.size() * kWave, -1);
+    int32_t at = 0, most = 0;
+    for (int32_t k = 0; k < n; ++k) {
+      row[i + k] = make_int2(at, lanes[i + k]);
+      at += lanes[i + k];
+      most = std::max(most, lanes[i + k]);
+    }
+    // equal parts of consecutive rows to consecutive lanes: their columns tend to
+    // be consecutive
+    int32_t l = 0;
+    for (int32_t part = 0; part < most; ++part)
+      for (int32_t k = 0; k < n; ++k)
+        if (part < lanes[i + k])
+          lane[(task.size() - 1) * kWave + l++] = k | part << 4 | (row[i + k].x + part) << 14;
+    i += n;
+  }
+  if (c.dres_task.ensure(sizeof(int4) * task.size()) || c.dres_lane.ensure(sizeof(int32_t) * lane.size()) ||
+      c.dres_row.ensure(sizeof(int2) * row.size()))
+    return 1;
+  HIPC(hipMemcpyAsync(c.dres_task.p, task.data(), sizeof(int4) * task.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipMemcpyAsync(c.dres_lane.p, lane.data(), sizeof(int32_t) * lane.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipMemcpyAsync(c.dres_row.p, row.data(), sizeof(int2) * row.size(), hipMemcpyHostToDevice, c.stream));
+  HIPC(hipStreamSynchronize(c.stream));  // the host vectors end here
+  o.ntasks = (int32_t)task.size();
+  c.dres_sym = true;
+  return 0;
+}
+// One task per wave up to all CUs: a wave's second task costs about what the barriers of
+// more workgroups cost in all (12^3 cube, us an iteration: 17.8 with 8 workgroups, 11.8 with 16,
+// 8.1 with 32, 7.0 with 35 and 64, 7.4 with 128; 20^3: 11.9 with 72, 9.7 with 128, 8.7
+// with 145).  One workgroup up to two tasks per wave saves the exchange (3^3: 4.4
+// against 6.2 with 2, 4^3: 5.7 against 6.0, but 5^3, 14 tasks: 11.0 against 6.2).
+static int32_t diag_shape(const Context& c) {
+  const int32_t t = c.dres.ntasks, most = std::min(c.res_cus, kResidentGridMax);
+  if (t == 0 || most < 1) return 0;
+  const int32_t grid = t <= 8 ? 1 : std::min(most, (t + 3) / 4);
+  return diag_lds_bytes(t, grid) <= 160 * 1024 ? grid : 0;
+}
+// 1: no memory for it
+static int32_t diag_setup(Context& c) {
+  DiagOp& o = c.dres;
+  const int32_t nrow = (c.N + 3) / 4 * 4;
+  o.zero_rec = nrow;
+  o.copy = 4 * ((int64_t)nrow + 4);
+  o.ring = (int32_t)std::max<int64_t>(4, std::min<int64_t>(64, (64 << 20) / (8 * o.copy)));
+  if (c.dres_z.ensure(sizeof(double) * o.copy * o.ring) || c.res_sync.ensure(sizeof(uint32_t) * kResidentSync)) {
+    c.dres_z.release();
+    (void)hipGetLastError();
+    return 1;
+  }
+  o.A = c.A.view;
+  o.task = c.dres_task.as<int4>();
+  o.lane = c.dres_lane.as<int32_t>();
+  o.row = c.dres_row.as<int2>();
+  o.n = c.N;
+  o.z = c.dres_z.as<double>();
+  o.alu = c.alu_diag.as<double>();
+  o.x = c.vx.as<double>();
+  o.r = c.vr.as<double>();
+  o.p = c.vp.as<double>();
+  o.q = c.vq.as<double>();
+  o.b = c.vb.as<double>();
+  o.hist = c.hist.as<double>();
+  o.sync = c.res_sync.as<uint32_t>();
+  o.state = c.st.as<KrylovState>();
+  return 0;
 }
 
 // Diagonal scaling of the device copies, hecmw_solver_scaling_fw_33 / _bk_33
@@ -1940,7 +2042,14 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
       if (e > 0) shape.grid = 0;
     }
   }
-  c.last_resident = shape.grid;
+  int32_t diag_grid = 0;
+  if (kind == 3 && method == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N) {
+    int32_t e = diag_tasks(c);
+    if (e < 0) return e;
+    if (e == 0) diag_grid = diag_shape(c);
+    if (diag_grid > 0 && diag_setup(c)) diag_grid = 0;
+  }
+  c.last_resident = std::max(shape.grid, diag_grid);
   // r0 = b - A x0; bnrm2 = b.b  (hecmw_solver_CG.f90:131-141)
   if (mixed && c.x_zero) {
     // x0 = 0 (the learned modes' sample solves): r0 = b exactly, without the FP64 product
@@ -2022,6 +2131,10 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
   int32_t enq = 0, nchunk = 0;
   if (shape.grid > 0) {
     if (int32_t e = resident_solve(c, shape)) return e;
+  } else if (diag_grid > 0) {
+    if (int32_t e = resident_loop(
+            c, [&] { return resident_diag_run(c.dres, diag_grid, kResidentBudget, c.stream); }, c.dres.sync))
+      return e;
   } else {
     // iterations: enqueue in chunks and poll the previous chunk's state while
     // the current one runs; kernels after the exit return at once
@@ -2068,7 +2181,7 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
   }
   h = c.h_st[0];
   out->Tsol = now_s() - t1;
-  if (timelog && shape.grid > 0) {
+  if (timelog && c.last_resident > 0) {
     out->time_Ax = h.time_Ax;
     out->time_precond = h.time_precond;
   } else if (timelog) {
