@@ -36,6 +36,7 @@ SOURCES = [
     ("resident.hip", True),
     ("resident_diag.hip", True),
     ("chol.hip", True),
+    ("ssor_flow.hip", True),
 ]
 
 

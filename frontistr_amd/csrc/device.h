@@ -83,6 +83,28 @@ struct Sell {
 struct KrylovState;
 
 // Multicolour SSOR operator (hecmw_precond_SSOR_33) as the sweeps see it.
+// The FP32 sweeps as one kernel (ssor_flow.hip).  Blocks of a row in groups of kFlowBlocks
+// (backward rows from their last block on), group[dir][s] the first of slice s: the
+// columns of lane 4 r + q, blocks q and q + 4, at col[dir][64 g + lane]; the values of
+// lane (row r, entry d), 3 j + e for entry (d, e) of block j, 16 bytes per plane at
+// [(planes g + i) 48 + 3 r + d], BF16 in 3 planes or FP32 in 6.
+constexpr int kFlowBlocks = 8;
+struct FlowOp {
+  const int32_t* group[2] = {nullptr, nullptr};
+  const int32_t* len[2] = {nullptr, nullptr};  // blocks of a row
+  const int2* col[2] = {nullptr, nullptr};
+  const void* val[2] = {nullptr, nullptr};
+  const int32_t* row_old = nullptr;
+  const float* alu = nullptr;
+  float4* rhs = nullptr;                       // r in slot order
+  void* rec = nullptr;                         // float4 [2][ns]: forward, then backward results
+  uint32_t* ticket = nullptr;
+  int32_t ns = 0, grid = 0;
+  bool b16 = false;
+};
+void flow_pack(const Sell<double>& m, const int32_t* group, bool desc, bool b16, void* val, int2* col, hipStream_t s);
+void flow_sweeps(const FlowOp& o, const float* r, const KrylovState* st, hipStream_t s);
+
 template <typename T>
 struct SsorOp {
   Sell<T> L, U;                // L'/U' per colour slice; columns are slot ids
@@ -96,6 +118,7 @@ struct SsorOp {
   int32_t last_bwd_empty;      // 1: the last colour's rows have no U' entries (their backward step is z -= 0)
   const uint16_t* Lv16 = nullptr;  // FP32 sweeps: L'/U' values in BF16 instead of L.val/U.val (null: T)
   const uint16_t* Uv16 = nullptr;
+  const FlowOp* flow = nullptr;    // FP32 sweeps: one kernel (ssor_flow.hip) instead of a launch per colour
 };
 void launch_to_bf16(int64_t n, const float* a, uint16_t* b, hipStream_t s);
 void ssor_apply(const SsorOp<double>& op, const double* r, double* z, const KrylovState* st, hipStream_t s);

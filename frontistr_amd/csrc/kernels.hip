@@ -879,7 +879,7 @@ __global__ __launch_bounds__(kBlock) void k_ssor_stage(int32_t n, const int32_t*
 }
 
 // z = zs back in node order; ND fused dots w0.z (and w1.z), FP64 accumulation
-template <typename T, int ND>
+template <typename T, int ND, int STRIDE>
 __global__ __launch_bounds__(kBlock) void k_ssor_unstage(int32_t n, const int32_t* __restrict__ node_slot,
                                                            const T* __restrict__ zs, T* __restrict__ z,
                                                            const T* __restrict__ w0, const T* __restrict__ w1,
@@ -891,7 +891,7 @@ __global__ __launch_bounds__(kBlock) void k_ssor_unstage(int32_t n, const int32_
     const int64_t t = node_slot[i];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const T v = zs[3 * t + d];
+      const T v = zs[STRIDE * t + d];
       z[3 * i + d] = v;
       if constexpr (ND > 0) acc[0] += (double)w0[3 * i + d] * (double)v;
       if constexpr (ND > 1) acc[KD - 1] += (double)w1[3 * i + d] * (double)v;
@@ -1390,13 +1390,20 @@ template <typename T, int ND>
 static int ssor_apply_run(const SsorOp<T>& op, const T* r, T* z, const T* w1, const KrylovState* st, double* part,
                           hipStream_t s) {
   const int gv = vec_grid(op.n);
+  if constexpr (sizeof(T) == 4)
+    if (op.flow) {
+      flow_sweeps(*op.flow, r, st, s);
+      k_ssor_unstage<T, ND, 4><<<gv, kBlock, 0, s>>>(op.n, op.node_slot, static_cast<const T*>(op.flow->rec) + 4 * (int64_t)op.flow->ns,
+                                                     z, r, w1, st, part);
+      return ND > 0 ? gv : 0;
+    }
   k_ssor_stage<T><<<gv, kBlock, 0, s>>>(op.n, op.node_slot, r, op.zs, st);
   for (int c = 0; c < op.ncolor; ++c) ssor_fwd_any<T>(op, c, st, s);
   for (int c = op.ncolor - 1; c >= 0; --c) {
     if (c == op.ncolor - 1 && op.last_bwd_empty) continue;
     ssor_bwd_any<T>(op, c, st, s);
   }
-  k_ssor_unstage<T, ND><<<gv, kBlock, 0, s>>>(op.n, op.node_slot, op.zs, z, r, w1, st, part);
+  k_ssor_unstage<T, ND, 3><<<gv, kBlock, 0, s>>>(op.n, op.node_slot, op.zs, z, r, w1, st, part);
   return ND > 0 ? gv : 0;
 }
 

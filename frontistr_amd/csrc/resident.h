@@ -55,6 +55,8 @@ constexpr int kSyncParts = 64 * 10;
 constexpr int kSyncSet = 2 * kResidentGridMax;
 static_assert(kResidentSync == kSyncParts + 3 * 2 * kSyncSet, "words of the exchange");
 
+constexpr int kAuxSc1 = 16;  // agent scope, as the cache bits of a buffer access
+
 // The mark of an entry that has not been computed: a quiet NaN with a payload
 // that no computed value keeps (unmarked replaces it by the plain NaN).
 constexpr int kMarkHi = 0x7FFADEAD;

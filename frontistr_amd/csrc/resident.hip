@@ -61,7 +61,6 @@ namespace {
 // take 16 bytes with the agent-scope bit.
 using V4 = __attribute__((__vector_size__(16))) uint32_t;
 using V2 = __attribute__((__vector_size__(8))) uint32_t;
-constexpr int kAuxSc1 = 16;
 __device__ __forceinline__ void gather16(__amdgpu_buffer_rsrc_t r, uint32_t off, double& a, double& b) {
   const V4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kAuxSc1);
   a = __hiloint2double((int)v[1], (int)v[0]);

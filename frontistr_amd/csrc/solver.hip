@@ -260,6 +260,13 @@ struct Context {
   DMem res_color_task, res_task, res_row, res_col, res_val, res_vec, res_sync, res_dsig;
   bool ssor16 = true;          // the flexible CG's FP32 sweeps read BF16 copies of the L'/U' values
   bool ssor16_valid = false;   // L.val16 / U.val16 hold the current values
+  // the FP32 sweeps as one kernel: packed columns, values in BF16 and in FP32
+  FlowOp flow;
+  bool flow_use = false;       // for this structure
+  bool ssor_round_valid = false;  // L.val32 / U.val32 hold the current values
+  bool flow_sym = false, flow_valid[2] = {false, false};
+  std::vector<int32_t> h_flow_group[2];  // first group of blocks of every slice
+  DMem flow_group[2], flow_col[2], flow_val[2][2], flow_rec;
   // DIAG
   bool diag_init = false;
   DMem row_diag, alu_diag;
@@ -345,7 +352,11 @@ struct Context {
   SsorOp<float> ssor_op32(bool v16) {
     SsorOp<float> op{L.view32, U.view32, row_old.as<int32_t>(), alu_ssor32.as<float>(), color_slice.data(),
                      ncolor, vzs32.as<float>(), node_slot.as<int32_t>(), N, ssor_last_bwd_empty};
-    if (v16) {
+    if (flow_use) {
+      for (int d = 0; d < 2; ++d) flow.val[d] = flow_val[v16 ? 1 : 0][d].p;
+      flow.b16 = v16;
+      op.flow = &flow;
+    } else if (v16) {
       op.Lv16 = L.val16.as<uint16_t>();
       op.Uv16 = U.val16.as<uint16_t>();
     }
@@ -359,6 +370,9 @@ struct Context {
       m->release();
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
                     &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
+      m->release();
+    for (DMem* m : {&flow_group[0], &flow_group[1], &flow_col[0], &flow_col[1], &flow_val[0][0], &flow_val[0][1], &flow_val[1][0],
+                    &flow_val[1][1], &flow_rec})
       m->release();
     for (DMem* m : {&dres_task, &dres_lane, &dres_row, &dres_z}) m->release();
     for (DMem* m : {&res_color_task, &res_task, &res_row, &res_col, &res_val, &res_vec, &res_sync, &res_dsig})
@@ -690,9 +704,16 @@ static int32_t setup_ssor_symbolic(Context& c, int32_t ncolor_in) {
     build_lu(std::integral_constant<int, kRowsS>{});
   if (int32_t e = upload_sell(hl, c.L, c.stream)) return e;
   if (int32_t e = upload_sell(hu, c.U, c.stream)) return e;
+  for (int d = 0; d < 2; ++d) {
+    const std::vector<int32_t>& ptr = d ? hu.ptr : hl.ptr;
+    std::vector<int32_t>& group = c.h_flow_group[d];
+    group.assign(ptr.size(), 0);
+    for (size_t s = 0; s + 1 < ptr.size(); ++s) group[s + 1] = group[s] + (ptr[s + 1] - ptr[s] + kFlowBlocks - 1) / kFlowBlocks;
+  }
   c.h_lenL = std::move(hl.len);
   c.h_lenU = std::move(hu.len);
   c.res_packets = 0;
+  c.flow_sym = false;
   // the slot of every node, for staging r into slot order and z back out
   std::vector<int32_t> node_slot(N, -1);
   for (int64_t t = 0; t < (int64_t)row_old.size(); ++t)
@@ -768,6 +789,61 @@ static int32_t round_sell(SellDev& d, hipStream_t s) {
   launch_to_f32(9 * d.view.nslots, d.view.val, d.view32.val, s);
   return 0;
 }
+// The FP32 sweeps as one kernel, if this structure takes it: slices of 16 rows, and no
+// couplings inside a colour (there a row would wait for one that is drawn with it).
+// 1: not taken, or no memory for the packed copy.
+static int32_t flow_setup(Context& c, bool v16) {
+  if (c.ssor_R != kRowsS || !c.ssor_proper || c.ssor_rows < 1) return 1;
+  const int32_t ns = (int32_t)c.ssor_rows, S = ns / kRowsS;
+  auto no_memory = [&] {
+    for (DMem* m : {&c.flow_group[0], &c.flow_group[1], &c.flow_col[0], &c.flow_col[1], &c.flow_val[0][0], &c.flow_val[0][1],
+                    &c.flow_val[1][0], &c.flow_val[1][1], &c.flow_rec})
+      m->release();
+    (void)hipGetLastError();
+    c.flow_sym = c.flow_valid[0] = c.flow_valid[1] = false;
+    return 1;
+  };
+  FlowOp& o = c.flow;
+  const bool sym = !c.flow_sym;
+  auto ngroup = [&](int d) { return (size_t)std::max(c.h_flow_group[d][S], 1); };
+  for (int d = 0; sym && d < 2; ++d) {
+    const std::vector<int32_t>& group = c.h_flow_group[d];
+    if (c.flow_group[d].ensure(sizeof(int32_t) * group.size()) || c.flow_col[d].ensure(sizeof(int2) * kWave * ngroup(d)) ||
+        c.flow_rec.ensure(sizeof(float4) * 3 * (size_t)ns + 256))
+      return no_memory();
+    HIPC(hipMemcpyAsync(c.flow_group[d].p, group.data(), sizeof(int32_t) * group.size(), hipMemcpyHostToDevice, c.stream));
+  }
+  if (sym) {
+    for (int d = 0; d < 2; ++d) {
+      o.group[d] = c.flow_group[d].as<int32_t>();
+      o.len[d] = (d ? c.U : c.L).view.len;
+      o.col[d] = c.flow_col[d].as<int2>();
+    }
+    o.row_old = c.row_old.as<int32_t>();
+    o.rec = c.flow_rec.p;
+    o.rhs = c.flow_rec.as<float4>() + 2 * (size_t)ns;
+    o.ticket = reinterpret_cast<uint32_t*>(o.rhs + ns);
+    o.ns = ns;
+    // four times the workgroups that a colour's slices occupy, so that the slices of the next
+    // colours are loaded in time (30^3 cube, us: 161 with as many, 101 with twice, 92 with
+    // four times, 90 with eight), up to one per CU, beyond which the waiting ones slow the
+    // others down (60^3, 111 per colour: 116 with 222, 126 with 444) unless a colour
+    // has work for more (72^3, 190 per colour: 184 with 250, 171 with 512)
+    const int32_t per = S / std::max(c.ncolor, 1) / 8 + 1;
+    o.grid = per > 160 ? 512 : std::min(4 * per, 256);
+  }
+  for (int d = 0; d < 2; ++d) {
+    DMem& v = c.flow_val[v16 ? 1 : 0][d];
+    if (v.ensure(ngroup(d) * 48 * 16 * (v16 ? 3 : 6))) return no_memory();
+    flow_pack((d ? c.U : c.L).view, o.group[d], d == 1, v16, v.p, sym ? c.flow_col[d].as<int2>() : nullptr, c.stream);
+  }
+  o.alu = c.alu_ssor32.as<float>();
+  HIPC(hipGetLastError());
+  c.flow_sym = true;
+  c.flow_valid[v16 ? 1 : 0] = true;
+  return 0;
+}
+
 // v16: the SSOR sweeps will read BF16 copies of the L'/U' values (rounded to
 // nearest even from the FP32 image)
 static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
@@ -776,8 +852,8 @@ static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
     c.a32_valid = true;
   }
   if (kind == 1 && !c.ssor32_valid) {
-    if (round_sell(c.L, c.stream) || round_sell(c.U, c.stream)) return HECMW33_ERROR_DEVICE;
     c.ssor16_valid = false;
+    c.ssor_round_valid = c.flow_valid[0] = c.flow_valid[1] = false;
     const int64_t nslot = c.ssor_rows;
     if (c.alu_ssor32.ensure(sizeof(float) * 9 * std::max<int64_t>(nslot, 1)) ||
         c.vzs32.ensure(sizeof(float) * 3 * std::max<int64_t>(nslot, 1)))
@@ -786,7 +862,16 @@ static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
     launch_to_f32(9 * nslot, c.alu_ssor.as<double>(), c.alu_ssor32.as<float>(), c.stream);
     c.ssor32_valid = true;
   }
-  if (kind == 1 && v16 && !c.ssor16_valid) {
+  if (kind == 1 && !c.flow_valid[v16 ? 1 : 0]) {
+    const int32_t e = flow_setup(c, v16);
+    if (e < 0) return e;
+    c.flow_use = e == 0;
+  }
+  if (kind == 1 && !c.flow_use && !c.ssor_round_valid) {
+    if (round_sell(c.L, c.stream) || round_sell(c.U, c.stream)) return HECMW33_ERROR_DEVICE;
+    c.ssor_round_valid = true;
+  }
+  if (kind == 1 && v16 && !c.flow_use && !c.ssor16_valid) {
     for (SellDev* d : {&c.L, &c.U}) {
       const int64_t n = 9 * std::max<int64_t>(d->view.nslots, 1);
       if (d->val16.ensure(sizeof(uint16_t) * n)) return HECMW33_ERROR_DEVICE;
