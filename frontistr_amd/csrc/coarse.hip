@@ -116,38 +116,38 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E(Sell<double> A, const
   block_reduce<36>(acc, Eblk + (int64_t)p * 36);
 }
 
-// dense E, column-major (the solver library's layout): E(6a+r, 6b+q) = Eblk[p][r][q]
+// E(6a+r, 6b+q) = Eblk[p][r][q], the blocks on and below the diagonal
 __global__ void k_coarse_scatter(int32_t npair, const int32_t* __restrict__ pa, const int32_t* __restrict__ pb,
-                                 const double* __restrict__ Eblk, double* __restrict__ E, int32_t lda) {
+                                 const double* __restrict__ Eblk, double* __restrict__ E, int32_t w) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)npair * 36) return;
   const int p = (int)(t / 36), e = (int)(t % 36);
   const int a = pa[p], b = pb[p];
   const int r = e / 6, q = e % 6;
-  E[(int64_t)(6 * b + q) * lda + 6 * a + r] = Eblk[t];
+  const int row = 6 * a + r, col = 6 * b + q;
+  if (row / 64 >= col / 64) E[coarse_band_index(w, row, col)] = Eblk[t];
 }
 
 // unit pivot for a coarse unknown whose column of Z is zero (E(k,k) exactly 0):
 // its restriction is exactly 0, so its value stays 0 and E stays invertible
-__global__ void k_coarse_unit_pivots(int32_t nc, double* __restrict__ E, int32_t lda) {
+__global__ void k_coarse_unit_pivots(int32_t np, double* __restrict__ E, int32_t w) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < nc && E[(int64_t)k * lda + k] == 0.0) E[(int64_t)k * lda + k] = 1.0;
+  if (k < np && E[coarse_band_index(w, k, k)] == 0.0) E[coarse_band_index(w, k, k)] = 1.0;
 }
 
-// W = the full array mirrored from the lower triangle that coarse_factor leaves
-// row-major in E's upper half ((r, c), c <= r, at E[r lda + c]): E^-1 in FP32, or
-// L^-1 below and on the diagonal with L^-T above in FP64 (with the learned modes E
+// W = the full array mirrored from the lower triangle that coarse_factor leaves: E^-1 in
+// FP32, or L^-1 below and on the diagonal with L^-T above in FP64 (with the learned modes E
 // is too ill-conditioned for FP32).  64 x 64 tiles through LDS, so that both halves
 // are written in rows.
 template <typename T>
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_mirror(int32_t nc, const double* __restrict__ E, int32_t lda,
+__global__ __launch_bounds__(kCoarseBlock) void k_coarse_mirror(int32_t nc, const double* __restrict__ E, int32_t np,
                                                                   T* __restrict__ W, int32_t ldw) {
   const int r0 = 64 * blockIdx.x, c0 = 64 * blockIdx.y;
   if (c0 > r0) return;
   __shared__ double tile[64][65];
   for (int k = threadIdx.x; k < 64 * 64; k += kCoarseBlock) {
     const int r = r0 + k / 64, c = c0 + k % 64;
-    double v = r < nc && c < nc ? E[(int64_t)max(r, c) * lda + min(r, c)] : 0.0;
+    double v = r < nc && c < nc ? E[coarse_inverse_index(np, max(r, c), min(r, c))] : 0.0;
     tile[k / 64][k % 64] = v;
     if (r < nc && c < ldw) W[(int64_t)r * ldw + c] = (T)v;
   }
@@ -588,15 +588,16 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E12(Sell<double> A, con
   block_reduce<36>(acc, Eblk + ((int64_t)p * 4 + blockIdx.y) * 36);
 }
 
-// dense E (column-major): E(12a + 6tr + r, 12b + 6tc + q) = tile (tr, tc) of pair p
+// E(12a + 6tr + r, 12b + 6tc + q) = tile (tr, tc) of pair p
 __global__ void k_coarse_scatter12(int32_t npair, const int32_t* __restrict__ pa, const int32_t* __restrict__ pb,
-                                   const double* __restrict__ Eblk, double* __restrict__ E, int32_t lda) {
+                                   const double* __restrict__ Eblk, double* __restrict__ E, int32_t w) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (int64_t)npair * 144) return;
   const int p = (int)(t / 144), e = (int)(t % 144);
   const int tile = e / 36, tr = tile >> 1, tc = tile & 1, r = (e % 36) / 6, q = e % 6;
   const int a = pa[p], b = pb[p];
-  E[(int64_t)(12 * b + 6 * tc + q) * lda + 12 * a + 6 * tr + r] = Eblk[t];
+  const int row = 12 * a + 6 * tr + r, col = 12 * b + 6 * tc + q;
+  if (row / 64 >= col / 64) E[coarse_band_index(w, row, col)] = Eblk[t];
 }
 
 // A Z per node and touched aggregate, 3x12 FP32 per entry, every entry kept
@@ -849,26 +850,26 @@ int coarse_fcg_pq(int64_t n3, const float* z, const float* az, float* p, float* 
 }
 
 void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, const int32_t* pa, const int32_t* pb,
-                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, double* E, int32_t lda, hipStream_t s) {
+                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, const CoarseBand& e, hipStream_t s) {
   if (npair <= 0) return;
   if (op.nm == 12) {
     k_coarse_E12<<<dim3((unsigned)npair, 4), kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, op.xm, Eblk);
     const int64_t ne = (int64_t)npair * 144;
-    k_coarse_scatter12<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, E, lda);
+    k_coarse_scatter12<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, e.E, e.w);
   } else {
     k_coarse_E<<<(unsigned)npair, kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, Eblk);
     const int64_t ne = (int64_t)npair * 36;
-    k_coarse_scatter<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, E, lda);
+    k_coarse_scatter<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, e.E, e.w);
   }
-  k_coarse_unit_pivots<<<(op.nc + 255) / 256, 256, 0, s>>>(op.nc, E, lda);
+  k_coarse_unit_pivots<<<(e.np + 255) / 256, 256, 0, s>>>(e.np, e.E, e.w);
 }
 
-void coarse_mirror(const CoarseOp& op, const double* E, int32_t lda, hipStream_t s) {
+void coarse_mirror(const CoarseOp& op, const double* T, int32_t np, hipStream_t s) {
   const dim3 g((unsigned)(op.ldw / 64), (unsigned)(op.ldw / 64));
   if (op.nm == 12)
-    k_coarse_mirror<double><<<g, kCoarseBlock, 0, s>>>(op.nc, E, lda, op.W64, op.ldw);
+    k_coarse_mirror<double><<<g, kCoarseBlock, 0, s>>>(op.nc, T, np, op.W64, op.ldw);
   else
-    k_coarse_mirror<float><<<g, kCoarseBlock, 0, s>>>(op.nc, E, lda, op.W, op.ldw);
+    k_coarse_mirror<float><<<g, kCoarseBlock, 0, s>>>(op.nc, T, np, op.W, op.ldw);
 }
 
 int coarse_apply(const CoarseOp& op, int32_t n, const float* r, float* z, const float* q, const KrylovState* st,

@@ -390,20 +390,30 @@ struct CoarseOp {
   double* tv64 = nullptr;
   double* yv64 = nullptr;
 };
+// E banded, in blocks of 64 x 64, column-major; block (i, j) with 0 <= i - j <= w at
+// E + ((w + 1) j + i - j) * 4096, the order padded to np with a unit diagonal
+struct CoarseBand {
+  double* E = nullptr;
+  int32_t np = 0, w = 0;
+};
 // E = Z^T A Z: the nm x nm block of every coupled aggregate pair (pa[p], pb[p]), summed
-// over the pair's nodes pn[pn_ptr[p]..pn_ptr[p+1]), then scattered into the dense E
+// over the pair's nodes pn[pn_ptr[p]..pn_ptr[p+1]), then scattered into the band's blocks
 // (Eblk: nm*nm doubles per pair)
 void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, const int32_t* pa, const int32_t* pb,
-                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, double* E, int32_t lda, hipStream_t s);
-// Cholesky factorization and inverse of the dense banded E (chol.hip): E is
-// column-major of order coarse_padded(nc), half bandwidth `band`; its upper triangle
-// receives, row-major, L^-1 (E = L L^T) or with `both` E^-1.  Linv: 64 doubles per
-// (padded) row; *info is set when E is not positive definite.
-int32_t coarse_padded(int32_t nc);
-void coarse_factor(double* E, int32_t nc, int32_t band, double* Linv, bool both, int32_t* info, hipStream_t s);
+                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, const CoarseBand& e, hipStream_t s);
+// Cholesky factorization and inverse of E (chol.hip).  T receives the lower triangle of
+// L^-1 (E = L L^T) or with `both` of E^-1, in columns of 16: coarse_inverse_index.
+// Linv: 64 doubles per (padded) row; *info is set when E is not positive definite.
+__host__ __device__ inline int64_t coarse_band_index(int w, int r, int c) {  // r / 64 >= c / 64
+  return ((int64_t)(w + 1) * (c / 64) + r / 64 - c / 64) * 4096 + r % 64 + 64 * (c % 64);
+}
+__host__ __device__ inline int64_t coarse_inverse_index(int np, int r, int c) {
+  return ((int64_t)(c / 16) * np + r) * 16 + c % 16;
+}
+void coarse_factor(const CoarseBand& e, double* Linv, double* T, bool both, int32_t* info, hipStream_t s);
 // the iterations' copies: E^-1 in FP32 (W) or, with twelve modes, L^-1 in FP64 (W64),
 // mirrored into full arrays
-void coarse_mirror(const CoarseOp& op, const double* E, int32_t lda, hipStream_t s);
+void coarse_mirror(const CoarseOp& op, const double* T, int32_t np, hipStream_t s);
 // The symmetric two-level step (W = A Z per node and touched aggregate):
 // build W from the symbolic node-major lists ncnt/nagg into the compacted
 // sc (per node: first slot, count) / aggW / W, dropping the entries that are

@@ -319,7 +319,7 @@ struct Context {
   int32_t coarse_nm_num = 0;      // modes per aggregate of the E^-1 built (6 or 12)
   int32_t coarse_w_nm = 0;        // modes per aggregate of the A Z built
   int64_t coarse_nw = 0;          // node-aggregate entries of A Z
-  DMem cg_agg, cg_aptr, cg_anodes, cg_dv, cg_pa, cg_pb, cg_pnptr, cg_pn, cg_Eblk, cg_E, cg_W, cg_cv, cg_tv, cg_yv, cg_info, cg_Linv;
+  DMem cg_agg, cg_aptr, cg_anodes, cg_dv, cg_pa, cg_pb, cg_pnptr, cg_pn, cg_Eblk, cg_E, cg_W, cg_cv, cg_tv, cg_yv, cg_info, cg_Linv, cg_T;
   DMem cg_ncnt, cg_nagg, cg_AZ, cg_sc, cg_aggW, cg_kept, vr1_32, vt32, vw32, vaz32;
   // multipoint constraints (hecMESH%mpc) for the MPC-CG product T^T A T
   // (Iarray 83 set, as hecmw_solve_iterative sets it for MPC_METHOD = 2)
@@ -369,7 +369,7 @@ struct Context {
                     &vmask})
       m->release();
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
-                    &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
+                    &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_T, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
       m->release();
     for (DMem* m : {&flow_group[0], &flow_group[1], &flow_col[0], &flow_col[1], &flow_val[0][0], &flow_val[0][1], &flow_val[1][0],
                     &flow_val[1][1], &flow_rec})
@@ -1250,10 +1250,15 @@ static int32_t coarse_numeric(Context& c, int32_t nm) {
   const int32_t nc = op.nc;
   // six modes: E^-1, c and y in FP32; twelve: in FP64
   const size_t we = nm == 12 ? sizeof(double) : sizeof(float);
-  const int32_t lda = coarse_padded(nc);
-  if (c.cg_info.ensure(sizeof(int32_t)) || c.cg_Linv.ensure(sizeof(double) * 64 * (size_t)lda) ||
+  // E's bandwidth follows from the coupled aggregate pairs
+  const int32_t band = std::max(0, std::min(nc - 1, nm * (c.coarse_band_agg + 1) - 1));
+  CoarseBand e;
+  e.np = (nc + 63) / 64 * 64;
+  e.w = std::min((band + 63) / 64, e.np / 64 - 1);
+  const size_t eband = (size_t)e.np * 64 * (e.w + 1);
+  if (c.cg_info.ensure(sizeof(int32_t)) || c.cg_Linv.ensure(sizeof(double) * 64 * (size_t)e.np) ||
       c.cg_Eblk.ensure(sizeof(double) * nm * nm * (size_t)std::max(c.coarse_npair, 1)) ||
-      c.cg_E.ensure(sizeof(double) * (size_t)lda * lda) || c.cg_W.ensure(we * (size_t)nc * op.ldw) ||
+      c.cg_E.ensure(sizeof(double) * eband) || c.cg_T.ensure(sizeof(double) * (size_t)e.np * e.np) || c.cg_W.ensure(we * (size_t)nc * op.ldw) ||
       c.cg_cv.ensure(we * op.ldw) || c.cg_yv.ensure(we * op.ldw) || c.cg_tv.ensure(we * op.ldw))
     return HECMW33_ERROR_DEVICE;
   op.W = nm == 12 ? nullptr : c.cg_W.as<float>();
@@ -1265,23 +1270,22 @@ static int32_t coarse_numeric(Context& c, int32_t nm) {
   op.tv64 = nm == 12 ? c.cg_tv.as<double>() : nullptr;
   HIPC(hipMemsetAsync(c.cg_cv.p, 0, we * op.ldw, c.stream));
   HIPC(hipMemsetAsync(c.cg_tv.p, 0, we * op.ldw, c.stream));
-  HIPC(hipMemsetAsync(c.cg_E.p, 0, sizeof(double) * (size_t)lda * lda, c.stream));
+  HIPC(hipMemsetAsync(c.cg_E.p, 0, sizeof(double) * eband, c.stream));
+  e.E = c.cg_E.as<double>();
   HIPC(hipMemsetAsync(c.cg_info.p, 0, sizeof(int32_t), c.stream));
   coarse_assemble(c.A.view, op, c.coarse_npair, c.cg_pa.as<int32_t>(), c.cg_pb.as<int32_t>(),
-                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.cg_Eblk.as<double>(), c.cg_E.as<double>(), lda,
-                  c.stream);
+                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.cg_Eblk.as<double>(), e, c.stream);
   HIPC(hipGetLastError());
   // six modes: E^-1 for one FP32 product per coarse solve; twelve: L^-1 for two FP64
   // triangular products, y = L^-T (L^-1 c), the same bytes read without forming
-  // L^-T L^-1.  E's bandwidth follows from the coupled aggregate pairs.
-  const int32_t band = std::max(0, std::min(nc - 1, nm * (c.coarse_band_agg + 1) - 1));
-  coarse_factor(c.cg_E.as<double>(), nc, band, c.cg_Linv.as<double>(), nm != 12, c.cg_info.as<int32_t>(), c.stream);
+  // L^-T L^-1.
+  coarse_factor(e, c.cg_Linv.as<double>(), c.cg_T.as<double>(), nm != 12, c.cg_info.as<int32_t>(), c.stream);
   int32_t info = 0;
   HIPC(hipMemcpyAsync(&info, c.cg_info.p, sizeof(int32_t), hipMemcpyDeviceToHost, c.stream));
   HIPC(hipStreamSynchronize(c.stream));
   c.coarse_ok = info == 0;
   c.coarse_w_valid = false;
-  if (c.coarse_ok) coarse_mirror(op, c.cg_E.as<double>(), lda, c.stream);
+  if (c.coarse_ok) coarse_mirror(op, c.cg_T.as<double>(), e.np, c.stream);
   HIPC(hipGetLastError());
   c.coarse_num = true;
   c.coarse_nm_num = nm;
