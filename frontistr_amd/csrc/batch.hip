@@ -52,7 +52,13 @@ namespace {
 
 constexpr int KS = 16;          // right-hand-side stride of every batch vector
 constexpr int kBT = 256;        // threads per workgroup
-constexpr int kTileRows = 128;  // rows per tile (at least; grown to cap the tile count)
+// Rows per tile: 16 (one pass of a workgroup) up to 128, such that every CU has about six
+// tiles.  With 128 whatever the batch, 24,160 rows made 192 tiles, less than one
+// workgroup of four waves per CU, each walking its rows' blocks one after the other: SpMM 84 us
+// against 28 with 16 rows (2,332 rows: 125 and 13; 42,694 rows: 99, and 39 with 32), the
+// solve 120 ms against 70 (88 and 20; 144 and 95, 99 with 16).  Many small tiles
+// only cost partial sums.
+constexpr int kTileRowsMin = 16, kTileRowsMax = 128, kTilesPerCu = 6;
 constexpr int kMaxTiles = 65536;
 constexpr int kChunk = 8;       // iterations per captured graph
 
@@ -1141,8 +1147,14 @@ static int32_t batch_load(hecmw33_batch& B, int32_t nsys, const hecmw33_sys* sys
       std::memcpy(&d64[9 * (size_t)(g0 + i)], A.D + 9 * (size_t)i, 72);
     }
   }
-  // tiles: runs of rows inside a system, at least kTileRows, count capped
-  int tr = kTileRows;
+  // tiles: runs of rows inside a system, count capped
+  {
+    int dev = 0;
+    BHIPC(hipGetDevice(&dev));
+    BHIPC(hipDeviceGetAttribute(&B.ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  }
+  int tr = kTileRowsMin;
+  while (tr < kTileRowsMax && (int64_t)tr * kTilesPerCu * B.ncu < B.nrows) tr *= 2;
   for (;;) {
     int64_t nt = 0;
     for (int s = 0; s < nsys; ++s) nt += (B.N[s] + tr - 1) / tr;
@@ -1174,11 +1186,6 @@ static int32_t batch_load(hecmw33_batch& B, int32_t nsys, const hecmw33_sys* sys
       B.part.ensure(sizeof(double) * 4 * KS * (size_t)B.ntiles) || batch_state_layout(B) ||
       B.qtile.ensure(sizeof(int32_t) * kqLists * (size_t)B.ntiles) || B.qn.ensure(sizeof(int32_t) * kqLists))
     return HECMW33_ERROR_DEVICE;
-  {
-    int dev = 0;
-    BHIPC(hipGetDevice(&dev));
-    BHIPC(hipDeviceGetAttribute(&B.ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  }
   hipStream_t st = B.stream;
   BHIPC(hipMemcpyAsync(B.rowptr.p, rp.data(), sizeof(int32_t) * rp.size(), hipMemcpyHostToDevice, st));
   BHIPC(hipMemcpyAsync(B.col.p, cl.data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice, st));

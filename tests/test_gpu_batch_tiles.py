@@ -1,0 +1,39 @@
+"""Batched solves with tiles of 16, 32, 64 and 128 rows (csrc/batch.hip picks them by the
+rows of the batch): the FP64 product is bitwise the restatement's SpMV (oracle/restate.c)
+whatever the tiles, the FP32 one within its rounding (2e-6 in the norm, as in the other
+batch tests), and a solve reaches its FP64 residual for every system, also for one that
+ends in a partial tile and one smaller than a tile."""
+import numpy as np
+import pytest
+
+import frontistr_amd as fa
+from oracle import restate
+
+pytestmark = pytest.mark.gpu
+
+
+# nodes per edge minus one of the largest system -> rows per tile on 256 CUs: 6 tiles per CU
+@pytest.mark.parametrize("n,rows_per_tile", [(3, 16), (29, 32), (37, 64), (47, 128)])
+def test_tiles_by_batch_size(n, rows_per_tile):
+    mats = [fa.gen_hex8(n, kind="lognormal", seed=n), fa.gen_hex8(1), fa.gen_tet10(2, 3, 2, seed=1)[0]]
+    rng = np.random.default_rng(n)
+    Bs = [rng.standard_normal((2, 3 * m.N)) for m in mats]
+    bs = fa.BatchSolver(mats, Bs)
+    info = bs.info()
+    assert info["tiles"] == sum(-(-m.N // rows_per_tile) for m in mats)
+    Y64, Y32 = bs.spmm(Bs, fp64=True), bs.spmm(Bs, fp64=False)
+    for m, X, y64, y32 in zip(mats, Bs, Y64, Y32):
+        for k in range(2):
+            y = restate.matvec(m, X[k])
+            assert np.array_equal(y64[k], y)
+            assert np.linalg.norm(y32[k] - y) <= 2e-6 * np.linalg.norm(y)
+    p = fa.gen_hex8(1)
+    p.set_iter(5000)
+    p.set_precond(3)
+    bs.solve(p.Iarray.copy(), p.Rarray.copy())
+    for s, m in enumerate(mats):
+        x = np.asarray(bs.x(s))
+        for k in range(2):
+            r = Bs[s][k] - restate.matvec(m, x[k])
+            assert np.linalg.norm(r) <= 1.001e-8 * np.linalg.norm(Bs[s][k])
+    bs.close()
