@@ -104,7 +104,7 @@ constexpr int kQRun = 16;
 
 struct Queue {
   int32_t* tile;  // [kqLists][ntiles] live tile ids, system by system
-  int32_t* n;     // [kqLists] live tiles per list
+  int32_t* n;     // [kqLists] live tiles per list, and a count of tails done
 };
 
 // what one launch walks (tile == nullptr: one tile per workgroup over every
@@ -140,24 +140,40 @@ __device__ __forceinline__ void walk_tiles(const QView& q, F&& body) {
 
 // Rebuild list LIST from the systems' flags (active: sys_active != 0; rel:
 // sys_rel != 0) and, for the active list, publish the live instance count the
-// host polls.
+// host polls.  By one workgroup of kTailThreads.
+constexpr int kTailThreads = 64 * KS;
 template <int LIST>
-__global__ __launch_bounds__(1024) void kb_queue(Tiles T, int32_t nsys, BState S, Queue Q) {
+__device__ __forceinline__ void build_queue(const Tiles& T, int32_t nsys, const BState& S, const Queue& Q) {
+  __shared__ int32_t flag[kTailThreads], first[kTailThreads], count[kTailThreads];
   int32_t* out = Q.tile + (int64_t)LIST * T.ntiles;
   int32_t off = 0, live_inst = 0;
-  for (int s = 0; s < nsys; ++s) {
-    const int32_t a = S.sys_active[s];
-    const bool sel = LIST == kqActive ? a != 0 : S.sys_rel[s] != 0;
-    live_inst += a;
-    if (!sel) continue;
-    const int32_t t0 = T.sys_tile0[s], nt = T.sys_ntile[s];
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) out[off + i] = t0 + i;
-    off += nt;
+  for (int s0 = 0; s0 < nsys; s0 += kTailThreads) {
+    const int n = min(kTailThreads, nsys - s0);
+    __syncthreads();
+    // at agent scope: other workgroups of this launch may have set them
+    if ((int)threadIdx.x < n) {
+      const int s = s0 + threadIdx.x;
+      flag[threadIdx.x] = __hip_atomic_load((LIST == kqActive ? S.sys_active : S.sys_rel) + s, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+      first[threadIdx.x] = T.sys_tile0[s];
+      count[threadIdx.x] = T.sys_ntile[s];
+    }
+    __syncthreads();
+    for (int k = 0; k < n; ++k) {
+      if (!flag[k]) continue;
+      live_inst += flag[k];
+      for (int i = threadIdx.x; i < count[k]; i += kTailThreads) out[off + i] = first[k] + i;
+      off += count[k];
+    }
   }
   if (threadIdx.x == 0) {
     Q.n[LIST] = off;
     if (LIST == kqActive) *S.active_total = live_inst;
   }
+}
+template <int LIST>
+__global__ __launch_bounds__(kTailThreads) void kb_queue(Tiles T, int32_t nsys, BState S, Queue Q) {
+  build_queue<LIST>(T, nsys, S, Q);
 }
 
 // The set-up launches (one workgroup per tile) keep the hardware's round-robin
@@ -171,6 +187,7 @@ __global__ __launch_bounds__(1024) void kb_queue(Tiles T, int32_t nsys, BState S
 template <int ND>
 __device__ __forceinline__ void tile_partials_rowlanes(const double (&acc)[ND], double* part, int pitch, int tile) {
   __shared__ double red[ND][kBT];
+  __syncthreads();  // the sums of the workgroup's tile before have been read
 #pragma unroll
   for (int d = 0; d < ND; ++d) red[d][threadIdx.x] = acc[d];
   __syncthreads();
@@ -201,33 +218,36 @@ __device__ __forceinline__ void kb_jacobi(const float* __restrict__ alu, int64_t
   x0 = a[0] * (x0 - a[2] * x2 - a[1] * x1);
 }
 
-// guard 0: every active system; 2: only systems whose residuals were just
-// replaced (their z is recomputed from the new r)
+__device__ __forceinline__ void diag_one_tile(int t, const Tiles& T, const float* __restrict__ alu, const float* r,
+                                              float* __restrict__ z, const float* __restrict__ q, const BState& S,
+                                              double* part) {
+#pragma clang fp contract(off)
+  const int s = T.sys[t];
+  const int k = threadIdx.x % KS, rl = threadIdx.x / KS;
+  const bool live = !S.done[s * KS + k];
+  double acc[2] = {0.0, 0.0};
+  const int r0 = T.row0[t], nr = T.nrows[t];
+  for (int i = rl; i < nr && live; i += kBT / KS) {
+    const int64_t g = r0 + i;
+    const int64_t o = (g * KS + k) * 3;
+    const float r0v = r[o], r1v = r[o + 1], r2v = r[o + 2];
+    float x0, x1, x2;
+    kb_jacobi(alu, g, r0v, r1v, r2v, x0, x1, x2);
+    z[o] = x0;
+    z[o + 1] = x1;
+    z[o + 2] = x2;
+    acc[0] += (double)r0v * x0 + (double)r1v * x1 + (double)r2v * x2;
+    acc[1] += (double)q[o] * x0 + (double)q[o + 1] * x1 + (double)q[o + 2] * x2;
+  }
+  tile_partials_rowlanes<2>(acc, part, T.ntiles, t);
+}
+// every active system, before the first iteration (after a residual replacement the
+// FP64 SpMM does this for its tiles)
 __global__ __launch_bounds__(kBT) void kb_diag(Tiles T, QView Qv, const float* __restrict__ alu,
                                                const float* __restrict__ r, float* __restrict__ z,
-                                               const float* __restrict__ q, BState S, double* part, int guard) {
+                                               const float* __restrict__ q, BState S, double* part) {
   walk_tiles(Qv, [&](int t) {
-#pragma clang fp contract(off)
-    const int s = T.sys[t];
-    if (S.sys_active[s] == 0) return;
-    if (guard == 2 && S.sys_rel[s] == 0) return;
-    const int k = threadIdx.x % KS, rl = threadIdx.x / KS;
-    const bool live = !S.done[s * KS + k];
-    double acc[2] = {0.0, 0.0};
-    const int r0 = T.row0[t], nr = T.nrows[t];
-    for (int i = rl; i < nr && live; i += kBT / KS) {
-      const int64_t g = r0 + i;
-      const int64_t o = (g * KS + k) * 3;
-      const float r0v = r[o], r1v = r[o + 1], r2v = r[o + 2];
-      float x0, x1, x2;
-      kb_jacobi(alu, g, r0v, r1v, r2v, x0, x1, x2);
-      z[o] = x0;
-      z[o + 1] = x1;
-      z[o + 2] = x2;
-      acc[0] += (double)r0v * x0 + (double)r1v * x1 + (double)r2v * x2;
-      acc[1] += (double)q[o] * x0 + (double)q[o + 1] * x1 + (double)q[o + 2] * x2;
-    }
-    tile_partials_rowlanes<2>(acc, part, T.ntiles, t);
+    if (S.sys_active[T.sys[t]] != 0) diag_one_tile(t, T, alu, r, z, q, S, part);
   });
 }
 
@@ -342,11 +362,20 @@ enum BEpi : int {
   kbEpiStore = 2,  // y = A x (either precision), no partials
 };
 
+// kbEpiRes: the tile's z = D^-1 r and its dots beside the new residual (alu null: not)
+struct BDiag {
+  const float* alu = nullptr;
+  const float* q = nullptr;
+  float* z = nullptr;
+  double* part = nullptr;
+};
+
 template <typename T, int LPR, int RPL, int U, int EPI>
 __device__ __forceinline__ void spmm_one_tile(int t, const Tiles& TL, const int32_t* __restrict__ rowptr,
                                               const int32_t* __restrict__ col, const T* __restrict__ val,
                                               const T* __restrict__ x, const void* __restrict__ w,
-                                              void* __restrict__ y, const BState& S, double* part, int guard) {
+                                              void* __restrict__ y, const BState& S, double* part, int guard,
+                                              const BDiag& D) {
 #pragma clang fp contract(off)
   constexpr int G = KS / RPL, NPH = LPR / G, RPW = 64 / LPR;
   constexpr int ND = EPI == kbEpiQ ? 2 : (EPI == kbEpiRes ? 1 : 0);
@@ -462,6 +491,7 @@ __device__ __forceinline__ void spmm_one_tile(int t, const Tiles& TL, const int3
     // thread (wave, slot, jg, ph=0) holds rhs jg*RPL+j; fixed-order sum over
     // the workgroup's rows for every (dot, rhs)
     __shared__ double red[ND][kBT][RPL];
+    __syncthreads();  // the sums of the workgroup's tile before have been read
 #pragma unroll
     for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -475,155 +505,196 @@ __device__ __forceinline__ void spmm_one_tile(int t, const Tiles& TL, const int3
       part[(int64_t)(d * KS + k) * TL.ntiles + t] = sum;
     }
   }
+  if constexpr (EPI == kbEpiRes)
+    if (D.alu) diag_one_tile(t, TL, D.alu, static_cast<const float*>(y), D.z, D.q, S, D.part);  // r: past the barrier above
 }
 
 template <typename T, int LPR, int RPL, int U, int EPI>
 __global__ __launch_bounds__(kBT) void kb_spmm(Tiles TL, QView Qv, const int32_t* __restrict__ rowptr,
                                                const int32_t* __restrict__ col, const T* __restrict__ val,
                                                const T* __restrict__ x, const void* __restrict__ w,
-                                               void* __restrict__ y, BState S, double* part, int guard) {
-  walk_tiles(Qv, [&](int t) { spmm_one_tile<T, LPR, RPL, U, EPI>(t, TL, rowptr, col, val, x, w, y, S, part, guard); });
+                                               void* __restrict__ y, BState S, double* part, int guard, BDiag D) {
+  walk_tiles(Qv, [&](int t) { spmm_one_tile<T, LPR, RPL, U, EPI>(t, TL, rowptr, col, val, x, w, y, S, part, guard, D); });
 }
 
 // ---- per-system tails: sum a system's tile partials, then the CG scalar logic ---------
 enum BTail : int { kbInit = 0, kbBeta = 1, kbAlpha = 2, kbRes = 3, kbRel = 4 };
 
-template <int TAIL, int ND>
-__global__ __launch_bounds__(kBT) void kb_tail(Tiles T, BState S, const double* part) {
-  const int s = blockIdx.x;
-  if (TAIL != kbInit && S.sys_active[s] == 0) return;
-  const int k = threadIdx.x % KS;
-  const int t0 = T.sys_tile0[s], nt = T.sys_ntile[s];
-  __shared__ double red[ND][kBT];
-  __shared__ int32_t flag[KS];
-  {
-    // 16 threads per right-hand side sweep the system's tile partials, which
-    // are contiguous per (dot, rhs), with 8 independent loads in flight; a
-    // fixed order throughout
-    constexpr int kSub = kBT / KS;
-    const int kl = threadIdx.x / kSub, sub = threadIdx.x % kSub;
+// totals of ND inner products of right-hand side `k` over a system's tiles, by one wave
+// (fixed order, the same on every lane)
+template <int ND>
+__device__ __forceinline__ void tile_totals(const Tiles& T, int t0, int nt, int k, const double* part, double (&tot)[ND]) {
+  const int lane = threadIdx.x & 63;
+  constexpr int kU = 8;
 #pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      const double* __restrict__ pp = part + (int64_t)(d * KS + kl) * T.ntiles + t0;
-      double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-      int i = sub;
-      for (; i + 7 * kSub < nt; i += 8 * kSub)
+  for (int d = 0; d < ND; ++d) tot[d] = 0.0;
+  for (int i0 = 0; i0 < nt; i0 += 64 * kU) {
+    double v[ND][kU];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[u] += pp[i + u * kSub];
-      for (; i < nt; i += kSub) a[0] += pp[i];
-      red[d][threadIdx.x] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-    }
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const int i = i0 + 64 * u + lane;
+        v[d][u] = part[(int64_t)(d * KS + k) * T.ntiles + t0 + min(i, nt - 1)];
+      }
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int u = 0; u < kU; ++u) tot[d] += i0 + 64 * u + lane < nt ? v[d][u] : 0.0;
   }
-  __syncthreads();
-  if (threadIdx.x < KS) {
-    double tot[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      double a = 0.0;
-      for (int m = 0; m < kBT / KS; ++m) a += red[d][k * (kBT / KS) + m];
-      tot[d] = a;
-    }
-    const int id = s * KS + k;
-    int32_t fl = 0;
-    if (TAIL == kbInit) {
-      // tot[0] = b.b, tot[1] = |b - A x0|^2
-      S.bnrm2[id] = tot[0];
-      S.rr_ref[id] = tot[ND - 1];
-      S.rho[id] = S.rho1[id] = S.zq[id] = S.pq[id] = S.rp[id] = S.alpha[id] = S.beta[id] = 0.0;
-      S.gap[id] = 1.0;
-      S.iter[id] = 1;
-      S.nindef[id] = 0;
-      S.rel[id] = 0;
-      S.error[id] = 0;
-      S.resid[id] = tot[0] == 0.0 ? 0.0 : sqrt(tot[ND - 1] / tot[0]);
-      // b = 0: x = 0 and nothing to do (hecmw_solver_CG.f90:135-141); the
-      // caller zeroes x for such instances
-      S.done[id] = (tot[0] == 0.0 || S.iprm[0] < 1) ? 1 : 0;
-      fl = !S.done[id];
-    } else if (!S.done[id]) {
-      if (TAIL == kbBeta) {
-        const double rho = tot[0];
-        S.rho[id] = rho;
-        S.zq[id] = tot[1];
-        const int it = S.iter[id];
-        if (rho == 0.0) {
-          S.done[id] = 1;
-        } else if (rho != rho) {
-          S.error[id] = kErrDivergeNan;
-          S.done[id] = 1;
-        } else if (it > 1 && rho * S.rho1[id] <= 0.0) {
-          S.nindef[id] += 1;
-          if (S.nindef[id] >= 3) {
-            S.error[id] = kErrDivergePc;
-            S.done[id] = 1;
-          }
-        }
-        if (!S.done[id]) S.beta[id] = it > 1 ? -S.zq[id] / S.pq[id] : 0.0;
-      } else if (TAIL == kbAlpha) {
-        const double pq = tot[0], rp = tot[1];
-        S.pq[id] = pq;
-        S.rp[id] = rp;
-        if (pq <= 0.0) {
-          S.error[id] = kErrDivergeMat;
-          S.done[id] = 1;
-        } else if (pq != pq || rp != rp) {
-          S.error[id] = kErrDivergeNan;
-          S.done[id] = 1;
-        } else {
-          S.alpha[id] = rp / pq;
-        }
-      } else if (TAIL == kbRes) {
-        const double rr = tot[0];
-        S.resid[id] = sqrt(rr / S.bnrm2[id]);
-        S.rel[id] = S.resid[id] * S.gap[id] <= S.prm[0] || rr <= S.prm[1] * S.rr_ref[id] ||
-                    (S.iter[id] % S.iprm[1]) == 0 || rr != rr;
-        fl = S.rel[id];
-      } else if (TAIL == kbRel) {
-        if (S.rel[id]) {
-          const double rr = tot[0];
-          const double rec = S.resid[id];
-          S.rr_ref[id] = rr;
-          S.resid[id] = sqrt(rr / S.bnrm2[id]);
-          if (rec > 0.0) S.gap[id] = fmin(1e3, fmax(1.0, S.resid[id] / rec));
-          S.rel[id] = 0;
-          if (S.resid[id] <= S.prm[0]) {
-            S.done[id] = 1;
-          } else if (rr != rr) {
-            S.error[id] = kErrDivergeNan;
-            S.done[id] = 1;
-          }
-        }
-        if (!S.done[id]) {
-          if (S.iter[id] >= S.iprm[0]) {
-            S.error[id] = kErrNoconv;
-            S.done[id] = 1;
-            S.iter[id] = S.iprm[0] + 1;
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) tot[d] += __shfl_xor(tot[d], off, 64);
+}
+
+// an instance's state in registers: all of it is read before the first use and the
+// first store, so that a tail waits for memory once
+struct Inst {
+  int32_t done, iter, rel, nindef, error;
+  double resid, gap, bnrm2, rr_ref, rho, rho1, pq;
+  __device__ __forceinline__ Inst(const BState& S, int id)
+      : done(S.done[id]), iter(S.iter[id]), rel(S.rel[id]), nindef(S.nindef[id]), error(S.error[id]), resid(S.resid[id]),
+        gap(S.gap[id]), bnrm2(S.bnrm2[id]), rr_ref(S.rr_ref[id]), rho(S.rho[id]), rho1(S.rho1[id]), pq(S.pq[id]) {}
+  __device__ __forceinline__ void stop(int32_t e) {
+    error = e ? e : error;
+    done = 1;
+  }
+};
+
+// beta of the next iteration from r.z and z.q
+__device__ __forceinline__ void tail_beta(const BState& S, int id, Inst& v, const double (&tot)[2]) {
+  v.rho = tot[0];
+  S.rho[id] = v.rho;
+  S.zq[id] = tot[1];
+  if (v.rho == 0.0) {
+    v.stop(0);
+  } else if (v.rho != v.rho) {
+    v.stop(kErrDivergeNan);
+  } else if (v.iter > 1 && v.rho * v.rho1 <= 0.0) {
+    v.nindef += 1;
+    S.nindef[id] = v.nindef;
+    if (v.nindef >= 3) v.stop(kErrDivergePc);
+  }
+  if (!v.done) S.beta[id] = v.iter > 1 ? -tot[1] / v.pq : 0.0;
+}
+
+// One workgroup per system, a wave per right-hand side.  kbRes and kbRel end with the
+// list that follows from their flags (the last workgroup to arrive builds it), and kbRel
+// goes on to the next iteration's beta, so that an iteration is eight launches: as
+// four kernels of their own the lists, beta and the DIAG step after a replacement took
+// 4-8 us each.
+template <int TAIL, int ND>
+__global__ __launch_bounds__(kTailThreads) void kb_tail(Tiles T, BState S, const double* part, const double* part_rz,
+                                                        Queue Q) {
+  const int s = blockIdx.x, k = threadIdx.x / 64, id = s * KS + k;
+  __shared__ int32_t flag[KS], gone[KS];
+  __shared__ int32_t last;
+  if (TAIL == kbInit || S.sys_active[s] != 0) {
+    Inst v(S, id);
+    const double tol = S.prm[0], delta2 = S.prm[1];
+    const int32_t maxit = S.iprm[0], nrec = S.iprm[1];
+    const int t0 = T.sys_tile0[s], nt = T.sys_ntile[s];
+    double tot[ND], rz[2] = {0.0, 0.0};
+    tile_totals<ND>(T, t0, nt, k, part, tot);
+    if (TAIL == kbRel) tile_totals<2>(T, t0, nt, k, part_rz, rz);
+    if (threadIdx.x % 64 == 0) {
+      int32_t fl = 0;
+      if (TAIL == kbInit) {
+        // tot[0] = b.b, tot[1] = |b - A x0|^2
+        S.bnrm2[id] = tot[0];
+        S.rr_ref[id] = tot[ND - 1];
+        S.rho[id] = S.rho1[id] = S.zq[id] = S.pq[id] = S.rp[id] = S.alpha[id] = S.beta[id] = 0.0;
+        S.gap[id] = 1.0;
+        S.iter[id] = 1;
+        S.nindef[id] = 0;
+        S.rel[id] = 0;
+        v.error = 0;
+        S.resid[id] = tot[0] == 0.0 ? 0.0 : sqrt(tot[ND - 1] / tot[0]);
+        // b = 0: x = 0 and nothing to do (hecmw_solver_CG.f90:135-141); the
+        // caller zeroes x for such instances
+        v.done = (tot[0] == 0.0 || maxit < 1) ? 1 : 0;
+      } else if (!v.done) {
+        if constexpr (TAIL == kbBeta) {
+          tail_beta(S, id, v, tot);
+        } else if (TAIL == kbAlpha) {
+          const double pq = tot[0], rp = tot[ND - 1];
+          S.pq[id] = pq;
+          S.rp[id] = rp;
+          if (pq <= 0.0) {
+            v.stop(kErrDivergeMat);
+          } else if (pq != pq || rp != rp) {
+            v.stop(kErrDivergeNan);
           } else {
-            S.rho1[id] = S.rho[id];
-            S.iter[id] += 1;
+            S.alpha[id] = rp / pq;
+          }
+        } else if (TAIL == kbRes) {
+          const double rr = tot[0];
+          v.resid = sqrt(rr / v.bnrm2);
+          S.resid[id] = v.resid;
+          fl = v.resid * v.gap <= tol || rr <= delta2 * v.rr_ref || v.iter % nrec == 0 || rr != rr;
+        } else if (TAIL == kbRel) {
+          if (v.rel) {
+            const double rr = tot[0];
+            const double rec = v.resid;
+            S.rr_ref[id] = rr;
+            v.resid = sqrt(rr / v.bnrm2);
+            S.resid[id] = v.resid;
+            if (rec > 0.0) S.gap[id] = fmin(1e3, fmax(1.0, v.resid / rec));
+            S.rel[id] = 0;
+            if (v.resid <= tol) {
+              v.stop(0);
+            } else if (rr != rr) {
+              v.stop(kErrDivergeNan);
+            }
+          }
+          if (!v.done) {
+            if (v.iter >= maxit) {
+              v.stop(kErrNoconv);
+              v.iter = maxit + 1;
+            } else {
+              v.rho1 = v.rho;
+              S.rho1[id] = v.rho1;
+              v.iter += 1;
+            }
+            S.iter[id] = v.iter;
           }
         }
       }
+      if (TAIL == kbRel || TAIL == kbInit) fl = !v.done;
+      flag[k] = fl;
+      gone[k] = v.done;
+      if constexpr (TAIL == kbRel)
+        if (!v.done) tail_beta(S, id, v, rz);
+      S.error[id] = v.error;
+      S.done[id] = v.done;
     }
-    if (TAIL == kbRel || TAIL == kbInit) fl = !S.done[id];
-    flag[k] = fl;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
+    __syncthreads();
     int32_t n = 0;
     for (int j = 0; j < KS; ++j) n += flag[j];
     // The FP64 residual costs the same for one right-hand side as for all of
     // a system's: when one asks for it, every live one is refreshed, so their
     // reference norms stay aligned and the next replacement comes later.
-    if (TAIL == kbRes && n > 0)
-      for (int j = 0; j < KS; ++j)
-        if (!S.done[s * KS + j]) S.rel[s * KS + j] = 1;
-    if (TAIL == kbRes) S.sys_rel[s] = n > 0;
-    // a finished system's tails return early from now on: clear its request
-    // here, or the FP64 residual SpMM would keep computing its tiles
-    if (TAIL == kbRel) S.sys_rel[s] = 0;
-    if (TAIL == kbRel || TAIL == kbInit) S.sys_active[s] = n;
-    if (TAIL == kbInit) S.sys_rel[s] = n > 0;
+    if (TAIL == kbRes && threadIdx.x < KS) S.rel[s * KS + threadIdx.x] = n > 0 && !gone[threadIdx.x];
+    if (threadIdx.x == 0) {
+      // a finished system's tails return early from now on: clear its request
+      // here, or the FP64 residual SpMM would keep computing its tiles
+      auto set = [](int32_t* p, int32_t x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+      if (TAIL == kbRes || TAIL == kbInit) set(S.sys_rel + s, n > 0);
+      if (TAIL == kbRel) set(S.sys_rel + s, 0);
+      if (TAIL == kbRel || TAIL == kbInit) set(S.sys_active + s, n);
+    }
+  }
+  if (TAIL == kbRes || TAIL == kbRel) {
+    if (threadIdx.x == 0) {
+      // the flags above first
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      last = __hip_atomic_fetch_add(Q.n + kqLists, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    if (threadIdx.x == 0) Q.n[kqLists] = 0;
+    build_queue<TAIL == kbRes ? kqRel : kqActive>(T, gridDim.x, S, Q);
   }
 }
 
@@ -651,14 +722,14 @@ __global__ void kb_to_f32(int64_t n, const double* __restrict__ a, float* __rest
 
 // ---- SpMM variant table ------------------------------------------------------------------
 using SpmmFn = void (*)(int grid, hipStream_t, Tiles, QView, const int32_t*, const int32_t*, const void*,
-                        const void*, const void*, void*, BState, double*, int);
+                        const void*, const void*, void*, BState, double*, int, BDiag);
 using OccFn = int (*)();
 
 template <typename T, int LPR, int RPL, int U, int EPI>
 void spmm_launch(int grid, hipStream_t st, Tiles tl, QView qv, const int32_t* rp, const int32_t* col, const void* val,
-                 const void* x, const void* w, void* y, BState S, double* part, int guard) {
+                 const void* x, const void* w, void* y, BState S, double* part, int guard, BDiag d) {
   kb_spmm<T, LPR, RPL, U, EPI><<<grid, kBT, 0, st>>>(tl, qv, rp, col, static_cast<const T*>(val),
-                                                     static_cast<const T*>(x), w, y, S, part, guard);
+                                                     static_cast<const T*>(x), w, y, S, part, guard, d);
 }
 
 // resident workgroups of a kernel per CU (the persistent grid is that times the CU count)
@@ -836,28 +907,23 @@ static void batch_enqueue_iteration(hecmw33_batch& B) {
   hipStream_t st = B.stream;
   double* part = B.part.as<double>();
   float *r = B.r.as<float>(), *z = B.z.as<float>(), *p = B.p.as<float>(), *q = B.q.as<float>();
-  // z = D^-1 r and its dots (r.z, z.q) come from the previous iteration's
-  // kb_update_diag (or kb_diag after a residual replacement, or before the
-  // first iteration), in the second half of the partials
+  // z = D^-1 r and its dots (r.z, z.q), in the second half of the partials, and beta come
+  // from the iteration before, or from the start of the solve
   double* part_rz = part + (size_t)2 * KS * B.ntiles;
-  kb_tail<kbBeta, 2><<<B.nsys, kBT, 0, st>>>(B.T, B.S, part_rz);
+  const BDiag diag{B.alu32.as<float>(), q, z, part_rz};
   kb_p<<<B.grid_p, kBT, 0, st>>>(B.T, qview(B, kqActive), z, p, B.S);
   kVariants[B.variant].q32(B.grid_q, st, B.T, qview(B, kqActive), B.rowptr.as<int32_t>(), B.col.as<int32_t>(),
-                           B.val32.p, p, r, q, B.S, part, 1);
-  kb_tail<kbAlpha, 2><<<B.nsys, kBT, 0, st>>>(B.T, B.S, part);
+                           B.val32.p, p, r, q, B.S, part, 1, BDiag{});
+  kb_tail<kbAlpha, 2><<<B.nsys, kTailThreads, 0, st>>>(B.T, B.S, part, nullptr, queue_of(B));
   kb_update_diag<<<B.grid_upd, kBT, 0, st>>>(B.T, qview(B, kqActive), B.alu32.as<float>(), p, q,
                                              B.dx.as<float>(), r, z, B.S, part, part_rz);
-  kb_tail<kbRes, 1><<<B.nsys, kBT, 0, st>>>(B.T, B.S, part);
-  // the systems whose residuals are replaced now, their x brought up to date
-  kb_queue<kqRel><<<1, 1024, 0, st>>>(B.T, B.nsys, B.S, queue_of(B));
+  // then the systems whose residuals are replaced now, their x brought up to date, z from the new r
+  kb_tail<kbRes, 1><<<B.nsys, kTailThreads, 0, st>>>(B.T, B.S, part, nullptr, queue_of(B));
   kb_fold<<<B.grid_res, kBT, 0, st>>>(B.T, qview(B, kqRel), B.dx.as<float>(), B.x.as<double>(), B.S, 2);
   kVariants64[B.variant64].res(B.grid_res, st, B.T, qview(B, kqRel), B.rowptr.as<int32_t>(),
-                               B.col.as<int32_t>(), B.val64.p, B.x.p, B.b.p, r, B.S, part, 2);
-  // systems whose residuals were just replaced: z from the new r
-  kb_diag<<<B.grid_diag, kBT, 0, st>>>(B.T, qview(B, kqRel), B.alu32.as<float>(), r, z, q, B.S, part_rz, 2);
-  kb_tail<kbRel, 1><<<B.nsys, kBT, 0, st>>>(B.T, B.S, part);
-  // the systems still running after this iteration, and their live count for the host
-  kb_queue<kqActive><<<1, 1024, 0, st>>>(B.T, B.nsys, B.S, queue_of(B));
+                               B.col.as<int32_t>(), B.val64.p, B.x.p, B.b.p, r, B.S, part, 2, diag);
+  // the systems still running after this iteration, their live count for the host, and beta
+  kb_tail<kbRel, 1><<<B.nsys, kTailThreads, 0, st>>>(B.T, B.S, part, part_rz, queue_of(B));
 }
 
 // ---- the autotuner's winners, persisted per (blocks per row, rows) bucket ------------------
@@ -995,8 +1061,8 @@ static int32_t batch_autotune(hecmw33_batch& B) {
   BHIPC(hipMemcpyAsync(B.S.sys_active, ones.data(), sizeof(int32_t) * B.nsys, hipMemcpyHostToDevice, B.stream));
   BHIPC(hipMemcpyAsync(B.S.sys_rel, ones.data(), sizeof(int32_t) * B.nsys, hipMemcpyHostToDevice, B.stream));
   // both live-tile lists: every tile
-  kb_queue<kqActive><<<1, 1024, 0, B.stream>>>(B.T, B.nsys, B.S, queue_of(B));
-  kb_queue<kqRel><<<1, 1024, 0, B.stream>>>(B.T, B.nsys, B.S, queue_of(B));
+  kb_queue<kqActive><<<1, kTailThreads, 0, B.stream>>>(B.T, B.nsys, B.S, queue_of(B));
+  kb_queue<kqRel><<<1, kTailThreads, 0, B.stream>>>(B.T, B.nsys, B.S, queue_of(B));
   auto timed = [&](auto one, int warm, int reps, float* ms) -> int32_t {
     for (int rep = 0; rep < warm; ++rep) one();
     BHIPC(hipEventRecord(e0, B.stream));
@@ -1012,7 +1078,7 @@ static int32_t batch_autotune(hecmw33_batch& B) {
     return timed(
         [&]() {
           kVariants[v].q32(g, B.stream, B.T, qview(B, kqActive), B.rowptr.as<int32_t>(), B.col.as<int32_t>(),
-                           B.val32.p, B.p.p, B.r.p, B.q.p, B.S, B.part.as<double>(), 1);
+                           B.val32.p, B.p.p, B.r.p, B.q.p, B.S, B.part.as<double>(), 1, BDiag{});
         },
         2, 5, &B.variant_ms[v]);
   };
@@ -1021,7 +1087,7 @@ static int32_t batch_autotune(hecmw33_batch& B) {
     return timed(
         [&]() {
           kVariants64[v].res(g, B.stream, B.T, qview(B, kqRel), B.rowptr.as<int32_t>(), B.col.as<int32_t>(),
-                             B.val64.p, B.x.p, B.b.p, B.r.p, B.S, B.part.as<double>(), 2);
+                             B.val64.p, B.x.p, B.b.p, B.r.p, B.S, B.part.as<double>(), 2, BDiag{});
         },
         1, 3, &B.variant64_ms[v]);
   };
@@ -1184,7 +1250,7 @@ static int32_t batch_load(hecmw33_batch& B, int32_t nsys, const hecmw33_sys* sys
       B.z.ensure(sizeof(float) * nv) ||
       B.p.ensure(sizeof(float) * nv) || B.q.ensure(sizeof(float) * nv) ||
       B.part.ensure(sizeof(double) * 4 * KS * (size_t)B.ntiles) || batch_state_layout(B) ||
-      B.qtile.ensure(sizeof(int32_t) * kqLists * (size_t)B.ntiles) || B.qn.ensure(sizeof(int32_t) * kqLists))
+      B.qtile.ensure(sizeof(int32_t) * kqLists * (size_t)B.ntiles) || B.qn.ensure(sizeof(int32_t) * (kqLists + 1)))
     return HECMW33_ERROR_DEVICE;
   hipStream_t st = B.stream;
   BHIPC(hipMemcpyAsync(B.rowptr.p, rp.data(), sizeof(int32_t) * rp.size(), hipMemcpyHostToDevice, st));
@@ -1231,6 +1297,7 @@ static int32_t batch_load(hecmw33_batch& B, int32_t nsys, const hecmw33_sys* sys
   B.T.sys_tile0 = B.sys_tile0.as<int32_t>();
   B.T.sys_ntile = B.sys_ntile.as<int32_t>();
   B.T.ntiles = B.ntiles;
+  BHIPC(hipMemsetAsync(B.qn.p, 0, sizeof(int32_t) * (kqLists + 1), st));
   for (BMem* m : {&B.r, &B.z, &B.p, &B.q}) kb_fill0<<<grid_of(nv), kBT, 0, st>>>(nv, m->as<float>());
   BHIPC(hipGetLastError());
   BHIPC(hipStreamSynchronize(st));
@@ -1268,13 +1335,14 @@ static int32_t batch_solve(hecmw33_batch& B, const int32_t* iarray, const double
   BHIPC(hipMemcpyAsync(B.S.sys_rel, sys1.data(), sizeof(int32_t) * B.nsys, hipMemcpyHostToDevice, st));
   // |b - A x0|^2 into the second dot slot
   kVariants64[B.variant64].res(B.ntiles, st, B.T, qall(), B.rowptr.as<int32_t>(), B.col.as<int32_t>(), B.val64.p,
-                               B.x.p, B.b.p, B.r.p, B.S, part + (size_t)KS * B.ntiles, 0);
-  kb_tail<kbInit, 2><<<B.nsys, kBT, 0, st>>>(B.T, B.S, part);
+                               B.x.p, B.b.p, B.r.p, B.S, part + (size_t)KS * B.ntiles, 0, BDiag{});
+  kb_tail<kbInit, 2><<<B.nsys, kTailThreads, 0, st>>>(B.T, B.S, part, nullptr, queue_of(B));
   // the first iteration's z = D^-1 r0 and its dots
   kb_diag<<<B.ntiles, kBT, 0, st>>>(B.T, qall(), B.alu32.as<float>(), B.r.as<float>(), B.z.as<float>(),
-                                    B.q.as<float>(), B.S, part + (size_t)2 * KS * B.ntiles, 0);
+                                    B.q.as<float>(), B.S, part + (size_t)2 * KS * B.ntiles);
+  kb_tail<kbBeta, 2><<<B.nsys, kTailThreads, 0, st>>>(B.T, B.S, part + (size_t)2 * KS * B.ntiles, nullptr, queue_of(B));
   // the systems the first iteration runs
-  kb_queue<kqActive><<<1, 1024, 0, st>>>(B.T, B.nsys, B.S, queue_of(B));
+  kb_queue<kqActive><<<1, kTailThreads, 0, st>>>(B.T, B.nsys, B.S, queue_of(B));
   BHIPC(hipGetLastError());
   BHIPC(hipStreamSynchronize(st));
   const auto t1 = std::chrono::steady_clock::now();
@@ -1389,13 +1457,13 @@ int32_t hecmw33_batch_spmm(hecmw33_batch* b, int32_t fp64, const double* const* 
   if (fp64) {
     const int v = fp64 >= 2 ? fp64 - 2 : b->variant64;
     kVariants64[v].st(b->ntiles, st, b->T, qall(), b->rowptr.as<int32_t>(), b->col.as<int32_t>(), b->val64.p, xin.p,
-                      nullptr, yout.p, b->S, nullptr, 0);
+                      nullptr, yout.p, b->S, nullptr, 0, BDiag{});
   } else {
     float* x32 = b->z.as<float>();  // scratch: the solve re-initialises it
     float* y32 = b->q.as<float>();
     kb_to_f32<<<grid_of(nv), kBT, 0, st>>>(nv, xin.as<double>(), x32);
     kVariants[b->variant].st32(b->ntiles, st, b->T, qall(), b->rowptr.as<int32_t>(), b->col.as<int32_t>(),
-                               b->val32.p, x32, nullptr, y32, b->S, nullptr, 0);
+                               b->val32.p, x32, nullptr, y32, b->S, nullptr, 0, BDiag{});
     BHIPC(hipStreamSynchronize(st));
     std::vector<float> hf(nv);
     BHIPC(hipMemcpy(hf.data(), y32, sizeof(float) * nv, hipMemcpyDeviceToHost));

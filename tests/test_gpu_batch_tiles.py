@@ -37,3 +37,38 @@ def test_tiles_by_batch_size(n, rows_per_tile):
             r = Bs[s][k] - restate.matvec(m, x[k])
             assert np.linalg.norm(r) <= 1.001e-8 * np.linalg.norm(Bs[s][k])
     bs.close()
+
+
+def test_instances_that_stop_at_different_times():
+    """A zero column, NOCONV for all others at MAXIT 6 (ITER 7), then a solve to the end on the
+    same loaded batch, whose instances converge in different iterations, one system long
+    before the others: every solution within 1e-6 of the restatement's DIAG-CG."""
+    mats = [fa.gen_hex8(1), fa.gen_hex8(9, kind="lognormal", seed=2), fa.gen_tet10(4, 2, 3, seed=1)[0], fa.gen_hex8(5)]
+    rng = np.random.default_rng(3)
+    Bs = [rng.standard_normal((3, 3 * m.N)) for m in mats]
+    Bs[1][2][:] = 0.0
+    bs = fa.BatchSolver(mats, Bs)
+    p = fa.gen_hex8(1)
+    p.set_precond(3)
+    p.set_iter(6)
+    it, er, rs, _ = bs.solve(p.Iarray.copy(), p.Rarray.copy())
+    live = np.ones_like(er, dtype=bool)
+    live[1, 2] = False
+    assert np.all(er[live] == 3001) and np.all(it[live] == 7)
+    assert it[1, 2] == 1 and er[1, 2] == 0 and np.all(bs.x(1)[2] == 0.0)
+    p.set_iter(5000)
+    it, er, rs, _ = bs.solve(p.Iarray.copy(), p.Rarray.copy())
+    assert np.all(er == 0) and np.all(rs <= 1e-8) and it[1, 2] == 1
+    for s, m in enumerate(mats):
+        X = bs.x(s)
+        for k in range(3):
+            mk = m.copy()
+            mk.B[:] = Bs[s][k]
+            mk.set_precond(3)
+            mk.set_iter(5000)
+            if not live[s, k]:
+                continue
+            xr, info = restate.solve_krylov(mk)
+            assert info["error"] == 0 and it[s, k] <= 1.3 * info["iter"] + 10
+            assert np.linalg.norm(X[k] - xr) <= 1e-6 * np.linalg.norm(xr)
+    bs.close()
