@@ -281,7 +281,10 @@ struct ResidentOp {
   const int32_t* node_slot = nullptr;
   double* rec = nullptr;                // the LU of D' and the vectors: per 16 slots, `planes` planes
   int32_t planes = 0;                   // kResidentPlanesCg or kResidentPlanesBi, which picks the method
-  double* zw = nullptr;                 // the gathered vectors, two copies of ns + 1 records
+  double* zw = nullptr;                 // the gathered vectors, `ring` copies of ns + 1 records
+  int32_t ring = 2;
+  bool cached = false;                  // gathers look into the caches first (ring > 2)
+  bool stream = false;                  // matrix loads leave the caches to the rest
   double* xn = nullptr;               // x in node order
   const double* b = nullptr;          // right-hand side in node order
   double* hist = nullptr;

@@ -14,9 +14,13 @@
 //    it again until it is: no barrier between colours, no flag, no store to be
 //    waited for.  (With grid barriers between the colours a step cost 3.7 us at
 //    9,261 nodes, 2.2 us of them the barrier.)
-//  * Every entry is written once per sweep.  Two copies alternate, and a
-//    backward sweep puts the marks back into the copy that the sweep before
-//    used; the reductions between the sweeps are grid barriers.
+//  * Every entry is written once per sweep.  Copies take turns, and a backward
+//    sweep puts the marks back into the copy that the sweep before used; the
+//    reductions between the sweeps are grid barriers.  With four copies the first
+//    look at an entry goes through the caches (a record is gathered about 13 times in
+//    a sweep, and past the caches that was half of the memory traffic at 72^3); an
+//    old line can only hold marks, which are asked for again past the caches, because
+//    the lines go once per turn of the copies.
 //
 // The iteration needs the off-diagonal blocks once, not twice as SSOR
 // application + product do.  With A = L + D + U and M = (D'+L) D'^-1 (D'+U)
@@ -34,11 +38,11 @@
 //     p, q, g; partial p.q
 // Measured, us per iteration, launches per colour -> resident (HEX8 cubes and a
 // TET10 box, relative residual 1e-10): 343 nodes 183 -> 47, 4,845 (TET10) 441 ->
-// 82, 9,261 298 -> 66, 29,791 289 -> 67, 74,088 376 -> 87, 389,017 717 -> 379,
-// 1,030,301 1400 -> 950, 2,248,091 2740 -> 2180.  Up to 100,000 nodes the 2 x 16
-// colour steps bound it (1.5-2 us each: gather round trip, row work, the way of
-// the stores to the neighbours' gathers); above, the round trips of a wave's
-// tasks (8 waves per CU; the matrix stream alone would take 200 us at 389,017).
+// 82, 9,261 298 -> 62, 29,791 289 -> 64, 74,088 376 -> 80, 389,017 717 -> 291,
+// 1,030,301 1400 -> 774.  Up to 100,000 nodes the 2 x 16 colour steps bound it
+// (1.5-2 us each: gather round trip, row work, the way of the stores to the
+// neighbours' gathers); above, the round trips of a wave's tasks (8 waves per CU; the
+// matrix stream alone would take 200 us at 389,017).
 //
 // The true residual b - A x (every 50 iterations and before convergence is
 // declared, as the reference does) is formed in natural order with the rows of
@@ -47,6 +51,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "device.h"
 #include "resident.h"
@@ -61,13 +66,15 @@ namespace {
 // take 16 bytes with the agent-scope bit.
 using V4 = __attribute__((__vector_size__(16))) uint32_t;
 using V2 = __attribute__((__vector_size__(8))) uint32_t;
+template <int AUX>
 __device__ __forceinline__ void gather16(__amdgpu_buffer_rsrc_t r, uint32_t off, double& a, double& b) {
-  const V4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kAuxSc1);
+  const V4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX);
   a = __hiloint2double((int)v[1], (int)v[0]);
   b = __hiloint2double((int)v[3], (int)v[2]);
 }
+template <int AUX>
 __device__ __forceinline__ double gather8(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  const V2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kAuxSc1);
+  const V2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX);
   return __hiloint2double((int)v[1], (int)v[0]);
 }
 
@@ -86,6 +93,19 @@ struct LdsMap {
     return sizeof(double) * (range + 2 * (size_t)(ncolor + 1) + (one_group_slots ? 12 * ((size_t)one_group_slots + 1) : 0));
   }
 };
+
+// aval_load past the caches' replacement
+__device__ __forceinline__ void aval_load_nt(const double* __restrict__ val, int64_t g, int r, double (&v)[9]) {
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  const double* __restrict__ b = val + g * (9 * kRowsA);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const D2 t = __builtin_nontemporal_load(reinterpret_cast<const D2*>(b + q * (2 * kRowsA) + 2 * r));
+    v[2 * q] = t.x;
+    v[2 * q + 1] = t.y;
+  }
+  v[8] = __builtin_nontemporal_load(b + 8 * kRowsA + r);
+}
 
 template <int T, int K, int MEM>
 struct Resident : GridGroup<T, MEM> {
@@ -124,11 +144,11 @@ struct Resident : GridGroup<T, MEM> {
     copy_size = ((int64_t)o.ns + 1) * kRec;
     if (MEM == kGrid) {
       zw0 = o.zw;
-      rsrc = __builtin_amdgcn_make_buffer_rsrc(o.zw, 0, (int)(uint32_t)(2 * sizeof(double) * copy_size), 0x00020000);
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(o.zw, 0, (int)(uint32_t)(o.ring * sizeof(double) * copy_size), 0x00020000);
     } else {
       zw0 = lds + Map::range + 2 * (nc + 1);
       // the state of the gathered vectors between launches is in o.zw
-      for (int64_t i = threadIdx.x; i < 2 * copy_size; i += T) zw0[i] = o.zw[i];
+      for (int64_t i = threadIdx.x; i < o.ring * copy_size; i += T) zw0[i] = o.zw[i];
     }
     // this workgroup's run of the tasks of every colour, and how many go before
     for (int i = threadIdx.x; i < 2 * (nc + 1); i += T) {
@@ -151,6 +171,19 @@ struct Resident : GridGroup<T, MEM> {
     __syncthreads();
   }
 
+  __device__ __forceinline__ int next_copy() const { return par + 1 == o.ring ? 0 : par + 1; }
+  __device__ __forceinline__ int last_copy() const { return par == 0 ? o.ring - 1 : par - 1; }
+  // The caches may hold lines of a copy from before its marks were put back: between the
+  // barrier behind the last gather or mark of that time and the next gather, they go.
+  __device__ __forceinline__ void drop_lines() {
+    if (MEM == kOneGroup || !o.cached) return;
+    if (wave == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    wg_barrier();
+  }
+  // once per turn of the ring, before copy cp is gathered
+  __device__ __forceinline__ void enter(int cp) {
+    if (cp == 0) drop_lines();
+  }
   __device__ __forceinline__ double* zw(int cp, int slot) const { return zw0 + cp * copy_size + (int64_t)kRec * slot; }
 
   // The wave's place j in the workgroup's order of the sweep in direction d (0
@@ -179,8 +212,13 @@ struct Resident : GridGroup<T, MEM> {
 #pragma unroll
       for (int e = 0; e < 9; ++e) v[k][e] = 0.0;
       if (used) {
-        c[k] = o.col[g * kWave + lane];
-        aval_load(o.val, g, lane, v[k]);
+        if (o.stream) {
+          c[k] = __builtin_nontemporal_load(o.col + g * kWave + lane);
+          aval_load_nt(o.val, g, lane, v[k]);
+        } else {
+          c[k] = o.col[g * kWave + lane];
+          aval_load(o.val, g, lane, v[k]);
+        }
       }
     }
   }
@@ -199,19 +237,25 @@ struct Resident : GridGroup<T, MEM> {
 #pragma unroll
     for (int k = 0; k < K; ++k) want[k] = true;
     uint64_t t0 = 0;
+    auto fetch = [&](int k, auto aux) {
+      const uint32_t off = (uint32_t)(cp * copy_size * 8) + (uint32_t)c[k] * (8u * kRec);
+      gather16<aux.value>(rsrc, off, x[k][0], x[k][1]);
+      if constexpr (NG > 1) {
+        gather16<aux.value>(rsrc, off + 16, x[k][2], x[k][3]);
+        gather16<aux.value>(rsrc, off + 32, x[k][4], x[k][5]);
+      } else {
+        x[k][2] = gather8<aux.value>(rsrc, off + 16);
+      }
+    };
     for (uint32_t spins = 1;; ++spins) {
 #pragma unroll
       for (int k = 0; k < K; ++k)
         if (want[k]) {
           if constexpr (MEM == kGrid) {
-            const uint32_t off = (uint32_t)(cp * copy_size * 8) + (uint32_t)c[k] * (8u * kRec);
-            gather16(rsrc, off, x[k][0], x[k][1]);
-            if constexpr (NG > 1) {
-              gather16(rsrc, off + 16, x[k][2], x[k][3]);
-              gather16(rsrc, off + 32, x[k][4], x[k][5]);
-            } else {
-              x[k][2] = gather8(rsrc, off + 16);
-            }
+            if (spins == 1 && o.cached)
+              fetch(k, std::integral_constant<int, 0>{});
+            else
+              fetch(k, std::integral_constant<int, kAuxSc1>{});
           } else {
             const volatile double* q = zw(cp, c[k]);
 #pragma unroll
@@ -374,7 +418,7 @@ struct RowCgBack : Row<R, MEM> {
     const double z = this->solve(h - s[0], e);
     if (!writes) return;
     double* now = this->zw(this->k.par, slot) + e;
-    double* old = this->zw(this->k.par ^ 1, slot) + e;
+    double* old = this->zw(this->k.last_copy(), slot) + e;
     this->put_zw(now, unmarked(z));
     this->put_zw(old, mark());
     this->put_zw(old + 3, mark());
@@ -419,7 +463,7 @@ struct RowCgFwd : Row<R, MEM> {
     const double t = (refresh ? h : az) - s[1];
     const double w = this->solve(t, e);
     if (!writes) return;
-    this->put_zw(this->zw(this->k.par ^ (refresh ? 1 : 0), slot) + 3 + e, unmarked(w));
+    this->put_zw(this->zw(refresh ? this->k.next_copy() : this->k.par, slot) + 3 + e, unmarked(w));
     if (refresh) {
       this->put(kH, t);
     } else {
@@ -518,7 +562,8 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
     uint64_t t0 = wall_clock64();
     {
       RowCgFwd<Res, MEM> f(k, iter > 1 ? rho / rho1 : 0.0, iter == 1, refresh);
-      k.template sweep<2>(0, k.par ^ (refresh ? 1 : 0), f);
+      if (refresh) k.enter(k.next_copy());
+      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f);
       double tot[1];
       k.reduce(f.acc, tot);
       if (!refresh) c1 = tot[0];
@@ -545,11 +590,13 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
     }
     double rho_next = 0.0;
     if (!ended) {
-      k.par ^= 1;
+      k.par = k.next_copy();
+      k.enter(k.par);
       RowCgBack<Res, MEM> f(k, alpha, upd);
       k.template sweep<1>(1, k.par, f);
       double tot[2];
       k.reduce(f.acc, tot);
+      if (!upd) k.drop_lines();  // the refresh wrote, and this sweep marked, the same copy's w
       if (upd) dnrm2 = tot[0];
       rho_next = tot[1];
       ticks[1] += wall_clock64() - t1;
@@ -621,7 +668,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
   }
   if (MEM == kOneGroup) {
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < 2 * k.copy_size; i += T) o.zw[i] = k.zw0[i];
+    for (int64_t i = threadIdx.x; i < o.ring * k.copy_size; i += T) o.zw[i] = k.zw0[i];
   }
 }
 
@@ -651,7 +698,7 @@ struct RowBiBack : Row<R, MEM> {
     }
     if (half) {
       x = this->get(kX);
-      pt = ld<MEM>(this->zw(this->k.par ^ 1, slot) + e);
+      pt = ld<MEM>(this->zw(this->k.last_copy(), slot) + e);
     } else if (!first) {
       p = this->get(kBp);
       hp = this->get(kHp);
@@ -669,7 +716,7 @@ struct RowBiBack : Row<R, MEM> {
     const double z = this->solve((half ? hr : hp) - s[0], e);
     if (!writes) return;
     double* now = this->zw(this->k.par, slot) + e;
-    double* old = this->zw(this->k.par ^ 1, slot) + e;
+    double* old = this->zw(this->k.last_copy(), slot) + e;
     this->put_zw(now, unmarked(z));
     this->put_zw(old, mark());
     this->put_zw(old + 3, mark());
@@ -708,7 +755,7 @@ struct RowBiFwd : Row<R, MEM> {
     const double t = (refresh ? h : az) - s[1];
     const double w = this->solve(t, e);
     if (!writes) return;
-    this->put_zw(this->zw(this->k.par ^ (refresh ? 1 : 0), slot) + 3 + e, unmarked(w));
+    this->put_zw(this->zw(refresh ? this->k.next_copy() : this->k.par, slot) + 3 + e, unmarked(w));
     if (refresh) {
       this->put(kHr, t);
     } else {
@@ -780,11 +827,13 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
     // p^ or s^, unless hr is made first
     if (!refresh) {
       const uint64_t t0 = wall_clock64();
-      k.par ^= 1;
+      k.par = k.next_copy();
+      k.enter(k.par);
       const double beta = iter > 1 ? (rho / rho1) * (alpha / omega) : 0.0;
       RowBiBack<Res, MEM> f(k, half, iter == 1, after_refresh, alpha, beta, omega);
       k.template sweep<1>(1, k.par, f);
       k.grid_sync();
+      if (after_refresh) k.drop_lines();  // the refresh wrote, and this sweep marked, the same copy's w
       after_refresh = false;
       ticks[1] += wall_clock64() - t0;
     }
@@ -792,7 +841,8 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
     {
       const uint64_t t0 = wall_clock64();
       RowBiFwd<Res, MEM> f(k, half, refresh);
-      k.template sweep<2>(0, k.par ^ (refresh ? 1 : 0), f);
+      if (refresh) k.enter(k.next_copy());
+      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f);
       k.reduce(f.acc, tot);
       ticks[refresh ? 1 : 0] += wall_clock64() - t0;
     }
@@ -875,7 +925,7 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
   }
   if (MEM == kOneGroup) {
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < 2 * k.copy_size; i += T) o.zw[i] = k.zw0[i];
+    for (int64_t i = threadIdx.x; i < o.ring * k.copy_size; i += T) o.zw[i] = k.zw0[i];
   }
 }
 
@@ -924,7 +974,7 @@ __global__ __launch_bounds__(kBlock) void k_resident_init(ResidentOp o, const do
   const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x, stride = (int64_t)gridDim.x * kBlock;
   // all entries marked, except the last record, which the unused blocks gather
   const int64_t nz = ((int64_t)o.ns + 1) * zw_rec;
-  for (int64_t t = i0; t < 2 * nz; t += stride) o.zw[t] = t % nz < (int64_t)o.ns * zw_rec ? mark() : 0.0;
+  for (int64_t t = i0; t < o.ring * nz; t += stride) o.zw[t] = t % nz < (int64_t)o.ns * zw_rec ? mark() : 0.0;
   for (int64_t t = i0; t < o.ns; t += stride) {
     const int32_t i = o.row_old[t];
     double* b = rec(o, (int)t);
