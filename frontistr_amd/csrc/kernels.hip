@@ -395,7 +395,7 @@ enum SpmvEpi : int {
   kEpiStoreTrue = 6,  // y = A x, only in residual-recompute iterations (MPC: A T x of a true residual)
 };
 
-template <int EPI>
+template <int EPI, bool NT>
 __global__ __launch_bounds__(kBlock) void k_spmv(Sell<double> a, const double* __restrict__ x,
                                                    const double* __restrict__ bw, double* __restrict__ y,
                                                    const KrylovState* st, double* part) {
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(Sell<double> a, const double* _
   for (int k = 0; k < K; ++k) acc[k] = 0.0;
   for (int s = sr.begin; s < sr.end; ++s) {
     double yv[3], xo[3];
-    sell_row<kSpmvChunk>(a, s, lane, x, yv, xo);
+    sell_row<kSpmvChunk, NT>(a, s, lane, x, yv, xo);
     const int64_t row = (int64_t)s * kRowsA + lane;
     if (row < a.nrows) {
       double o[3];
@@ -1226,7 +1226,13 @@ __global__ __launch_bounds__(kBlock) void k_stream_read(const double2* __restric
 template <int EPI>
 static void spmv_launch(int g, hipStream_t s, const Sell<double>& a, const double* x, const double* bw, double* y,
                         const KrylovState* st, double* part) {
-  k_spmv<EPI><<<g, kBlock, 0, s>>>(a, x, bw, y, st, part);
+  // A matrix beyond the 256 MB memory-side cache comes from HBM every time: its loads then leave
+  // the caches to x (us: 60^3 87.5 -> 78.5, 72^3 144 -> 133 = 5.9 TB/s, 100^3 382 -> 359; 52^3,
+  // 310 MB, 54.8 -> 54.4).  Smaller ones stay there between products (44^3 29.6).
+  if (a.nslots * 76 > (int64_t)256 << 20)
+    k_spmv<EPI, true><<<g, kBlock, 0, s>>>(a, x, bw, y, st, part);
+  else
+    k_spmv<EPI, false><<<g, kBlock, 0, s>>>(a, x, bw, y, st, part);
 }
 
 // y = A x (or T^T A T x with MPC) with the epilogue EPI; returns the number of

@@ -94,19 +94,6 @@ struct LdsMap {
   }
 };
 
-// aval_load past the caches' replacement
-__device__ __forceinline__ void aval_load_nt(const double* __restrict__ val, int64_t g, int r, double (&v)[9]) {
-  typedef double D2 __attribute__((ext_vector_type(2)));
-  const double* __restrict__ b = val + g * (9 * kRowsA);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const D2 t = __builtin_nontemporal_load(reinterpret_cast<const D2*>(b + q * (2 * kRowsA) + 2 * r));
-    v[2 * q] = t.x;
-    v[2 * q + 1] = t.y;
-  }
-  v[8] = __builtin_nontemporal_load(b + 8 * kRowsA + r);
-}
-
 template <int T, int K, int MEM>
 struct Resident : GridGroup<T, MEM> {
   using Map = LdsMap<T>;

@@ -25,6 +25,18 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
+// aval_load past the caches' replacement
+__device__ __forceinline__ void aval_load_nt(const double* __restrict__ val, int64_t g, int r, double (&v)[9]) {
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  const double* __restrict__ b = val + g * (9 * kRowsA);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const D2 t = __builtin_nontemporal_load(reinterpret_cast<const D2*>(b + q * (2 * kRowsA) + 2 * r));
+    v[2 * q] = t.x;
+    v[2 * q + 1] = t.y;
+  }
+  v[8] = __builtin_nontemporal_load(b + 8 * kRowsA + r);
+}
 
 constexpr int kSpmvChunk = 4;
 
@@ -41,7 +53,7 @@ constexpr int kSpmvChunk = 4;
 // a branch of their own, one more dependent round trip per chunk).  Not FULL
 // (the row's last chunk): slots past the end re-read the last block and are
 // masked out of the sum.
-template <int U, bool FULL>
+template <int U, bool FULL, bool NT>
 __device__ __forceinline__ void sell_chunk(const Sell<double>& a, int base, int lane, const int32_t* __restrict__ colp,
                                            const double* __restrict__ x, int k0, int len, double (&y)[3],
                                            double (&xo)[3]) {
@@ -50,12 +62,15 @@ __device__ __forceinline__ void sell_chunk(const Sell<double>& a, int base, int 
 #pragma unroll
   for (int j = 0; j < U; ++j) {
     kk[j] = (FULL || k0 + j < len) ? k0 + j : len - 1;
-    c[j] = colp[(int64_t)kk[j] * kRowsA];
+    c[j] = NT ? __builtin_nontemporal_load(colp + (int64_t)kk[j] * kRowsA) : colp[(int64_t)kk[j] * kRowsA];
   }
   double v[U][9], xv[U][3];
 #pragma unroll
   for (int j = 0; j < U; ++j) {
-    aval_load(a.val, (int64_t)base + kk[j], lane, v[j]);
+    if (NT)
+      aval_load_nt(a.val, (int64_t)base + kk[j], lane, v[j]);
+    else
+      aval_load(a.val, (int64_t)base + kk[j], lane, v[j]);
     xv[j][0] = x[3 * (int64_t)c[j]];
     xv[j][1] = x[3 * (int64_t)c[j] + 1];
     xv[j][2] = x[3 * (int64_t)c[j] + 2];
@@ -83,7 +98,7 @@ __device__ __forceinline__ void sell_chunk(const Sell<double>& a, int base, int 
   }
 }
 
-template <int U>
+template <int U, bool NT = false>
 __device__ __forceinline__ void sell_row(const Sell<double>& a, int s, int lane, const double* __restrict__ x,
                                          double (&y)[3], double (&xo)[3]) {
 #pragma clang fp contract(off)
@@ -95,8 +110,8 @@ __device__ __forceinline__ void sell_row(const Sell<double>& a, int s, int lane,
   y[0] = y[1] = y[2] = -0.0;
   const int32_t* __restrict__ colp = a.col + (int64_t)base * kRowsA + lane;
   int k0 = 0;
-  for (; k0 + U <= len; k0 += U) sell_chunk<U, true>(a, base, lane, colp, x, k0, len, y, xo);
-  if (k0 < len) sell_chunk<U, false>(a, base, lane, colp, x, k0, len, y, xo);
+  for (; k0 + U <= len; k0 += U) sell_chunk<U, true, NT>(a, base, lane, colp, x, k0, len, y, xo);
+  if (k0 < len) sell_chunk<U, false, NT>(a, base, lane, colp, x, k0, len, y, xo);
 }
 
 // LU solve with the factors of hecmw_precond_SSOR_33.F90:183-195 (inverted
