@@ -1430,9 +1430,10 @@ static int32_t resident_tasks(Context& c, const ResidentShape& sh) {
 //    more workgroups add bandwidth (30^3, 195 tasks: 128 and 256 workgroups 71.6
 //    and 66.6 us; 72^3, 641 and 379 us), below that only barrier time (14^3, 21
 //    tasks: 61-65 us from 32 to 256; 10^3, 8 tasks: 60 us with 32).
-//  * One workgroup, its gathered vectors in LDS, up to 1000 nodes where they fit
-//    (6^3 cube, 343 nodes: 47 us against 53 with 32 workgroups; TET10 box, 315
-//    nodes: 55 against 65; 10^3, 1331 nodes: equal).
+//  * One workgroup, its gathered vectors in LDS, up to 450 nodes where they fit (us per
+//    iteration with 1 and with 32 workgroups: 125 nodes 43 and 48, 343 nodes 47 and 51,
+//    512 nodes 61 and 58, 729 nodes 73 and 55, 1000 nodes 103 and 65; TET10 box, 315
+//    nodes: 55 and 65).
 static ResidentShape resident_shape(const Context& c) {
   ResidentShape sh;
   int32_t longest = 0;
@@ -1446,7 +1447,7 @@ static ResidentShape resident_shape(const Context& c) {
   if (longest > 2 * kWave) sh.packets = 4;
   const int64_t tasks = lanes / (2 * (int64_t)c.ncolor * kWave);
   sh.grid = tasks < 16 ? 32 : tasks < 64 ? 128 : 256;
-  if (c.N <= 1000 && resident_one_group(c.ncolor, (int)c.ssor_rows)) sh.grid = 1;
+  if (c.N <= 450 && resident_one_group(c.ncolor, (int)c.ssor_rows)) sh.grid = 1;
   sh.grid = std::min(sh.grid, std::min(c.res_cus, kResidentGridMax));
   return sh;
 }

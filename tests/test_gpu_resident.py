@@ -52,14 +52,16 @@ def _device_solve(m, x0=None):
 # name: system, workgroups that the rule picks
 SYSTEMS = {
     "one_element": (lambda: fa.gen_hex8(1), 1),                     # a row per colour
-    "one_group": (lambda: fa.gen_hex8(7, kind="lognormal", seed=2), 1),
+    "one_group": (lambda: fa.gen_hex8(6, kind="lognormal", seed=2), 1),
+    "just_past_one_group": (lambda: fa.gen_hex8(7, kind="lognormal", seed=2), 32),
     "past_one_group": (lambda: fa.gen_hex8(10), 32),
     "tet10_small": (lambda: fa.gen_tet10(3, 2, 4, seed=1)[0], 1),
     "grid_128": (lambda: fa.gen_hex8(15, kind="lognormal", seed=2), 128),
     "grid_256": (lambda: fa.gen_hex8(25), 256),
     "long_rows": (lambda: random_system(900, deg=150, seed=3), None),    # more than 128 blocks in a row
-    "odd_rows": (lambda: random_system(777, deg=9, seed=5), 1),
-    "two_parts": (lambda: random_system(500, deg=6, seed=6, components=2), 1),
+    "odd_rows": (lambda: random_system(777, deg=9, seed=5), 32),
+    "odd_rows_one_group": (lambda: random_system(433, deg=9, seed=5), 1),
+    "two_parts": (lambda: random_system(500, deg=6, seed=6, components=2), 32),
 }
 
 
