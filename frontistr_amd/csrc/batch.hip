@@ -856,6 +856,7 @@ struct hecmw33_batch {
   // live-tile work queues and the persistent grids that walk them
   BMem qtile, qn;
   int ncu = 0;
+  int tile_rows = 0;  // rows per tile
   int grid_p = 0, grid_q = 0, grid_upd = 0, grid_res = 0, grid_diag = 0;
   int tune_cached = 0;  // 1: the SpMM shapes came from the autotuner's persisted winners
 
@@ -931,9 +932,9 @@ static void batch_enqueue_iteration(hecmw33_batch& B) {
 }
 
 // ---- the autotuner's winners, persisted per (blocks per row, rows) bucket ------------------
-// Key: the device (architecture and CU count), the mean blocks per row rounded, and floor(log2(rows)).
+// Key: the device (architecture and CU count), the rows per tile, the mean blocks per row rounded, and floor(log2(rows)).
 // Value: the names of the FP32 and FP64 SpMM shapes that won on a batch of that bucket.  Kept in a
-// text file, one "<arch> <cus> <blocks/row> <log2 rows> <fp32 shape> <fp64 shape>" line per bucket,
+// text file, one "<arch>-t<rows per tile> <cus> <blocks/row> <log2 rows> <fp32 shape> <fp64 shape>" line per bucket,
 // and in this process for that file: $HECMW33_TUNE_CACHE names the file ("off": nothing is kept and
 // every load times the shapes), else $XDG_CACHE_HOME/hecmw33/batch_tune.txt, else
 // $HOME/.cache/hecmw33/batch_tune.txt.  A line whose shape names this library does not have is
@@ -1013,6 +1014,9 @@ static TuneKey tune_key(const hecmw33_batch& B) {
     const size_t c = arch.find(':');
     if (c != std::string::npos) arch = arch.substr(0, c);
   }
+  // the shapes' order depends on the rows per tile: winners found on other tiles (and
+  // lines from before tiles had several sizes) are kept in the file, but not taken
+  arch += "-t" + std::to_string(B.tile_rows);
   const int bpr = (int)std::lround((double)B.nnzb / (double)std::max<int64_t>(1, B.nrows));
   int lrows = 0;
   while ((int64_t(2) << lrows) <= B.nrows) ++lrows;
@@ -1242,6 +1246,7 @@ static int32_t batch_load(hecmw33_batch& B, int32_t nsys, const hecmw33_sys* sys
     s_nt[s] = (int32_t)t_row0.size() - s_t0[s];
   }
   B.ntiles = (int32_t)t_row0.size();
+  B.tile_rows = tr;
   // device buffers
   const int64_t nv = B.nrows * KS * 3;
   if (B.rowptr.ensure(sizeof(int32_t) * rp.size()) || B.col.ensure(sizeof(int32_t) * nnz) ||

@@ -266,7 +266,7 @@ struct Context {
   bool ssor_round_valid = false;  // L.val32 / U.val32 hold the current values
   bool flow_sym = false, flow_valid[2] = {false, false};
   std::vector<int32_t> h_flow_group[2];  // first group of blocks of every slice
-  DMem flow_group[2], flow_col[2], flow_val[2][2], flow_rec;
+  DMem flow_group[2], flow_mem, flow_val[2];  // groups; columns, records and counter; values in FP32 and in BF16
   // DIAG
   bool diag_init = false;
   DMem row_diag, alu_diag;
@@ -349,11 +349,15 @@ struct Context {
     return SsorOp<double>{L.view,  U.view, row_old.as<int32_t>(), alu_ssor.as<double>(), color_slice.data(), ncolor,
                           vzs.as<double>(), node_slot.as<int32_t>(), N, ssor_last_bwd_empty};
   }
+  // bytes of the packed values of direction d
+  size_t flow_val_bytes(int d, bool v16) const {
+    return (size_t)std::max(h_flow_group[d].back(), 1) * 48 * 16 * (v16 ? 3 : 6);
+  }
   SsorOp<float> ssor_op32(bool v16) {
     SsorOp<float> op{L.view32, U.view32, row_old.as<int32_t>(), alu_ssor32.as<float>(), color_slice.data(),
                      ncolor, vzs32.as<float>(), node_slot.as<int32_t>(), N, ssor_last_bwd_empty};
     if (flow_use) {
-      for (int d = 0; d < 2; ++d) flow.val[d] = flow_val[v16 ? 1 : 0][d].p;
+      for (int d = 0; d < 2; ++d) flow.val[d] = flow_val[v16 ? 1 : 0].as<char>() + d * flow_val_bytes(0, v16);
       flow.b16 = v16;
       op.flow = &flow;
     } else if (v16) {
@@ -371,9 +375,7 @@ struct Context {
     for (DMem* m : {&cg_agg, &cg_aptr, &cg_anodes, &cg_dv, &cg_pa, &cg_pb, &cg_pnptr, &cg_pn, &cg_Eblk, &cg_E, &cg_W,
                     &cg_cv, &cg_tv, &cg_yv, &cg_info, &cg_Linv, &cg_T, &cg_ncnt, &cg_nagg, &cg_AZ, &cg_sc, &cg_aggW, &cg_kept, &vr1_32, &vt32, &vw32, &vaz32})
       m->release();
-    for (DMem* m : {&flow_group[0], &flow_group[1], &flow_col[0], &flow_col[1], &flow_val[0][0], &flow_val[0][1], &flow_val[1][0],
-                    &flow_val[1][1], &flow_rec})
-      m->release();
+    for (DMem* m : {&flow_group[0], &flow_group[1], &flow_mem, &flow_val[0], &flow_val[1]}) m->release();
     for (DMem* m : {&dres_task, &dres_lane, &dres_row, &dres_z}) m->release();
     for (DMem* m : {&res_color_task, &res_task, &res_row, &res_col, &res_val, &res_vec, &res_sync, &res_dsig})
       m->release();
@@ -709,6 +711,8 @@ static int32_t setup_ssor_symbolic(Context& c, int32_t ncolor_in) {
     std::vector<int32_t>& group = c.h_flow_group[d];
     group.assign(ptr.size(), 0);
     for (size_t s = 0; s + 1 < ptr.size(); ++s) group[s + 1] = group[s] + (ptr[s + 1] - ptr[s] + kFlowBlocks - 1) / kFlowBlocks;
+    if (c.flow_group[d].ensure(sizeof(int32_t) * group.size())) return HECMW33_ERROR_DEVICE;
+    HIPC(hipMemcpyAsync(c.flow_group[d].p, group.data(), sizeof(int32_t) * group.size(), hipMemcpyHostToDevice, c.stream));
   }
   c.h_lenL = std::move(hl.len);
   c.h_lenU = std::move(hu.len);
@@ -796,33 +800,31 @@ static int32_t flow_setup(Context& c, bool v16) {
   if (c.ssor_R != kRowsS || !c.ssor_proper || c.ssor_rows < 1) return 1;
   const int32_t ns = (int32_t)c.ssor_rows, S = ns / kRowsS;
   auto no_memory = [&] {
-    for (DMem* m : {&c.flow_group[0], &c.flow_group[1], &c.flow_col[0], &c.flow_col[1], &c.flow_val[0][0], &c.flow_val[0][1],
-                    &c.flow_val[1][0], &c.flow_val[1][1], &c.flow_rec})
-      m->release();
+    for (DMem* m : {&c.flow_mem, &c.flow_val[0], &c.flow_val[1]}) m->release();
     (void)hipGetLastError();
     c.flow_sym = c.flow_valid[0] = c.flow_valid[1] = false;
     return 1;
   };
   FlowOp& o = c.flow;
   const bool sym = !c.flow_sym;
-  auto ngroup = [&](int d) { return (size_t)std::max(c.h_flow_group[d][S], 1); };
-  for (int d = 0; sym && d < 2; ++d) {
-    const std::vector<int32_t>& group = c.h_flow_group[d];
-    if (c.flow_group[d].ensure(sizeof(int32_t) * group.size()) || c.flow_col[d].ensure(sizeof(int2) * kWave * ngroup(d)) ||
-        c.flow_rec.ensure(sizeof(float4) * 3 * (size_t)ns + 256))
-      return no_memory();
-    HIPC(hipMemcpyAsync(c.flow_group[d].p, group.data(), sizeof(int32_t) * group.size(), hipMemcpyHostToDevice, c.stream));
-  }
   if (sym) {
+    // one allocation: records and r (16 bytes each), columns, counter
+    const size_t rec = sizeof(float4) * 3 * (size_t)ns;
+    size_t col[2];
+    for (int d = 0; d < 2; ++d) col[d] = sizeof(int2) * kWave * (size_t)std::max(c.h_flow_group[d][S], 1);
+    if (c.flow_mem.ensure(rec + col[0] + col[1] + sizeof(uint32_t))) return no_memory();
+    char* p = c.flow_mem.as<char>();
+    o.rec = p;
+    o.rhs = reinterpret_cast<float4*>(p) + 2 * (size_t)ns;
+    p += rec;
     for (int d = 0; d < 2; ++d) {
+      o.col[d] = reinterpret_cast<int2*>(p);
+      p += col[d];
       o.group[d] = c.flow_group[d].as<int32_t>();
       o.len[d] = (d ? c.U : c.L).view.len;
-      o.col[d] = c.flow_col[d].as<int2>();
     }
+    o.ticket = reinterpret_cast<uint32_t*>(p);
     o.row_old = c.row_old.as<int32_t>();
-    o.rec = c.flow_rec.p;
-    o.rhs = c.flow_rec.as<float4>() + 2 * (size_t)ns;
-    o.ticket = reinterpret_cast<uint32_t*>(o.rhs + ns);
     o.ns = ns;
     // four times the workgroups that a colour's slices occupy, so that the slices of the next
     // colours are loaded in time (30^3 cube, us: 161 with as many, 101 with twice, 92 with
@@ -832,11 +834,11 @@ static int32_t flow_setup(Context& c, bool v16) {
     const int32_t per = S / std::max(c.ncolor, 1) / 8 + 1;
     o.grid = per > 160 ? 512 : std::min(4 * per, 256);
   }
-  for (int d = 0; d < 2; ++d) {
-    DMem& v = c.flow_val[v16 ? 1 : 0][d];
-    if (v.ensure(ngroup(d) * 48 * 16 * (v16 ? 3 : 6))) return no_memory();
-    flow_pack((d ? c.U : c.L).view, o.group[d], d == 1, v16, v.p, sym ? c.flow_col[d].as<int2>() : nullptr, c.stream);
-  }
+  DMem& v = c.flow_val[v16 ? 1 : 0];
+  if (v.ensure(c.flow_val_bytes(0, v16) + c.flow_val_bytes(1, v16))) return no_memory();
+  for (int d = 0; d < 2; ++d)
+    flow_pack((d ? c.U : c.L).view, o.group[d], d == 1, v16, v.as<char>() + d * c.flow_val_bytes(0, v16),
+              sym ? const_cast<int2*>(o.col[d]) : nullptr, c.stream);
   o.alu = c.alu_ssor32.as<float>();
   HIPC(hipGetLastError());
   c.flow_sym = true;
@@ -855,10 +857,7 @@ static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
     c.ssor16_valid = false;
     c.ssor_round_valid = c.flow_valid[0] = c.flow_valid[1] = false;
     const int64_t nslot = c.ssor_rows;
-    if (c.alu_ssor32.ensure(sizeof(float) * 9 * std::max<int64_t>(nslot, 1)) ||
-        c.vzs32.ensure(sizeof(float) * 3 * std::max<int64_t>(nslot, 1)))
-      return HECMW33_ERROR_DEVICE;
-    HIPC(hipMemsetAsync(c.vzs32.p, 0, sizeof(float) * 3 * std::max<int64_t>(nslot, 1), c.stream));
+    if (c.alu_ssor32.ensure(sizeof(float) * 9 * std::max<int64_t>(nslot, 1))) return HECMW33_ERROR_DEVICE;
     launch_to_f32(9 * nslot, c.alu_ssor.as<double>(), c.alu_ssor32.as<float>(), c.stream);
     c.ssor32_valid = true;
   }
@@ -868,7 +867,9 @@ static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
     c.flow_use = e == 0;
   }
   if (kind == 1 && !c.flow_use && !c.ssor_round_valid) {
-    if (round_sell(c.L, c.stream) || round_sell(c.U, c.stream)) return HECMW33_ERROR_DEVICE;
+    const size_t zs = sizeof(float) * 3 * (size_t)std::max<int64_t>(c.ssor_rows, 1);
+    if (c.vzs32.ensure(zs) || round_sell(c.L, c.stream) || round_sell(c.U, c.stream)) return HECMW33_ERROR_DEVICE;
+    HIPC(hipMemsetAsync(c.vzs32.p, 0, zs, c.stream));
     c.ssor_round_valid = true;
   }
   if (kind == 1 && v16 && !c.flow_use && !c.ssor16_valid) {

@@ -72,3 +72,22 @@ def test_instances_that_stop_at_different_times():
             assert info["error"] == 0 and it[s, k] <= 1.3 * info["iter"] + 10
             assert np.linalg.norm(X[k] - xr) <= 1e-6 * np.linalg.norm(xr)
     bs.close()
+
+
+def test_tuned_shapes_belong_to_their_tiles(tmp_path, monkeypatch):
+    """A saved winner from other tiles (here a line without any) stays in the file but is not
+    taken; the winner that the load finds is, by the next one."""
+    import torch
+    path = tmp_path / "tune.txt"
+    monkeypatch.setenv("HECMW33_TUNE_CACHE", str(path))
+    m = fa.gen_hex8(6)
+    B = np.random.default_rng(1).standard_normal((1, 3 * m.N))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    old = "gfx950 %d %d %d lpr64_rpl1_u1 lpr16_rpl1_u1" % (cus, round((m.N + m.NPL + m.NPU) / m.N), int(np.log2(m.N)))
+    path.write_text(old + "\n")
+    for cached in (False, True):
+        bs = fa.BatchSolver([m], [B])
+        assert bs.info()["tune_cached"] == cached
+        bs.close()
+    lines = path.read_text().strip().splitlines()
+    assert old in lines and len(lines) == 2 and any(l.startswith("gfx950-t16 ") for l in lines)
