@@ -43,11 +43,21 @@ __device__ __forceinline__ double cwave_sum(double v) {
   return v;
 }
 
-// Fixed-order sum of K values over the workgroup; thread k < K gets total k.
-template <int K>
+// Fixed-order sum of K values over a workgroup of T threads; thread k < K writes total k.
+template <int K, int T = kCoarseBlock>
 __device__ __forceinline__ void block_reduce(double (&v)[K], double* out) {
-  __shared__ double red[K][kCoarseWaves];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  if constexpr (T == kWave) {
+    double own = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double w = cwave_sum(v[k]);
+      if (lane == k) own = w;
+    }
+    if (lane < K) out[lane] = own;
+    return;
+  }
+  __shared__ double red[K][kCoarseWaves];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const double w = cwave_sum(v[k]);
@@ -65,9 +75,11 @@ __device__ __forceinline__ void block_reduce(double (&v)[K], double* out) {
 // E block of the aggregate pair p = (a, b):
 //   E_ab = sum over the nodes i of a that touch b, blocks j of row i with
 //   agg(j) = b, of Z_i^T A_ij Z_j.
-// One workgroup per pair; each thread sums its nodes' blocks in registers, then
-// a fixed-order reduction, so E is the same on every run.
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_E(Sell<double> A, const int32_t* __restrict__ agg,
+// One workgroup of T threads per pair, SUB threads per node (each takes every SUB-th
+// block of the row); they sum their blocks in registers, then a fixed-order
+// reduction, so E is the same on every run.  See coarse_assemble for T and SUB.
+template <int T, int SUB>
+__global__ __launch_bounds__(T) void k_coarse_E(Sell<double> A, const int32_t* __restrict__ agg,
                                                             const int32_t* __restrict__ pb,
                                                             const int32_t* __restrict__ pn_ptr,
                                                             const int32_t* __restrict__ pn,
@@ -78,13 +90,13 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E(Sell<double> A, const
 #pragma unroll
   for (int k = 0; k < 36; ++k) acc[k] = 0.0;
   const int t1 = pn_ptr[p + 1];
-  for (int t = pn_ptr[p] + threadIdx.x; t < t1; t += kCoarseBlock) {
+  for (int t = pn_ptr[p] + threadIdx.x / SUB; t < t1; t += T / SUB) {
     const int i = pn[t];
     const double ix = dv[3 * (int64_t)i], iy = dv[3 * (int64_t)i + 1], iz = dv[3 * (int64_t)i + 2];
     const int sl = i / A.rows, l = i % A.rows;
     const int64_t base = (int64_t)A.ptr[sl] * A.rows;
     const int len = A.len[i];
-    for (int k = 0; k < len; ++k) {
+    for (int k = threadIdx.x % SUB; k < len; k += SUB) {
       const int64_t slot = base + (int64_t)k * A.rows + l;
       const int j = A.col[slot];
       if (agg[j] != b) continue;
@@ -113,7 +125,7 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E(Sell<double> A, const
       }
     }
   }
-  block_reduce<36>(acc, Eblk + (int64_t)p * 36);
+  block_reduce<36, T>(acc, Eblk + (int64_t)p * 36);
 }
 
 // E(6a+r, 6b+q) = Eblk[p][r][q], the blocks on and below the diagonal
@@ -549,7 +561,8 @@ __device__ __forceinline__ void zblock(const float* __restrict__ dv, const float
 }
 
 // tile (tr, tc) = blockIdx.y of E_ab: rows 6 tr.., columns 6 tc.. of Z_a^T A Z_b
-__global__ __launch_bounds__(kCoarseBlock) void k_coarse_E12(Sell<double> A, const int32_t* __restrict__ agg,
+template <int T, int SUB>
+__global__ __launch_bounds__(T) void k_coarse_E12(Sell<double> A, const int32_t* __restrict__ agg,
                                                               const int32_t* __restrict__ pb,
                                                               const int32_t* __restrict__ pn_ptr,
                                                               const int32_t* __restrict__ pn,
@@ -561,14 +574,14 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E12(Sell<double> A, con
 #pragma unroll
   for (int k = 0; k < 36; ++k) acc[k] = 0.0;
   const int t1 = pn_ptr[p + 1];
-  for (int t = pn_ptr[p] + threadIdx.x; t < t1; t += kCoarseBlock) {
+  for (int t = pn_ptr[p] + threadIdx.x / SUB; t < t1; t += T / SUB) {
     const int i = pn[t];
     double zi[3][6];
     zblock(dv, xm, i, tr, zi);
     const int sl = i / A.rows, l = i % A.rows;
     const int64_t base = (int64_t)A.ptr[sl] * A.rows;
     const int len = A.len[i];
-    for (int k = 0; k < len; ++k) {
+    for (int k = threadIdx.x % SUB; k < len; k += SUB) {
       const int j = A.col[base + (int64_t)k * A.rows + l];
       if (agg[j] != b) continue;
       double v[9], zj[3][6];
@@ -585,7 +598,7 @@ __global__ __launch_bounds__(kCoarseBlock) void k_coarse_E12(Sell<double> A, con
         }
     }
   }
-  block_reduce<36>(acc, Eblk + ((int64_t)p * 4 + blockIdx.y) * 36);
+  block_reduce<36, T>(acc, Eblk + ((int64_t)p * 4 + blockIdx.y) * 36);
 }
 
 // E(12a + 6tr + r, 12b + 6tc + q) = tile (tr, tc) of pair p
@@ -850,14 +863,27 @@ int coarse_fcg_pq(int64_t n3, const float* z, const float* az, float* p, float* 
 }
 
 void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, const int32_t* pa, const int32_t* pb,
-                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, const CoarseBand& e, hipStream_t s) {
+                     const int32_t* pn_ptr, const int32_t* pn, int64_t npn, double* Eblk, const CoarseBand& e,
+                     hipStream_t s) {
   if (npair <= 0) return;
+  // Up to 64 nodes per pair one wave with eight lanes per node: with a thread per node most
+  // of 256 stay idle and the others walk their row alone.  E (six modes) / E12 in us, 21,952
+  // pairs, one wave against 256 threads: 30^3 (5 nodes per pair) 137 and 648 / 565 and 3621, 48^3
+  // (14) 244 and 738 / 968 and 3999, 64^3 (27) 507 and 855 / 1899 and 4640, 100^3 (85) 1704 and
+  // 1413 / 6216 and 7753, 130^3 (163) 3636 and 2362 / 12,772 and 11,916.
+  const bool few = npn <= 64 * (int64_t)npair;
   if (op.nm == 12) {
-    k_coarse_E12<<<dim3((unsigned)npair, 4), kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, op.xm, Eblk);
+    if (few)
+      k_coarse_E12<kWave, 8><<<dim3((unsigned)npair, 4), kWave, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, op.xm, Eblk);
+    else
+      k_coarse_E12<kCoarseBlock, 1><<<dim3((unsigned)npair, 4), kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, op.xm, Eblk);
     const int64_t ne = (int64_t)npair * 144;
     k_coarse_scatter12<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, e.E, e.w);
   } else {
-    k_coarse_E<<<(unsigned)npair, kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, Eblk);
+    if (few)
+      k_coarse_E<kWave, 8><<<(unsigned)npair, kWave, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, Eblk);
+    else
+      k_coarse_E<kCoarseBlock, 1><<<(unsigned)npair, kCoarseBlock, 0, s>>>(A, op.agg, pb, pn_ptr, pn, op.dv, Eblk);
     const int64_t ne = (int64_t)npair * 36;
     k_coarse_scatter<<<(unsigned)((ne + 255) / 256), 256, 0, s>>>(npair, pa, pb, Eblk, e.E, e.w);
   }

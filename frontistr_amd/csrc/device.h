@@ -400,10 +400,11 @@ struct CoarseBand {
   int32_t np = 0, w = 0;
 };
 // E = Z^T A Z: the nm x nm block of every coupled aggregate pair (pa[p], pb[p]), summed
-// over the pair's nodes pn[pn_ptr[p]..pn_ptr[p+1]), then scattered into the band's blocks
+// over the pair's nodes pn[pn_ptr[p]..pn_ptr[p+1]) (npn in all), then scattered into the band's blocks
 // (Eblk: nm*nm doubles per pair)
 void coarse_assemble(const Sell<double>& A, const CoarseOp& op, int32_t npair, const int32_t* pa, const int32_t* pb,
-                     const int32_t* pn_ptr, const int32_t* pn, double* Eblk, const CoarseBand& e, hipStream_t s);
+                     const int32_t* pn_ptr, const int32_t* pn, int64_t npn, double* Eblk, const CoarseBand& e,
+                     hipStream_t s);
 // Cholesky factorization and inverse of E (chol.hip).  T receives the lower triangle of
 // L^-1 (E = L L^T) or with `both` of E^-1, in columns of 16: coarse_inverse_index.
 // Linv: 64 doubles per (padded) row; *info is set when E is not positive definite.

@@ -1275,7 +1275,7 @@ static int32_t coarse_numeric(Context& c, int32_t nm) {
   e.E = c.cg_E.as<double>();
   HIPC(hipMemsetAsync(c.cg_info.p, 0, sizeof(int32_t), c.stream));
   coarse_assemble(c.A.view, op, c.coarse_npair, c.cg_pa.as<int32_t>(), c.cg_pb.as<int32_t>(),
-                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.cg_Eblk.as<double>(), e, c.stream);
+                  c.cg_pnptr.as<int32_t>(), c.cg_pn.as<int32_t>(), c.coarse_nw, c.cg_Eblk.as<double>(), e, c.stream);
   HIPC(hipGetLastError());
   // six modes: E^-1 for one FP32 product per coarse solve; twelve: L^-1 for two FP64
   // triangular products, y = L^-T (L^-1 c), the same bytes read without forming
