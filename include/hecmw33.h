@@ -227,7 +227,7 @@ int32_t hecmw33_ctx_history(hecmw33_ctx* ctx, double* hist, int32_t cap);
  * aggregate of the last two-level solve (6, or 12 with the learned ones), [16] error samples and
  * [17] FCG iterations per sample of the last learned fit, [18] its harvest and [19] its fit time
  * (microseconds), [20] coarse unknowns (modes per aggregate x aggregates), [21] workgroups of the
- * resident kernel that ran the last solve (0: launches per colour). */
+ * resident kernel that ran the last solve (0: a launch per kernel). */
 int32_t hecmw33_ctx_info(hecmw33_ctx* ctx, int64_t* info, int32_t n);
 /* the multipoint constraints of a device context (as hecmw33_set_mpc) */
 int32_t hecmw33_ctx_set_mpc(hecmw33_ctx* ctx, int32_t N, int32_t n_mpc, const int32_t* mpc_index,
