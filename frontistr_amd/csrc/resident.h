@@ -61,9 +61,21 @@ constexpr int kAuxSc1 = 16;  // agent scope, as the cache bits of a buffer acces
 // that no computed value keeps (unmarked replaces it by the plain NaN).
 constexpr int kMarkHi = 0x7FFADEAD;
 __device__ __forceinline__ double mark() { return __hiloint2double(kMarkHi, 0); }
-__device__ __forceinline__ bool marked(double v) { return __double2hiint(v) == kMarkHi; }
+__host__ __device__ __forceinline__ bool marked(double v) { return (int)(__builtin_bit_cast(uint64_t, v) >> 32) == kMarkHi; }
 __device__ __forceinline__ double unmarked(double v) {
   return marked(v) ? __hiloint2double(0x7FF80000, 0) : v;
+}
+
+// Whether a gathered record has to be asked for again: {z} of a backward sweep, {z w} of a
+// forward one, where w is what the sweep computes.  z stands in memory by then, but the
+// record comes in several loads, and one that the caches serve may bring marks of z from a
+// line of the backward sweep beside a w that has just arrived: unless the sweep leaves z
+// aside (`with_z` false, the refresh, before there is one), every entry counts.
+template <int NG>
+__host__ __device__ __forceinline__ bool missing(const double (&x)[3 * NG], bool with_z) {
+  bool m = marked(x[3 * NG - 3]) | marked(x[3 * NG - 2]) | marked(x[3 * NG - 1]);
+  if (NG > 1 && with_z) m |= marked(x[0]) | marked(x[1]) | marked(x[2]);
+  return m;
 }
 
 template <int J>

@@ -19,8 +19,9 @@
 //    reductions between the sweeps are grid barriers.  With four copies the first
 //    look at an entry goes through the caches (a record is gathered about 13 times in
 //    a sweep, and past the caches that was half of the memory traffic at 72^3); an
-//    old line can only hold marks, which are asked for again past the caches, because
-//    the lines go once per turn of the copies.
+//    old line can only hold marks, because the lines go once per turn of the copies, and
+//    a record with a mark in any entry that the sweep uses is asked for again past the
+//    caches.
 //
 // The iteration needs the off-diagonal blocks once, not twice as SSOR
 // application + product do.  With A = L + D + U and M = (D'+L) D'^-1 (D'+U)
@@ -216,10 +217,10 @@ struct Resident : GridGroup<T, MEM> {
     if (t >= 0) load(t);
   }
 
-  // the gathered records of the task's blocks from copy `cp`, again until the
-  // entries that this sweep computes (z backward, w forward) are there
+  // the gathered records of the task's blocks from copy `cp`, again until their
+  // entries are there (see missing)
   template <int NG>
-  __device__ __forceinline__ void gather(int cp, double (&x)[K][3 * NG]) {
+  __device__ __forceinline__ void gather(int cp, bool with_z, double (&x)[K][3 * NG]) {
     bool want[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) want[k] = true;
@@ -252,7 +253,7 @@ struct Resident : GridGroup<T, MEM> {
       bool more = false;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
-        want[k] = marked(x[k][3 * NG - 3]) | marked(x[k][3 * NG - 2]) | marked(x[k][3 * NG - 1]);
+        want[k] = missing<NG>(x[k], with_z);
         more |= want[k];
       }
       if (!__any(more) || dead) break;
@@ -263,9 +264,10 @@ struct Resident : GridGroup<T, MEM> {
   // One sweep in direction d over copy `cp` of the gathered records, NG vectors
   // gathered, row work by f; `begin` has been called for it, and is called for
   // the sweep in the other direction at the end.  Row work takes four lanes
-  // per row (lane 4 r + e: entry e, the fourth mirrors the third).
+  // per row (lane 4 r + e: entry e, the fourth mirrors the third).  with_z: f uses
+  // the sums over the gathered z (a refresh has none yet).
   template <int NG, class F>
-  __device__ __forceinline__ void sweep(int d, int cp, F& f) {
+  __device__ __forceinline__ void sweep(int d, int cp, F& f, bool with_z = true) {
     const int2* r = range + d * (o.ncolor + 1);
     const int total = r[o.ncolor].y;
     const int e = (lane & 3) < 3 ? lane & 3 : 2, row = lane >> 2;
@@ -289,7 +291,7 @@ struct Resident : GridGroup<T, MEM> {
       while ((int32_t)(__hip_atomic_load(fin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - first) < 0)
         __builtin_amdgcn_s_sleep(1);
       double x[K][3 * NG];
-      gather<NG>(cp, x);
+      gather<NG>(cp, with_z, x);
 #pragma unroll
       for (int g = 0; g < NG; ++g)
 #pragma unroll
@@ -550,7 +552,7 @@ __global__ __launch_bounds__(T) void k_resident_cg(ResidentOp o, int budget) {
     {
       RowCgFwd<Res, MEM> f(k, iter > 1 ? rho / rho1 : 0.0, iter == 1, refresh);
       if (refresh) k.enter(k.next_copy());
-      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f);
+      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f, !refresh);
       double tot[1];
       k.reduce(f.acc, tot);
       if (!refresh) c1 = tot[0];
@@ -829,7 +831,7 @@ __global__ __launch_bounds__(T) void k_resident_bicg(ResidentOp o, int budget) {
       const uint64_t t0 = wall_clock64();
       RowBiFwd<Res, MEM> f(k, half, refresh);
       if (refresh) k.enter(k.next_copy());
-      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f);
+      k.template sweep<2>(0, refresh ? k.next_copy() : k.par, f, !refresh);
       k.reduce(f.acc, tot);
       ticks[refresh ? 1 : 0] += wall_clock64() - t0;
     }
