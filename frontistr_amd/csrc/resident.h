@@ -66,6 +66,14 @@ __device__ __forceinline__ double unmarked(double v) {
   return marked(v) ? __hiloint2double(0x7FF80000, 0) : v;
 }
 
+// The copy of the ring whose first gather is preceded by dropping the caches' lines, of all
+// copies.  A copy's old lines must be gone before it is gathered again, so none of them may
+// come back between the drop and the marks' return: the copy before this one gets its marks
+// right after the drop, and a BiCGSTAB sweep of s^ reads p^ in the copy that it marks.  The
+// sweeps of s^ take the even copies (the first sweep of p^ takes copy 1, a refresh takes the
+// copy of the sweep that follows it), so the line is drawn at an odd one.
+__host__ __device__ __forceinline__ bool drops_lines(int copy) { return copy == 1; }
+
 // Whether a gathered record has to be asked for again: {z} of a backward sweep, {z w} of a
 // forward one, where w is what the sweep computes.  z stands in memory by then, but the
 // record comes in several loads, and one that the caches serve may bring marks of z from a

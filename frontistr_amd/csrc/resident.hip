@@ -170,7 +170,7 @@ struct Resident : GridGroup<T, MEM> {
   }
   // once per turn of the ring, before copy cp is gathered
   __device__ __forceinline__ void enter(int cp) {
-    if (cp == 0) drop_lines();
+    if (drops_lines(cp)) drop_lines();
   }
   __device__ __forceinline__ double* zw(int cp, int slot) const { return zw0 + cp * copy_size + (int64_t)kRec * slot; }
 

@@ -19,6 +19,7 @@ extern "C" int missing1(const double* x) {
 extern "C" int missing2(const double* x, int with_z) {
   return missing<2>(*reinterpret_cast<const double(*)[6]>(x), with_z != 0);
 }
+extern "C" int drops(int copy) { return drops_lines(copy); }
 """
 
 
@@ -69,3 +70,99 @@ def test_a_record_from_lines_of_different_age_is_asked_for_again(rules, with_z):
 def test_values_that_are_not_marks_are_taken(rules):
     x = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, 5e-324])
     assert not rules.missing2(x.ctypes.data, 1) and not rules.missing1(x.ctypes.data)
+
+
+class Ring:
+    """One record of each of four copies, and what the caches may hold of it at worst: every
+    state that a load since the lines were last dropped can have seen, whatever the load's
+    scope.  The sweeps' accesses in their order (k_resident_cg, k_resident_bicg)."""
+
+    def __init__(self, rules, par):
+        self.rules, self.par, self.n = rules, par, 0
+        self.mem = [("mark", "mark")] * 4
+        self.lines = [set() for _ in range(4)]
+
+    def drop(self):
+        self.lines = [set() for _ in range(4)]
+
+    def enter(self, cp):
+        if self.rules.drops(cp):
+            self.drop()
+
+    def next(self):
+        return (self.par + 1) % 4
+
+    def load(self, cp):
+        self.lines[cp].add(self.mem[cp])
+
+    def put(self, cp, z=None, w=None):
+        z0, w0 = self.mem[cp]
+        self.mem[cp] = (z or z0, w or w0)
+
+    def look(self, cp, now, field):
+        """A gather through the caches: nothing but a mark or the present value."""
+        seen = {s[field] for s in self.lines[cp] | {self.mem[cp]}}
+        assert seen <= {"mark", now}, (cp, seen, now)
+
+    def backward(self, after_refresh=False, reads_last=False):
+        last, self.par = self.par, self.next()
+        self.enter(self.par)
+        self.n += 1
+        z = "z%d" % self.n
+        for _ in range(2):  # before and after the record is written
+            self.load(self.par)
+            self.look(self.par, z, 0)
+            if reads_last:  # another row of the line may have been marked or not
+                self.load(last)
+            self.put(self.par, z=z)
+        self.put(last, z="mark", w="mark")
+        if after_refresh:
+            self.put(self.par, w="mark")
+            self.drop()
+
+    def forward(self):
+        w = "w%d" % self.n
+        for _ in range(2):
+            self.load(self.par)
+            self.look(self.par, "z%d" % self.n, 0)
+            self.look(self.par, w, 1)
+            self.put(self.par, w=w)
+
+    def refresh(self):
+        cp = self.next()
+        self.enter(cp)
+        self.n += 1
+        u = "u%d" % self.n
+        for _ in range(2):
+            self.load(cp)
+            self.look(cp, u, 1)
+            self.put(cp, w=u)
+
+
+@pytest.mark.parametrize("par", [0, 1, 2, 3])
+@pytest.mark.parametrize("period", [3, 4, 5, 1000])
+def test_cg_looks_find_no_old_value_in_the_caches(rules, par, period):
+    r = Ring(rules, par)
+    fresh = True
+    for it in range(40):
+        if fresh:
+            r.refresh()
+        r.backward(after_refresh=fresh)
+        r.forward()
+        fresh = it % period == period - 1
+
+
+@pytest.mark.parametrize("par", [0, 2])  # as the solve starts, and as its launches end
+@pytest.mark.parametrize("period", [1, 2, 3, 1000])
+def test_bicgstab_looks_find_no_old_value_in_the_caches(rules, par, period):
+    r = Ring(rules, par)
+    fresh = True
+    for it in range(40):
+        if fresh:
+            r.refresh()
+        r.backward(after_refresh=fresh)
+        r.forward()
+        r.backward(reads_last=True)
+        r.forward()
+        r.load(r.par)  # x += omega s^
+        fresh = it % period == period - 1
