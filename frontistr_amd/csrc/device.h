@@ -262,6 +262,7 @@ void bi_update(int64_t n3, const double* pt, const double* stv, const double* t,
 // in A's paired planes (aval_index, group t K + k % K).  Blocks without an entry
 // have value 0 and column ns, a record that is always there.  The tasks of L'
 // come first, then those of U'.
+constexpr int kLdsBytes = 160 * 1024;   // LDS of a CU
 constexpr int kResidentGridMax = 256;   // workgroups (one per CU)
 constexpr int kResidentSync = 640 + 12 * kResidentGridMax;  // words: abort flag, counts, entries of the exchanges
 constexpr int kResidentPlanesCg = 27;   // of 16 slots in a row record: the LU and six vectors (CG)

@@ -86,6 +86,12 @@ __host__ __device__ __forceinline__ bool missing(const double (&x)[3 * NG], bool
   return m;
 }
 
+// The LDS that a resident kernel may ask for.  A kernel's attributes belong to the process, so
+// every launch of any context sets this one value, whatever its own size is.
+inline hipError_t allow_lds(const void* kernel) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+}
+
 template <int J>
 __device__ __forceinline__ double quad_bcast(double v) {
   constexpr int ctrl = J | (J << 2) | (J << 4) | (J << 6);

@@ -984,8 +984,7 @@ template <int T, int K, int MEM>
 hipError_t launch(const ResidentOp& o, int grid, int budget, hipStream_t s) {
   const auto f = o.planes == kBiPlanes ? k_resident_bicg<T, K, MEM> : k_resident_cg<T, K, MEM>;
   const size_t lds = LdsMap<T>::bytes(o.ncolor, MEM == kOneGroup ? o.ns : 0);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+  if (hipError_t e = allow_lds(reinterpret_cast<const void*>(f))) return e;
   k_resident_reset<<<1, 256, 0, s>>>(o.sync);
   ResidentOp op = o;
   void* args[] = {&op, &budget};
@@ -1009,7 +1008,7 @@ void resident_alu(const ResidentOp& o, const double* alu, int rows, hipStream_t 
 void resident_init(const ResidentOp& o, const ResidentShape& sh, const double* r, hipStream_t st) {
   k_resident_init<<<std::min(std::max((o.ns + kBlock - 1) / kBlock, 1), 2048), kBlock, 0, st>>>(o, r, sh.grid == 1 ? 6 : 8);
 }
-bool resident_one_group(int ncolor, int ns) { return LdsMap<512>::bytes(ncolor, ns) <= 160 * 1024; }
+bool resident_one_group(int ncolor, int ns) { return LdsMap<512>::bytes(ncolor, ns) <= kLdsBytes; }
 
 hipError_t resident_run(const ResidentOp& o, const ResidentShape& sh, int budget, hipStream_t s) {
   if (sh.grid == 1) {

@@ -377,8 +377,7 @@ template <int R, bool STREAM, int MEM>
 hipError_t launch(const DiagOp& o, int grid, int budget, hipStream_t s) {
   const auto f = k_resident_diag_cg<R, STREAM, MEM>;
   const size_t lds = diag_lds_bytes(o.ntasks, grid);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+  if (hipError_t e = allow_lds(reinterpret_cast<const void*>(f))) return e;
   k_diag_reset<<<1, 256, 0, s>>>(o);
   DiagOp op = o;
   void* args[] = {&op, &budget};

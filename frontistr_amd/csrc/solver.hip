@@ -1608,7 +1608,7 @@ static int32_t diag_shape(const Context& c) {
   const int32_t t = c.dres.ntasks, most = std::min(c.res_cus, kResidentGridMax);
   if (t == 0 || most < 1) return 0;
   const int32_t grid = t <= 8 ? 1 : std::min(most, (t + 3) / 4);
-  return diag_lds_bytes(t, grid) <= 160 * 1024 ? grid : 0;
+  return diag_lds_bytes(t, grid) <= kLdsBytes ? grid : 0;
 }
 // 1: no memory for it
 static int32_t diag_setup(Context& c) {
