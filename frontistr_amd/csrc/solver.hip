@@ -252,6 +252,8 @@ struct Context {
   uint64_t ssor_num = 0;        // bumped at every numeric SSOR set-up
   int32_t res_cus = 0;          // compute units (0: no cooperative launches)
   int32_t last_resident = 0;    // workgroups of the last solve's resident kernel (0: launch per colour)
+  bool no_resident = false;     // launches only, for a solve whose cooperative launch was refused
+  bool no_waits = false;        // launches only, since a kernel's wait for other workgroups ran out
   bool ssor_proper = false;     // no L'/U' column lies in its row's own colour
   ResidentOp res;
   DiagOp dres;
@@ -1459,7 +1461,7 @@ static ResidentShape resident_shape(const Context& c) {
 // per iteration, no constraint products; gathered records
 // within the 4 GiB of a buffer resource, the colours' ranges within LDS.
 static bool resident_fits(const Context& c, int32_t kind, int32_t iterpremax, bool mixed) {
-  return kind == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N &&
+  return kind == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N && !c.no_resident && !c.no_waits &&
          c.ssor_gen == c.val_gen && c.ssor_proper && c.ssor_rows < 30000000 && c.ncolor <= 512;
 }
 
@@ -1522,20 +1524,27 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t metho
   return 0;
 }
 
+// krylov_once: the solve has to run again from x0, which vz holds, on launches
+constexpr int32_t kAgain = 1;
+
 // The Krylov loop as resident launches of `kResidentBudget` iterations (a bounded
 // stay on the GPU), from r0 in vr and the initial state on the device; the end
-// state in c.h_st[0].
+// state in c.h_st[0].  kAgain: HIP refuses the cooperative launch, or a workgroup waited too long
+// for the others, as on a GPU that is shared in time.
 constexpr int kResidentBudget = 512;
 static int32_t resident_loop(Context& c, const std::function<hipError_t()>& run, const uint32_t* sync) {
   for (;;) {
-    HIPC(run());
+    if (run() != hipSuccess) {
+      (void)hipGetLastError();
+      return kAgain;
+    }
     uint32_t abort = 0;
     HIPC(hipMemcpyAsync(&c.h_st[0], c.st.p, sizeof(KrylovState), hipMemcpyDeviceToHost, c.stream));
     HIPC(hipMemcpyAsync(&abort, sync, sizeof(abort), hipMemcpyDeviceToHost, c.stream));
     HIPC(hipStreamSynchronize(c.stream));
     if (abort) {
-      set_error("resident solve: a workgroup waited 20 s for the others");
-      return HECMW33_ERROR_DEVICE;
+      c.no_waits = true;
+      return kAgain;
     }
     if (c.h_st[0].done) return 0;
   }
@@ -2022,7 +2031,7 @@ static int32_t learned_modes(Context& c, const int32_t* iarray, const double* ra
   return 0;
 }
 
-static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_out* out) {
+static int32_t krylov_once(Context& c, int32_t* iarray, double* rarray, hecmw33_out* out) {
   const double t0 = now_s();
   const int32_t method = IA(iarray, I_METHOD);
   const int32_t pc = IA(iarray, I_PRECOND);
@@ -2142,13 +2151,14 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
     }
   }
   int32_t diag_grid = 0;
-  if (kind == 3 && method == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N) {
+  if (kind == 3 && method == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N && !c.no_resident && !c.no_waits) {
     int32_t e = diag_tasks(c);
     if (e < 0) return e;
     if (e == 0) diag_grid = diag_shape(c);
     if (diag_grid > 0 && diag_setup(c)) diag_grid = 0;
   }
   c.last_resident = std::max(shape.grid, diag_grid);
+  if (c.last_resident > 0) HIPC(hipMemcpyAsync(c.vz.p, c.vx.p, vbytes, hipMemcpyDeviceToDevice, c.stream));
   // r0 = b - A x0; bnrm2 = b.b  (hecmw_solver_CG.f90:131-141)
   if (mixed && c.x_zero) {
     // x0 = 0 (the learned modes' sample solves): r0 = b exactly, without the FP64 product
@@ -2310,6 +2320,20 @@ static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_
   c.last_fallback_iter = learned ? h.fallback_iter : 0;
   c.last_learned_off = learned ? h.learned_off : 1;
   return 0;
+}
+
+static int32_t krylov_core(Context& c, int32_t* iarray, double* rarray, hecmw33_out* out) {
+  const double t0 = now_s();
+  int32_t e = krylov_once(c, iarray, rarray, out);
+  if (e != kAgain) return e;
+  // the factors and the set-up stand (precond_setup has cleared the flags that ask for them)
+  HIPC(hipMemcpyAsync(c.vx.p, c.vz.p, sizeof(double) * 3 * (size_t)c.NP, hipMemcpyDeviceToDevice, c.stream));
+  const double lost = now_s() - t0;
+  c.no_resident = true;
+  e = krylov_once(c, iarray, rarray, out);
+  c.no_resident = false;
+  out->Tset += lost;
+  return e;
 }
 
 static std::mutex g_mu;

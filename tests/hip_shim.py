@@ -1,7 +1,7 @@
 """A child process in which some HIP calls of the library go through functions of this file's
-own: they count and log them, and can refuse a cooperative launch or fail an allocation (the
-real hipMalloc is then asked for more than any card has, so that HIP's last error is what a
-full card leaves).  The functions come before HIP's in the process's symbol order, because
+own: they count and log them, and can refuse a cooperative launch, report that a kernel gave
+up a wait (its word reads 1 on the host) or fail an allocation (the real hipMalloc is then
+asked for more than any card has, so that HIP's last error is what a full card leaves).  The functions come before HIP's in the process's symbol order, because
 they are loaded first and globally."""
 import os
 import subprocess
@@ -15,6 +15,7 @@ SOURCE = r"""
 #include <stddef.h>
 
 int coop_calls = 0, coop_refuse = 0;            /* refuse the next `coop_refuse` cooperative launches */
+int gave_up = 0;                                /* the next `gave_up` abort words read 1 */
 int malloc_calls = 0, malloc_fail_at = -1, malloc_fail_n = 1; /* fail calls malloc_fail_at ... */
 int attr_n = 0, attr_value[256];
 const void* attr_func[256];
@@ -33,6 +34,17 @@ int hipFuncSetAttribute(const void* func, int attr, int value) {
   int (*f)(const void*, int, int) = (int (*)(const void*, int, int))real("hipFuncSetAttribute");
   if (attr_n < 256) attr_func[attr_n] = func, attr_value[attr_n++] = value;
   return f(func, attr, value);
+}
+int hipMemcpyAsync(void* dst, const void* src, size_t n, int kind, void* s) {
+  int (*f)(void*, const void*, size_t, int, void*) = (int (*)(void*, const void*, size_t, int, void*))real("hipMemcpyAsync");
+  const int e = f(dst, src, n, kind, s);
+  if (e == 0 && n == 4 && kind == 2 && gave_up > 0) {
+    int (*sync)(void*) = (int (*)(void*))real("hipStreamSynchronize");
+    gave_up--;
+    sync(s);
+    *(int*)dst = 1;
+  }
+  return e;
 }
 typedef struct { unsigned x, y, z; } dim3_t;
 int hipLaunchCooperativeKernel(const void* func, dim3_t g, dim3_t b, void** args, unsigned lds, void* s) {
