@@ -99,6 +99,7 @@ struct FlowOp {
   float4* rhs = nullptr;                       // r in slot order
   void* rec = nullptr;                         // float4 [2][ns]: forward, then backward results
   uint32_t* ticket = nullptr;
+  uint32_t* gave_up = nullptr;                 // host memory, set where a wait ran out
   int32_t ns = 0, grid = 0;
   bool b16 = false;
 };

@@ -264,6 +264,7 @@ struct Context {
   bool ssor16_valid = false;   // L.val16 / U.val16 hold the current values
   // the FP32 sweeps as one kernel: packed columns, values in BF16 and in FP32
   FlowOp flow;
+  uint32_t* flow_gave_up = nullptr;  // pinned host word: a wait in the sweeps ran out
   bool flow_use = false;       // for this structure
   bool ssor_round_valid = false;  // L.val32 / U.val32 hold the current values
   bool flow_sym = false, flow_valid[2] = {false, false};
@@ -391,6 +392,7 @@ struct Context {
       for (DMem* m : {&s->ptr, &s->len, &s->col, &s->src, &s->val, &s->val32, &s->val16}) m->release();
     for (hipEvent_t e : events) (void)hipEventDestroy(e);
     if (h_st) (void)hipHostFree(h_st);
+    if (flow_gave_up) (void)hipHostFree(flow_gave_up);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -445,6 +447,8 @@ static int32_t ctx_init(Context& c) {
   if (coop) HIPC(hipDeviceGetAttribute(&c.res_cus, hipDeviceAttributeMultiprocessorCount, dev));
   HIPC(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   HIPC(hipHostMalloc((void**)&c.h_st, 2 * sizeof(KrylovState), hipHostMallocDefault));
+  HIPC(hipHostMalloc((void**)&c.flow_gave_up, sizeof(uint32_t), hipHostMallocDefault));
+  *c.flow_gave_up = 0;
   if (c.st.ensure(sizeof(KrylovState)) || c.part.ensure(sizeof(double) * 4 * kMaxPartials))
     return HECMW33_ERROR_DEVICE;
   HIPC(hipMemsetAsync(c.st.p, 0, sizeof(KrylovState), c.stream));
@@ -826,6 +830,7 @@ static int32_t flow_setup(Context& c, bool v16) {
       o.len[d] = (d ? c.U : c.L).view.len;
     }
     o.ticket = reinterpret_cast<uint32_t*>(p);
+    o.gave_up = c.flow_gave_up;
     o.row_old = c.row_old.as<int32_t>();
     o.ns = ns;
     // four times the workgroups that a colour's slices occupy, so that the slices of the next
@@ -848,6 +853,15 @@ static int32_t flow_setup(Context& c, bool v16) {
   return 0;
 }
 
+// Whether a wait in the FP32 sweeps that have run ended early, so that marks (NaN) went on:
+// from now on this context takes the launches.
+static bool flow_failed(Context& c) {
+  if (!c.flow_use || !*static_cast<volatile uint32_t*>(c.flow_gave_up)) return false;
+  *c.flow_gave_up = 0;
+  c.no_waits = true;
+  return true;
+}
+
 // v16: the SSOR sweeps will read BF16 copies of the L'/U' values (rounded to
 // nearest even from the FP32 image)
 static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
@@ -863,7 +877,9 @@ static int32_t setup_f32(Context& c, int32_t kind, bool v16) {
     launch_to_f32(9 * nslot, c.alu_ssor.as<double>(), c.alu_ssor32.as<float>(), c.stream);
     c.ssor32_valid = true;
   }
-  if (kind == 1 && !c.flow_valid[v16 ? 1 : 0]) {
+  if (kind == 1 && c.no_waits) {
+    c.flow_use = false;
+  } else if (kind == 1 && !c.flow_valid[v16 ? 1 : 0]) {
     const int32_t e = flow_setup(c, v16);
     if (e < 0) return e;
     c.flow_use = e == 0;
@@ -2158,7 +2174,8 @@ static int32_t krylov_once(Context& c, int32_t* iarray, double* rarray, hecmw33_
     if (diag_grid > 0 && diag_setup(c)) diag_grid = 0;
   }
   c.last_resident = std::max(shape.grid, diag_grid);
-  if (c.last_resident > 0) HIPC(hipMemcpyAsync(c.vz.p, c.vx.p, vbytes, hipMemcpyDeviceToDevice, c.stream));
+  if (c.last_resident > 0 || (mixed && kind == 1 && c.flow_use))
+    HIPC(hipMemcpyAsync(c.vz.p, c.vx.p, vbytes, hipMemcpyDeviceToDevice, c.stream));
   // r0 = b - A x0; bnrm2 = b.b  (hecmw_solver_CG.f90:131-141)
   if (mixed && c.x_zero) {
     // x0 = 0 (the learned modes' sample solves): r0 = b exactly, without the FP64 product
@@ -2287,6 +2304,7 @@ static int32_t krylov_once(Context& c, int32_t* iarray, double* rarray, hecmw33_
     HIPC(hipStreamSynchronize(c.stream));
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
+    if (mixed && kind == 1 && flow_failed(c)) return kAgain;
   }
   h = c.h_st[0];
   out->Tsol = now_s() - t1;
@@ -2719,18 +2737,32 @@ int32_t hecmw33_ctx_ssor_device(hecmw33_ctx* ctx, const void* r_dev, void* z_dev
   hipEvent_t e0, e1;
   HIPC(hipEventCreate(&e0));
   HIPC(hipEventCreate(&e1));
-  HIPC(hipEventRecord(e0, c.stream));
-  for (int i = 0; i < count; ++i) {
-    if (fp32)
-      ssor_apply_f32(c.ssor_op32(fp32 == 1), static_cast<const float*>(r_dev), static_cast<float*>(z_dev), nullptr, c.stream);
-    else
-      ssor_apply(c.ssor_op(), static_cast<const double*>(r_dev), static_cast<double*>(z_dev), nullptr, c.stream);
-  }
-  HIPC(hipEventRecord(e1, c.stream));
-  HIPC(hipEventSynchronize(e1));
   float t = 0.f;
-  HIPC(hipEventElapsedTime(&t, e0, e1));
-  HIPC(hipGetLastError());
+  auto run = [&]() -> int32_t {
+    HIPC(hipEventRecord(e0, c.stream));
+    for (int i = 0; i < count; ++i) {
+      if (fp32)
+        ssor_apply_f32(c.ssor_op32(fp32 == 1), static_cast<const float*>(r_dev), static_cast<float*>(z_dev), nullptr, c.stream);
+      else
+        ssor_apply(c.ssor_op(), static_cast<const double*>(r_dev), static_cast<double*>(z_dev), nullptr, c.stream);
+    }
+    HIPC(hipEventRecord(e1, c.stream));
+    HIPC(hipEventSynchronize(e1));
+    HIPC(hipEventElapsedTime(&t, e0, e1));
+    HIPC(hipGetLastError());
+    return 0;
+  };
+  if (int32_t e = run()) return e;
+  if (fp32 && flow_failed(c)) {
+    const char *r = static_cast<const char*>(r_dev), *z = static_cast<const char*>(z_dev);
+    const ptrdiff_t bytes = (ptrdiff_t)sizeof(float) * 3 * c.N;
+    if (r < z + bytes && z < r + bytes) {
+      set_error("hecmw33_ctx_ssor_device: a wait in the sweeps ran out, and r is overwritten by z");
+      return HECMW33_ERROR_DEVICE;
+    }
+    if (int32_t e = setup_f32(c, 1, fp32 == 1)) return e;
+    if (int32_t e = run()) return e;
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (ms) *ms = (double)t / count;

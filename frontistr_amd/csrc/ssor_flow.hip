@@ -144,10 +144,11 @@ struct Flow {
       for (int i = 0; i < 2 * N; ++i) more |= want[i];
       if (!__any(more || want_own) || dead) break;
       if ((spins & 1023u) == 0) {
-        // a wait that has run long is given up: marks, which are NaN, go on
+        // a wait that has run long is given up: marks, which are NaN, go on, and the host is told
         const uint64_t now = wall_clock64();
         if (t0 == 0) t0 = now;
         dead = __any(now - t0 > kWaitTicks);
+        if (dead && lane == 0) __hip_atomic_store(o.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
   }

@@ -1,6 +1,6 @@
 """A child process in which some HIP calls of the library go through functions of this file's
 own: they count and log them, and can refuse a cooperative launch, report that a kernel gave
-up a wait (its word reads 1 on the host) or fail an allocation (the real hipMalloc is then
+up a wait (its word on the host reads 1) or fail an allocation (the real hipMalloc is then
 asked for more than any card has, so that HIP's last error is what a full card leaves).  The functions come before HIP's in the process's symbol order, because
 they are loaded first and globally."""
 import os
@@ -16,6 +16,8 @@ SOURCE = r"""
 
 int coop_calls = 0, coop_refuse = 0;            /* refuse the next `coop_refuse` cooperative launches */
 int gave_up = 0;                                /* the next `gave_up` abort words read 1 */
+int flow_gave_up = 0, *flow_word = NULL;        /* the next `flow_gave_up` waits for an event set the sweeps' word */
+int launches = 0;
 int malloc_calls = 0, malloc_fail_at = -1, malloc_fail_n = 1; /* fail calls malloc_fail_at ... */
 int attr_n = 0, attr_value[256];
 const void* attr_func[256];
@@ -46,7 +48,28 @@ int hipMemcpyAsync(void* dst, const void* src, size_t n, int kind, void* s) {
   }
   return e;
 }
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  int (*f)(void**, size_t, unsigned) = (int (*)(void**, size_t, unsigned))real("hipHostMalloc");
+  const int e = f(p, n, flags);
+  if (e == 0 && n == 4) flow_word = *p;
+  return e;
+}
+int hipEventSynchronize(void* ev) {
+  int (*f)(void*) = (int (*)(void*))real("hipEventSynchronize");
+  const int e = f(ev);
+  if (flow_gave_up > 0 && flow_word) {
+    flow_gave_up--;
+    *flow_word = 1;
+  }
+  return e;
+}
 typedef struct { unsigned x, y, z; } dim3_t;
+int hipLaunchKernel(const void* func, dim3_t g, dim3_t b, void** args, size_t lds, void* s) {
+  int (*f)(const void*, dim3_t, dim3_t, void**, size_t, void*) =
+      (int (*)(const void*, dim3_t, dim3_t, void**, size_t, void*))real("hipLaunchKernel");
+  launches++;
+  return f(func, g, b, args, lds, s);
+}
 int hipLaunchCooperativeKernel(const void* func, dim3_t g, dim3_t b, void** args, unsigned lds, void* s) {
   int (*f)(const void*, dim3_t, dim3_t, void**, unsigned, void*) =
       (int (*)(const void*, dim3_t, dim3_t, void**, unsigned, void*))real("hipLaunchCooperativeKernel");

@@ -77,3 +77,97 @@ def test_a_refused_launch_or_an_ended_wait_leaves_the_solve_to_the_launches(tmp_
     starts again from x0 (the second time bit for bit what it was the first time)."""
     out = hip_shim.run(tmp_path, SOLVE.format(method=method, precond=precond, make=make))
     assert out[-1] == "done", out
+
+
+FLOW = """
+import torch
+m = fa.gen_hex8(12, kind='lognormal', seed=2)
+m.set_precond(1)
+ctx = fa.DeviceContext()
+ctx.load(m)
+r = torch.from_numpy(np.random.default_rng(3).standard_normal(3 * m.NP).astype(np.float32)).cuda()
+def apply():
+    z = torch.zeros_like(r)
+    torch.cuda.synchronize()
+    before = val("launches").value
+    ctx.ssor_device(r.data_ptr(), z.data_ptr(), 1, fp32=True, bf16={bf16})
+    return z.cpu().numpy(), val("launches").value - before
+first, n0 = apply()
+want, n1 = apply()
+assert n1 <= 4 and np.array_equal(first, want)
+val("flow_gave_up").value = 1
+z, n2 = apply()
+assert val("flow_gave_up").value == 0 and n2 >= n1 + 2 * ctx.info()["ncolor"], (n1, n2)
+assert np.array_equal(z, want)
+z, n3 = apply()
+assert 2 * ctx.info()["ncolor"] <= n3 < n2 and np.array_equal(z, want), (n1, n2, n3)
+ctx.close()
+# in place r is gone: an error instead of a wrong answer
+ctx = fa.DeviceContext()
+ctx.load(m)
+val("flow_gave_up").value = 1
+z = r.clone()
+torch.cuda.synchronize()
+try:
+    ctx.ssor_device(z.data_ptr(), z.data_ptr(), 1, fp32=True, bf16={bf16})
+    print("no error")
+except fa.HecmwError:
+    pass
+ctx.close()
+print("done")
+"""
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_an_ended_wait_in_the_fp32_sweeps_leaves_the_application_to_the_launches(tmp_path, bf16):
+    """Where a wait of the one-kernel sweeps ends early, NaN marks go on as values: the
+    application is done again by the launches (the same numbers, bit for bit), and the ones after it."""
+    out = hip_shim.run(tmp_path, FLOW.format(bf16=bf16))
+    assert out[-1] == "done", out
+
+
+MIXED = """
+import torch
+n = 14
+m = fa.gen_hex8(n, kind='lognormal', seed=2)
+m.set_iter(3000)
+m.set_resid(1e-10)
+m.set_precond(1)
+m.set_mixed()
+if {coarse}:
+    m.set_coarse(30, deflation=True)
+if {learned}:
+    m.set_i(m.I_SOLVER_OPT, 2)
+b = torch.from_numpy(m.B).cuda()
+x0 = torch.from_numpy(np.random.default_rng(5).standard_normal(m.B.size) * 1e-3).cuda()
+def solve(ctx, at):
+    x = x0.clone()
+    torch.cuda.synchronize()
+    val("flow_gave_up").value = at
+    before = val("launches").value
+    r = ctx.solve_device(b.data_ptr(), x.data_ptr(), m.Iarray.copy(), m.Rarray)
+    left = val("flow_gave_up").value
+    val("flow_gave_up").value = 0
+    return x.cpu().numpy(), r, val("launches").value - before, left
+def context():
+    ctx = fa.DeviceContext()
+    ctx.set_coords(fa.hex8_coords(n))
+    ctx.load(m)
+    return ctx
+one = context()
+x, r, n1, _ = solve(one, 0)
+two = context()
+y, q, n2, left = solve(two, 1)
+print(r.iter, q.iter, r.resid, q.resid, n1, n2)
+assert left == 0 and r.error == 0 and q.error == 0
+assert r.iter == q.iter and r.resid == q.resid and np.array_equal(x, y)
+assert n2 > n1 + 2 * two.info()["ncolor"] * (q.iter - 1)
+print("done")
+"""
+
+
+@pytest.mark.parametrize("coarse,learned", [(0, 0), (1, 0), (1, 1)])
+def test_an_ended_wait_in_a_flexible_cg_starts_it_again_on_the_launches(tmp_path, coarse, learned):
+    """Also inside the sample solves of the learned modes, which start from x = 0."""
+    out = hip_shim.run(tmp_path, MIXED.format(coarse=coarse, learned=learned))
+    assert out[-1] == "done", out
