@@ -291,7 +291,7 @@ struct Resident : GridGroup<T, MEM> {
       while ((int32_t)(__hip_atomic_load(fin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) - first) < 0)
         __builtin_amdgcn_s_sleep(1);
       double x[K][3 * NG];
-      gather<NG>(cp, with_z, x);
+      gather<NG>(cp, MEM == kGrid && o.cached && with_z, x);
 #pragma unroll
       for (int g = 0; g < NG; ++g)
 #pragma unroll
