@@ -144,11 +144,11 @@ struct Flow {
       for (int i = 0; i < 2 * N; ++i) more |= want[i];
       if (!__any(more || want_own) || dead) break;
       if ((spins & 1023u) == 0) {
-        // a wait that has run long is given up: marks, which are NaN, go on, and the host is told
+        // a wait that has run long is given up: marks, which are NaN, go on, and at the end
+        // the host is told
         const uint64_t now = wall_clock64();
         if (t0 == 0) t0 = now;
         dead = __any(now - t0 > kWaitTicks);
-        if (dead && lane == 0) __hip_atomic_store(o.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
   }
@@ -221,6 +221,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_ssor_flow(FlowOp o, const Kryl
     task = now * kFlowWaves + wave;
     if (task < ntask) f.load(task);
   }
+  if (f.dead && f.lane == 0) __hip_atomic_store(o.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // r into slot order, the records marked, the counter at zero
