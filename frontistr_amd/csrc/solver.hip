@@ -1571,9 +1571,15 @@ static int32_t resident_solve(Context& c, const ResidentShape& sh) {
 }
 
 // ---- resident CG with block-diagonal scaling (resident_diag.hip) -------------------------------
+static int32_t diag_no_memory(Context& c) {
+  for (DMem* m : {&c.dres_task, &c.dres_lane, &c.dres_row, &c.dres_z}) m->release();
+  c.dres_sym = false;
+  (void)hipGetLastError();
+  return 1;
+}
 // Workgroups for this system, 0: the launch-per-kernel solve.  The tasks are made here;
 // rows whose four-row group needs more than 64 lanes, or more tasks than the LDS of the
-// workgroups hold, are not taken.
+// workgroups hold, are not taken.  1: no memory for the tasks.
 static int32_t diag_tasks(Context& c) {
   if (c.dres_sym) return 0;
   const int32_t N = c.N, nrow = (N + 3) / 4 * 4;
@@ -1615,7 +1621,7 @@ static int32_t diag_tasks(Context& c) {
   }
   if (c.dres_task.ensure(sizeof(int4) * task.size()) || c.dres_lane.ensure(sizeof(int32_t) * lane.size()) ||
       c.dres_row.ensure(sizeof(int2) * row.size()))
-    return 1;
+    return diag_no_memory(c);
   HIPC(hipMemcpyAsync(c.dres_task.p, task.data(), sizeof(int4) * task.size(), hipMemcpyHostToDevice, c.stream));
   HIPC(hipMemcpyAsync(c.dres_lane.p, lane.data(), sizeof(int32_t) * lane.size(), hipMemcpyHostToDevice, c.stream));
   HIPC(hipMemcpyAsync(c.dres_row.p, row.data(), sizeof(int2) * row.size(), hipMemcpyHostToDevice, c.stream));
@@ -1642,11 +1648,8 @@ static int32_t diag_setup(Context& c) {
   o.zero_rec = nrow;
   o.copy = 4 * ((int64_t)nrow + 4);
   o.ring = (int32_t)std::max<int64_t>(4, std::min<int64_t>(64, (64 << 20) / (8 * o.copy)));
-  if (c.dres_z.ensure(sizeof(double) * o.copy * o.ring) || c.res_sync.ensure(sizeof(uint32_t) * kResidentSync)) {
-    c.dres_z.release();
-    (void)hipGetLastError();
-    return 1;
-  }
+  if (c.dres_z.ensure(sizeof(double) * o.copy * o.ring) || c.res_sync.ensure(sizeof(uint32_t) * kResidentSync))
+    return diag_no_memory(c);
   o.A = c.A.view;
   o.task = c.dres_task.as<int4>();
   o.lane = c.dres_lane.as<int32_t>();

@@ -171,3 +171,55 @@ def test_an_ended_wait_in_a_flexible_cg_starts_it_again_on_the_launches(tmp_path
     """Also inside the sample solves of the learned modes, which start from x = 0."""
     out = hip_shim.run(tmp_path, MIXED.format(coarse=coarse, learned=learned))
     assert out[-1] == "done", out
+
+
+NO_MEMORY = """
+import torch
+m = fa.gen_hex8(9, kind='lognormal', seed=2)
+m.set_precond({precond})
+m.set_sigma_diag({sigma})
+m.set_iter(3000)
+m.set_resid(1e-10)
+xr, info = restate.solve_krylov(m)
+ia = m.Iarray.copy()
+ia[m.I_FLAG_NUMFACT - 1] = ia[m.I_FLAG_SYMBFACT - 1] = 0
+b = torch.from_numpy(m.B).cuda()
+def solve(ctx):
+    x = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    before = val("malloc_calls").value
+    r = ctx.solve_device(b.data_ptr(), x.data_ptr(), ia, m.Rarray)
+    x = x.cpu().numpy()
+    assert r.error == 0 and np.linalg.norm(x - xr) <= 1e-6 * np.linalg.norm(xr)
+    return ctx.info()["resident"], val("malloc_calls").value - before
+ctx = fa.DeviceContext()
+ctx.load(m)
+resident, calls = solve(ctx)
+assert resident > 0 and calls == {calls}, (resident, calls)
+ctx.close()
+for k in range(1, calls):  # the first is the residual history's, which every solve needs
+    ctx = fa.DeviceContext()
+    ctx.load(m)
+    val("malloc_fail_at").value = val("malloc_calls").value + k
+    try:
+        r1, _ = solve(ctx)
+    except fa.HecmwError as e:
+        print(k, e)
+        continue
+    val("malloc_fail_at").value = -1
+    r2, _ = solve(ctx)
+    ctx.close()
+    print(k, "resident", r1, r2)
+    assert r1 == 0 and r2 == resident
+    ok = k
+assert ok == calls - 1
+print("done")
+"""
+
+
+@pytest.mark.parametrize("precond,sigma,calls", [(3, 1.0, 6)])
+def test_a_resident_solve_without_memory_runs_on_the_launches(tmp_path, precond, sigma, calls):
+    """Whichever of a resident solve's own allocations fails: the launches solve it, and the next
+    solve, with memory, is resident."""
+    out = hip_shim.run(tmp_path, NO_MEMORY.format(precond=precond, sigma=sigma, calls=calls))
+    assert out[-1] == "done" and not [l for l in out if "error" in l], out
