@@ -1517,7 +1517,7 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t metho
   }
   o.dsig = nullptr;
   if (c.ssor_sigma != 1.0) {
-    if (c.res_dsig.ensure(sizeof(double) * 3 * (size_t)ns)) return HECMW33_ERROR_DEVICE;
+    if (c.res_dsig.ensure(sizeof(double) * 3 * (size_t)ns)) return resident_no_memory(c);
     resident_dsig(ns, c.row_old.as<int32_t>(), c.dD.as<double>(), c.ssor_sigma, c.res_dsig.as<double>(), c.stream);
     o.dsig = c.res_dsig.as<double>();
   }

@@ -217,7 +217,7 @@ print("done")
 """
 
 
-@pytest.mark.parametrize("precond,sigma,calls", [(3, 1.0, 6)])
+@pytest.mark.parametrize("precond,sigma,calls", [(3, 1.0, 6), (1, 1.0, 8), (1, 1.35, 9)])
 def test_a_resident_solve_without_memory_runs_on_the_launches(tmp_path, precond, sigma, calls):
     """Whichever of a resident solve's own allocations fails: the launches solve it, and the next
     solve, with memory, is resident."""
