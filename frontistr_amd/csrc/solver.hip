@@ -1577,19 +1577,35 @@ static int32_t diag_no_memory(Context& c) {
   (void)hipGetLastError();
   return 1;
 }
-// Workgroups for this system, 0: the launch-per-kernel solve.  The tasks are made here;
-// rows whose four-row group needs more than 64 lanes, or more tasks than the LDS of the
-// workgroups hold, are not taken.  1: no memory for the tasks.
+// One task per wave up to all CUs: a wave's second task costs about what the barriers of
+// more workgroups cost in all (12^3 cube, us an iteration: 17.8 with 8 workgroups, 11.8 with 16,
+// 8.1 with 32, 7.0 with 35 and 64, 7.4 with 128; 20^3: 11.9 with 72, 9.7 with 128, 8.7
+// with 145).  One workgroup up to two tasks per wave saves the exchange (3^3: 4.4
+// against 6.2 with 2, 4^3: 5.7 against 6.0, but 5^3, 14 tasks: 11.0 against 6.2).
+// 0: t tasks do not fit, and the launch-per-kernel solve runs.
+static int32_t diag_shape(const Context& c, int32_t t) {
+  const int32_t most = std::min(c.res_cus, kResidentGridMax);
+  if (t == 0 || most < 1) return 0;
+  const int32_t grid = t <= 8 ? 1 : std::min(most, (t + 3) / 4);
+  return diag_lds_bytes(t, grid) <= kLdsBytes ? grid : 0;
+}
+// The tasks of this system (none: not taken).  Rows whose four-row group needs more than 64
+// lanes, or more tasks than the LDS of the workgroups hold, are not taken; above 172,000 nodes
+// full tasks of 16 rows would not fit either, and none are made.  1: no memory for the tasks.
 static int32_t diag_tasks(Context& c) {
   if (c.dres_sym) return 0;
   const int32_t N = c.N, nrow = (N + 3) / 4 * 4;
+  DiagOp& o = c.dres;
+  o.ntasks = 0;
+  if (diag_shape(c, (N + kResidentRows - 1) / kResidentRows) == 0) {
+    c.dres_sym = true;
+    return 0;
+  }
   const int32_t *iL = c.h_indexL.data(), *iU = c.h_indexU.data();
   std::vector<int4> task;
   std::vector<int32_t> lane, lanes(nrow, 0);
   std::vector<int2> row(nrow);
   for (int32_t i = 0; i < N; ++i) lanes[i] = (1 + iL[i + 1] - iL[i] + iU[i + 1] - iU[i] + kDiagK - 1) / kDiagK;
-  DiagOp& o = c.dres;
-  o.ntasks = 0;
   for (int32_t i = 0; i < nrow;) {
     int32_t used = 0, n = 0;
     while (n < kResidentRows && i + n < nrow) {
@@ -1629,17 +1645,6 @@ static int32_t diag_tasks(Context& c) {
   o.ntasks = (int32_t)task.size();
   c.dres_sym = true;
   return 0;
-}
-// One task per wave up to all CUs: a wave's second task costs about what the barriers of
-// more workgroups cost in all (12^3 cube, us an iteration: 17.8 with 8 workgroups, 11.8 with 16,
-// 8.1 with 32, 7.0 with 35 and 64, 7.4 with 128; 20^3: 11.9 with 72, 9.7 with 128, 8.7
-// with 145).  One workgroup up to two tasks per wave saves the exchange (3^3: 4.4
-// against 6.2 with 2, 4^3: 5.7 against 6.0, but 5^3, 14 tasks: 11.0 against 6.2).
-static int32_t diag_shape(const Context& c) {
-  const int32_t t = c.dres.ntasks, most = std::min(c.res_cus, kResidentGridMax);
-  if (t == 0 || most < 1) return 0;
-  const int32_t grid = t <= 8 ? 1 : std::min(most, (t + 3) / 4);
-  return diag_lds_bytes(t, grid) <= kLdsBytes ? grid : 0;
 }
 // 1: no memory for it
 static int32_t diag_setup(Context& c) {
@@ -2173,7 +2178,7 @@ static int32_t krylov_once(Context& c, int32_t* iarray, double* rarray, hecmw33_
   if (kind == 3 && method == 1 && iterpremax == 1 && !mixed && !c.mpc_use && c.NP == c.N && !c.no_resident && !c.no_waits) {
     int32_t e = diag_tasks(c);
     if (e < 0) return e;
-    if (e == 0) diag_grid = diag_shape(c);
+    if (e == 0) diag_grid = diag_shape(c, c.dres.ntasks);
     if (diag_grid > 0 && diag_setup(c)) diag_grid = 0;
   }
   c.last_resident = std::max(shape.grid, diag_grid);
