@@ -247,6 +247,8 @@ struct Context {
   uint64_t ssor_gen = 0;        // val_gen that the SSOR factors were made from
   double ssor_sigma = 1.0;
   std::vector<int32_t> h_lenL, h_lenU;  // blocks of every row slot
+  int32_t res_longest = 0;      // most blocks of a row of L', U'
+  int64_t res_lanes = 0;        // lanes of all rows at two blocks each
   int32_t res_packets = 0;      // blocks per lane of the packed structure (0: none built)
   uint64_t res_num = 0;         // numeric set-up (ssor_num) that the packed values hold
   uint64_t ssor_num = 0;        // bumped at every numeric SSOR set-up
@@ -722,6 +724,13 @@ static int32_t setup_ssor_symbolic(Context& c, int32_t ncolor_in) {
   }
   c.h_lenL = std::move(hl.len);
   c.h_lenU = std::move(hu.len);
+  c.res_longest = 0;
+  c.res_lanes = 0;
+  for (const std::vector<int32_t>* len : {&c.h_lenL, &c.h_lenU})
+    for (int32_t l : *len) {
+      c.res_longest = std::max(c.res_longest, l);
+      c.res_lanes += (l + 1) / 2;
+    }
   c.res_packets = 0;
   c.flow_sym = false;
   // the slot of every node, for staging r into slot order and z back out
@@ -1455,16 +1464,9 @@ static int32_t resident_tasks(Context& c, const ResidentShape& sh) {
 //    nodes: 55 and 65).
 static ResidentShape resident_shape(const Context& c) {
   ResidentShape sh;
-  int32_t longest = 0;
-  int64_t lanes = 0;
-  for (const std::vector<int32_t>* len : {&c.h_lenL, &c.h_lenU})
-    for (int32_t l : *len) {
-      longest = std::max(longest, l);
-      lanes += (l + 1) / 2;
-    }
-  if (longest > kWave * kResidentPackets || c.res_cus < 1) return sh;
-  if (longest > 2 * kWave) sh.packets = 4;
-  const int64_t tasks = lanes / (2 * (int64_t)c.ncolor * kWave);
+  if (c.res_longest > kWave * kResidentPackets || c.res_cus < 1) return sh;
+  if (c.res_longest > 2 * kWave) sh.packets = 4;
+  const int64_t tasks = c.res_lanes / (2 * (int64_t)c.ncolor * kWave);
   sh.grid = tasks < 16 ? 32 : tasks < 64 ? 128 : 256;
   if (c.N <= 450 && resident_one_group(c.ncolor, (int)c.ssor_rows)) sh.grid = 1;
   sh.grid = std::min(sh.grid, std::min(c.res_cus, kResidentGridMax));
