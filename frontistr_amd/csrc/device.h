@@ -103,6 +103,8 @@ struct FlowOp {
   int32_t ns = 0, grid = 0;
   bool b16 = false;
 };
+// Whether a buffer resource, 4 GiB, reaches the two records of every row slot.
+inline bool flow_reaches(int64_t slots) { return 32 * slots <= (int64_t)UINT32_MAX; }
 void flow_pack(const Sell<double>& m, const int32_t* group, bool desc, bool b16, void* val, int2* col, hipStream_t s);
 void flow_sweeps(const FlowOp& o, const float* r, const KrylovState* st, hipStream_t s);
 

@@ -808,11 +808,12 @@ static int32_t round_sell(SellDev& d, hipStream_t s) {
   launch_to_f32(9 * d.view.nslots, d.view.val, d.view32.val, s);
   return 0;
 }
-// The FP32 sweeps as one kernel, if this structure takes it: slices of 16 rows, and no
-// couplings inside a colour (there a row would wait for one that is drawn with it).
+// The FP32 sweeps as one kernel, if this structure takes it: slices of 16 rows, no
+// couplings inside a colour (there a row would wait for one that is drawn with it), and
+// records within the 4 GiB of a buffer resource.
 // 1: not taken, or no memory for the packed copy.
 static int32_t flow_setup(Context& c, bool v16) {
-  if (c.ssor_R != kRowsS || !c.ssor_proper || c.ssor_rows < 1) return 1;
+  if (c.ssor_R != kRowsS || !c.ssor_proper || c.ssor_rows < 1 || !flow_reaches(c.ssor_rows)) return 1;
   const int32_t ns = (int32_t)c.ssor_rows, S = ns / kRowsS;
   auto no_memory = [&] {
     for (DMem* m : {&c.flow_mem, &c.flow_val[0], &c.flow_val[1]}) m->release();
