@@ -1493,7 +1493,8 @@ int32_t hecmw33_batch_spmm(hecmw33_batch* b, int32_t fp64, const double* const* 
 // [0] rows, [1] blocks, [2] tiles, [3] FP32 shape, [4] nv32, [5..5+nv32) FP32 shape times in us (SpMM +
 // dots; 0 when the shapes came from the persisted winners), FP64 shape, nv64, FP64 shape times in us,
 // then: shapes from the persisted winners (0/1), CU count, the persistent grids of the p, q = A p,
-// update, residual and DIAG launches
+// update and residual launches, and the one that kb_diag by itself would take (it runs over
+// every tile)
 int32_t hecmw33_batch_info(hecmw33_batch* b, int64_t* info, int32_t n) {
   if (!b || !info) return HECMW33_ERROR_ARGS;
   std::vector<int64_t> v = {b->nrows, b->nnzb, b->ntiles, b->variant, kNumVariants};

@@ -82,7 +82,6 @@ struct Sell {
 // iteration.
 struct KrylovState;
 
-// Multicolour SSOR operator (hecmw_precond_SSOR_33) as the sweeps see it.
 // The FP32 sweeps as one kernel (ssor_flow.hip).  Blocks of a row in groups of kFlowBlocks
 // (backward rows from their last block on), group[dir][s] the first of slice s: the
 // columns of lane 4 r + q, blocks q and q + 4, at col[dir][64 g + lane]; the values of
@@ -108,6 +107,7 @@ inline bool flow_reaches(int64_t slots) { return 32 * slots <= (int64_t)UINT32_M
 void flow_pack(const Sell<double>& m, const int32_t* group, bool desc, bool b16, void* val, int2* col, hipStream_t s);
 void flow_sweeps(const FlowOp& o, const float* r, const KrylovState* st, hipStream_t s);
 
+// Multicolour SSOR operator (hecmw_precond_SSOR_33) as the sweeps see it.
 template <typename T>
 struct SsorOp {
   Sell<T> L, U;                // L'/U' per colour slice; columns are slot ids
@@ -267,7 +267,7 @@ void bi_update(int64_t n3, const double* pt, const double* stv, const double* t,
 // come first, then those of U'.
 constexpr int kLdsBytes = 160 * 1024;   // LDS of a CU
 constexpr int kResidentGridMax = 256;   // workgroups (one per CU)
-constexpr int kResidentSync = 640 + 12 * kResidentGridMax;  // words: abort flag, counts, entries of the exchanges
+constexpr int kResidentSync = 64 + 12 * kResidentGridMax;  // words: abort flag, entries of the exchanges
 constexpr int kResidentPlanesCg = 27;   // of 16 slots in a row record: the LU and six vectors (CG)
 constexpr int kResidentPlanesBi = 39;   // or ten (BiCGSTAB)
 constexpr int kResidentPackets = 4;     // most blocks per lane

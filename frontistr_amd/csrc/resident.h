@@ -48,10 +48,9 @@ __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0
 // orders a wave's own LDS accesses (the LDS serves a wave in order)
 __device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
-// what the workgroups share in `sync`: an abort flag, the root and eight group counts of
-// arrivals, each in words of its own, and from word kSyncParts on three sets of two
-// entries per workgroup for the exchanges
-constexpr int kSyncParts = 64 * 10;
+// what the workgroups share in `sync`: an abort flag in lines of its own, and from word
+// kSyncParts on three sets of two entries per workgroup for the exchanges
+constexpr int kSyncParts = 64;
 constexpr int kSyncSet = 2 * kResidentGridMax;
 static_assert(kResidentSync == kSyncParts + 3 * 2 * kSyncSet, "words of the exchange");
 

@@ -109,7 +109,7 @@ struct Resident : GridGroup<T, MEM> {
 
   const ResidentOp& o;
   __amdgpu_buffer_rsrc_t rsrc;
-  double* zw0;           // the two copies of the gathered records, copy_size doubles each
+  double* zw0;           // the copies of the gathered records (o.ring), copy_size doubles each
   int64_t copy_size;
   double* prod;
   uint32_t* fin;

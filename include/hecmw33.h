@@ -60,7 +60,10 @@ typedef struct hecmw33_out {
   double resid;          /* RESID of the Krylov loop */
   double resid_true;     /* hecmw_rel_resid_L2 after the solve (hecmw33_solve only) */
   double Tset, Tsol, Tcomm;
-  double time_Ax, time_precond;  /* filled when TIMELOG (Iarray 22) >= 1 */
+  double time_Ax, time_precond;  /* filled when TIMELOG (Iarray 22) >= 1.  A solve in one resident kernel has no
+                                  * product apart from its preconditioner: time_Ax is then, with SSOR, its forward
+                                  * sweeps (which give A z and do half of M^-1), with DIAG its products and p, q;
+                                  * time_precond the backward sweeps, or the rest of an iteration */
   double t_upload;       /* host->device copies of this call (not part of Tset/Tsol) */
 } hecmw33_out;
 
