@@ -16,6 +16,13 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP library)")
 
 
+def pytest_collection_modifyitems(items):
+    """Tests that run the library in a child process go first.  HIP gives the GPU's cooperative
+    queue to one process: once this one has launched cooperatively, it refuses a child's
+    cooperative launches (401), and the child's solves take the launches."""
+    items.sort(key=lambda i: not (hasattr(i, "function") and "hip_shim" in i.function.__code__.co_names))
+
+
 @pytest.fixture(scope="session")
 def has_gpu():
     import frontistr_amd as fa
