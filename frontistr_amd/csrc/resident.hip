@@ -16,8 +16,8 @@
 //    9,261 nodes, 2.2 us of them the barrier.)
 //  * Every entry is written once per sweep.  Copies take turns, and a backward
 //    sweep puts the marks back into the copy that the sweep before used; the
-//    reductions between the sweeps are grid barriers.  With four copies the first
-//    look at an entry goes through the caches (a record is gathered about 13 times in
+//    reductions between the sweeps are grid barriers.  With four copies (from 17,000 nodes
+//    on) the first look at an entry goes through the caches (a record is gathered about 13 times in
 //    a sweep, and past the caches that was half of the memory traffic at 72^3); an
 //    old line can only hold marks, because the lines go once per turn of the copies, and
 //    a record with a mark in any entry that the sweep uses is asked for again past the
@@ -39,7 +39,7 @@
 //     p, q, g; partial p.q
 // Measured, us per iteration, launches per colour -> resident (HEX8 cubes and a
 // TET10 box, relative residual 1e-10): 343 nodes 183 -> 47, 4,845 (TET10) 441 ->
-// 82, 9,261 298 -> 62, 29,791 289 -> 64, 74,088 376 -> 80, 389,017 717 -> 291,
+// 80, 9,261 298 -> 64, 29,791 289 -> 65, 74,088 376 -> 81, 389,017 717 -> 288,
 // 1,030,301 1400 -> 774.  Up to 100,000 nodes the 2 x 16 colour steps bound it
 // (1.5-2 us each: gather round trip, row work, the way of the stores to the
 // neighbours' gathers); above, the round trips of a wave's tasks (8 waves per CU; the

@@ -1496,12 +1496,14 @@ static int32_t resident_setup(Context& c, const ResidentShape& sh, int32_t metho
   }
   const int32_t planes = method == 2 ? kResidentPlanesBi : kResidentPlanesCg;
   const bool new_rec = sym || o.planes != planes;
-  // Gathers through the caches from 6,000 nodes on (us per iteration, past them -> through:
-  // 14^3 58.1 -> 58.7, 20^3 63.6 -> 62.4, 30^3 67.1 -> 63.7, 41^3 87.8 -> 80.2, 72^3 383 -> 313), as long
+  // Gathers through the caches from 17,000 nodes on (us per iteration, past them -> through:
+  // 14^3 elements 59.4 -> 60.6, 20^3 63.5 -> 64.4, 24^3 66.5 -> 66.7, 27^3 69.2 -> 68.5, 30^3 67.2
+  // -> 65.1, 41^3 88.1 -> 81.4, 72^3 350 -> 288; BiCGSTAB 20^3 143 -> 145.6, 30^3 149 -> 143.7): below,
+  // the looks at z that they need cost more than the trips past the caches.  And as long
   // as four copies fit the 4 GiB of the buffer resource.  Matrix loads that leave the
   // caches alone when the matrix is larger than the 256 MB memory-side cache anyway
   // (41^3, 146 MB: 80.2 -> 87.6; 55^3, 340 MB: 158.7 -> 145.8; 72^3 313 -> 291).
-  o.cached = sh.grid > 1 && c.N > 6000 && ns < 16000000;
+  o.cached = sh.grid > 1 && c.N > 17000 && ns < 16000000;
   o.ring = o.cached ? 4 : 2;
   o.stream = (int64_t)(c.NPL + c.NPU) * 76 > (int64_t)256 << 20;
   if (new_rec && (c.res_vec.ensure(sizeof(double) * (planes * (size_t)ns + 8 * (size_t)o.ring * ((size_t)ns + 1))) ||
