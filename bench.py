@@ -39,10 +39,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# HBM bytes per launch of the in-solve SpMV (k_spmv<2>) on the 100^3 cube, from
+# HBM bytes per launch of the in-solve SpMV (k_spmv<2, true>) on the 100^3 cube, from
 # two rocprofv3 passes (FETCH_SIZE x 2.000, WRITE_SIZE x 1.000, the factors a
 # 1 GiB copy of the same run gives); profiles/spmv_hex8_100_traffic.md
-SPMV_TRAFFIC_100 = 2199539866
+SPMV_TRAFFIC_100 = 2198309344
 # HBM bytes per FP32 multicolour SSOR application (BF16 L'/U' values) on the
 # 160^3 lognormal cube (stage, 17 + 16 colour launches, unstage), from two
 # rocprofv3 passes over `bench.py --only ssor` (FETCH_SIZE x 2.000, WRITE_SIZE
